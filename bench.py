@@ -53,9 +53,9 @@ BYTES_PER_SITE_STEP = {"f64": 272, "f32c": 152, "f32s": 152}
 DESIGN_BYTES_PER_SITE_STEP = {"f64": 256, "f32c": 152, "tb_f64": 32, "tb_f32c": 32, "tb_f32s": 32}
 KERNEL_NAMES = {"f64": "cf::k_march<double, 1, S, false> (4 stage kernels)",
                 "f32c": "cf::k_march<float, 2, S, false> (4 stage kernels)",
-                "tb_f64": "cf::k_rk4_tb_ring<false>",
-                "tb_f32c": "cf::k_rk4_tb<float, true, false>",
-                "tb_f32s": "cf::k_rk4_tb_sa<false, {paced}, {rows}, {cols}>"}  # region shape per N
+                "tb_f64": "cf::k_rk4_tb<0, false, ...>",  # storage form, lambda; the region shape is picked per launch
+                "tb_f32c": "cf::k_rk4_tb<1, false, ...>",
+                "tb_f32s": "cf::k_rk4_tb<2, false, ...>"}
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "rk4_tb_N512_pmc_traffic.md")
 # What bounds each path's kernel at N=512, from the committed PMC summaries: the FP32-comp
 # blocked kernel issues VALU 76% of its cycles (float <-> double conversions on top of the
@@ -231,7 +231,8 @@ def ensemble_workload(args):
     ens.init_grf(seeds, cfl.CF_SPEC_GAUSS, (0.5,), 0.5)
     tuned_grid = ens.tune(dt, reps=3)
     plan = {n: ens.get_plan(n)[0] for n in (64, 96, 128)}
-    regions = {n: "24x40" if ens.get_region(n) == cfl.CF_ENS_REGION_24X40 else "32x32" for n in (64, 96, 128)}
+    shapes = {cfl.CF_ENS_REGION_24X40: "24x40", cfl.CF_ENS_REGION_32X32: "32x32", cfl.CF_ENS_REGION_28X36: "28x36"}
+    regions = {n: shapes[ens.get_region(n)] for n in (64, 96, 128)}
     # capture + first launch outside the timed region (the graph is reused)
     ens.run(t0, 0, steps, dt, use_graph=True)
     torch.cuda.synchronize()
@@ -717,9 +718,6 @@ def main():
         canon = BYTES_PER_SITE_STEP[mode.replace("tb_", "")]
         kb = DESIGN_BYTES_PER_SITE_STEP[mode]
         kname = KERNEL_NAMES[mode]
-        if mode == "tb_f32s":
-            rows, cols = cfl.rk4_tb_f32s_region(N)
-            kname = kname.format(paced="true" if pace > 0 else "false", rows=rows, cols=cols)
         results[mode] = {"value": rate, "ms_per_step": ms, "wall_s": wall,
                          "kernel": kname,
                          "kernel_bytes_per_site_step": kb,

@@ -25,8 +25,9 @@ CF_PREC_F32S = 2
 CF_NOALLOC_MAX_N = 128  # largest N of cf_rk4_run_tb_f64_noalloc
 
 CF_ENS_GRID_FLAT = -1  # ensemble plan: one block per work unit
-CF_ENS_REGION_32X32 = 0  # ensemble block region (b rows x c columns): 24 x 24 tiles
-CF_ENS_REGION_24X40 = 1  # 16 x 32 tiles
+CF_ENS_REGION_32X32 = 0  # ensemble block region (b rows x c columns): 28 x 28 tiles
+CF_ENS_REGION_24X40 = 1  # 20 x 36 tiles
+CF_ENS_REGION_28X36 = 2  # 24 x 32 tiles
 
 CF_VAR_FIXED_CURVATURE = 1
 CF_VAR_SQRT_POTENTIAL = 2

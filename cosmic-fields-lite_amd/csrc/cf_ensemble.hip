@@ -3,12 +3,12 @@
 // All realisations of an ensemble take their RK4 steps in one kernel per step
 // over a table of work units (one output tile of one lattice over a chunk of
 // a-planes, the unit of the temporally blocked step, cf_tb_body.hpp). Two launch
-// forms: a fixed grid of 1024-thread blocks, each running a list of units that
+// forms: a fixed grid of blocks, each running a list of units that
 // the host balanced by longest-processing-time-first over their iteration counts
 // (so the mix of N = 64 / 96 / 128 lattices finishes together), or one block per
 // unit, longest first. No atomics and no inter-block communication. The block's
-// region shape (32 x 32 or 24 x 40 columns, so 24 x 24 or 16 x 32 tiles) and the
-// chunk are chosen per lattice size; the autotuner times the candidates.
+// region shape (32 x 32, 24 x 40 or 28 x 36 sites, so 28 x 28, 20 x 36 or 24 x 32 tiles)
+// and the chunk are chosen per lattice size; the autotuner times the candidates.
 //
 // The step scalars a(t), H(t) of every stage live in a device table, so the
 // kernels of a whole run can be captured once into a hipGraph and replayed
@@ -43,17 +43,29 @@ struct EnsUnit {
   int64_t b0, c0, a0, a1;
 };
 
-// Region shapes of a unit's block (rows along b x columns along c): 32 x 32 (24 x 24
-// tiles, 1024 threads) and 24 x 40 (16 x 32 tiles, 960 threads: 1.88 region columns
-// per output site against 1.78, but tiles that divide N = 64 and 128 where 24 x 24
-// leaves 27% of the covered area outside the lattice).
-constexpr int ENS_R1_B = 24, ENS_R1_C = 40;
+// Region shapes of a unit's block, by CF_ENS_REGION_*. With float forces blocks are 512
+// threads with two columns each, two blocks per CU; with FP64 arithmetic 1024 threads with
+// one column each (two columns of FP64 and the unit's descriptors exceed 128 VGPRs: 30
+// spilled).
+constexpr int ENS_REGIONS = 3;
+constexpr int ENS_RB[ENS_REGIONS] = {32, 24, 28}, ENS_RC[ENS_REGIONS] = {32, 40, 36};
+template <int MODE, int REGION>
+using EnsShape = std::conditional_t<MODE != TB_F32S, TbShape<ENS_RB[REGION], ENS_RC[REGION], 1, 1024>,
+                                    TbShape<ENS_RB[REGION], ENS_RC[REGION], 2, 512>>;
+template <int MODE>
+constexpr int ens_threads() {
+  return MODE != TB_F32S ? 1024 : 512;
+}
+template <int MODE>
+constexpr int ens_lds() {
+  return std::max({EnsShape<MODE, 0>::LDS, EnsShape<MODE, 1>::LDS, EnsShape<MODE, 2>::LDS});
+}
 inline int ens_tile_b(int region, int64_t N) {
-  const int t = region == CF_ENS_REGION_24X40 ? ENS_R1_B - 2 * TBH : TBR - 2 * TBH;
+  const int t = ENS_RB[region] - 2 * TBH;
   return N < t ? (int)N : t;
 }
 inline int ens_tile_c(int region, int64_t N) {
-  const int t = region == CF_ENS_REGION_24X40 ? ENS_R1_C - 2 * TBH : TBR - 2 * TBH;
+  const int t = ENS_RC[region] - 2 * TBH;
   return N < t ? (int)N : t;
 }
 
@@ -77,19 +89,18 @@ __device__ __forceinline__ V wave_uniform(const V &v) {
 }
 
 // One work unit of the step: its lattice's step scalars, then the temporally
-// blocked body over a region of RB x RC columns.
-template <class T, bool F32C, bool LAM, bool DEFER, bool LANE_NBR = true, int RB = TBR, int RC = TBR, bool SA = false,
-          bool PACE = false>
-__device__ __forceinline__ void ens_unit(TbLds<T> &lds, const EnsReal *__restrict__ reals, const EnsUnit &e,
+// blocked body over a region of shape SH.
+template <int MODE, bool LAM, class SH, bool PACE>
+__device__ __forceinline__ void ens_unit(void *smem, const EnsReal *__restrict__ reals, const EnsUnit &e,
                                          const EnsStepCoef &sc, int parity, double c_m, double lam, double dt,
-                                         int pace = 0) {
+                                         int pace) {
   const EnsReal &R = reals[e.real];
   // Select this step's buffers first, then make each pointer uniform: indexing
   // x[parity] after the struct is in registers leaves the compiler treating the
   // pointers as divergent (plane addresses then run on the vector unit and every
   // buffer-resource build re-reads them lane by lane).
-  const T *xin = wave_uniform((const T *)(parity ? R.x[1] : R.x[0]));
-  T *xout = wave_uniform((T *)(parity ? R.x[0] : R.x[1]));
+  const void *xin = wave_uniform((const void *)(parity ? R.x[1] : R.x[0]));
+  void *xout = wave_uniform((void *)(parity ? R.x[0] : R.x[1]));
   const float *lin = wave_uniform(parity ? R.lo[1] : R.lo[0]);
   float *lout = wave_uniform(parity ? R.lo[0] : R.lo[1]);
   const int64_t N = wave_uniform(R.N);
@@ -112,7 +123,7 @@ __device__ __forceinline__ void ens_unit(TbLds<T> &lds, const EnsReal *__restric
   k.dt3 = dt / 3.0;
   k = wave_uniform(k);  // the divisions above ran on the vector unit (no scalar FP64)
   TbStepF kf{};  // single-precision stencil: the scalars rounded to float, as on the host
-  if constexpr (SA) {
+  if constexpr (MODE == TB_F32S) {
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
       kf.c_h[s] = (float)k.c_h[s];
@@ -134,38 +145,39 @@ __device__ __forceinline__ void ens_unit(TbLds<T> &lds, const EnsReal *__restric
   u.Tc = e.Tc;
   u.NA = N;
   u.pace = pace;
-  tb_unit<T, F32C, LAM, DEFER, LANE_NBR, TB_KG, false, RB, RC, SA, PACE>(lds, u, k, xin, lin, xout, lout, nullptr,
-                                                                       TbPsi{}, kf);
+  tb_unit<MODE, LAM, SH, TB_KG, PACE>(smem, u, k, kf, xin, lin, xout, lout);
 }
 
-// A unit in its region shape (a wave-uniform branch; lane neighbours only in rows of
-// 32 columns).
-template <class T, bool F32C, bool LAM, bool DEFER, bool LANE_NBR, bool SA = false, bool PACE = false>
-__device__ __forceinline__ void ens_unit_any(TbLds<T> &lds, const EnsReal *__restrict__ reals, const EnsUnit &unit,
+// A unit in its region shape (a wave-uniform branch).
+template <int MODE, bool LAM, bool PACE>
+__device__ __forceinline__ void ens_unit_any(void *smem, const EnsReal *__restrict__ reals, const EnsUnit &unit,
                                              const EnsStepCoef &sc, int parity, double c_m, double lam, double dt,
-                                             int pace = 0) {
+                                             int pace) {
   const EnsUnit e = wave_uniform(unit);
-  if (e.region == CF_ENS_REGION_24X40)
-    ens_unit<T, F32C, LAM, DEFER, false, ENS_R1_B, ENS_R1_C, SA, PACE>(lds, reals, e, sc, parity, c_m, lam, dt,
-                                                                        pace);
+  if (e.region == CF_ENS_REGION_28X36)
+    ens_unit<MODE, LAM, EnsShape<MODE, CF_ENS_REGION_28X36>, PACE>(smem, reals, e, sc, parity, c_m, lam, dt, pace);
+  else if (e.region == CF_ENS_REGION_24X40)
+    ens_unit<MODE, LAM, EnsShape<MODE, CF_ENS_REGION_24X40>, PACE>(smem, reals, e, sc, parity, c_m, lam, dt, pace);
   else
-    ens_unit<T, F32C, LAM, DEFER, LANE_NBR, TBR, TBR, SA, PACE>(lds, reals, e, sc, parity, c_m, lam, dt, pace);
+    ens_unit<MODE, LAM, EnsShape<MODE, CF_ENS_REGION_32X32>, PACE>(smem, reals, e, sc, parity, c_m, lam, dt, pace);
 }
+
+// Element type of the plane buffers (the same for every shape of a mode).
+template <int MODE>
+using EnsElem = TbElem<MODE, EnsShape<MODE, 0>>;
 
 // Persistent form: a fixed grid; block b runs units unit_off[b] .. unit_off[b+1]-1
-// (an LPT-balanced list). Stores are not deferred: the unit loop leaves less
-// register room than a single unit.
-template <class T, bool F32C, bool LAM>
-__global__ __launch_bounds__(1024) void k_ens_tb(const EnsReal *__restrict__ reals,
-                                                 const int32_t *__restrict__ unit_off,
-                                                 const EnsUnit *__restrict__ units,
-                                                 const EnsStepCoef *__restrict__ steps, int64_t step, int parity,
-                                                 double c_m, double lam, double dt) {
-  __shared__ TbLds<T> lds;
+// (an LPT-balanced list). PACE (TB_F32S only): every unit's plane iterations follow pace
+// ticks of the real-time counter from the unit's start (cf_tb_body.hpp).
+template <int MODE, bool LAM, bool PACE>
+__global__ __launch_bounds__(ens_threads<MODE>()) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_ens_tb(
+    const EnsReal *__restrict__ reals, const int32_t *__restrict__ unit_off, const EnsUnit *__restrict__ units,
+    const EnsStepCoef *__restrict__ steps, int64_t step, int parity, double c_m, double lam, double dt, int pace) {
+  __shared__ __attribute__((aligned(16))) EnsElem<MODE> smem[ens_lds<MODE>()];
   const EnsStepCoef sc = steps[step];
   const int beg = unit_off[blockIdx.x], end = unit_off[blockIdx.x + 1];
   for (int i = beg; i < end; ++i) {
-    ens_unit_any<T, F32C, LAM, false, true>(lds, reals, units[i], sc, parity, c_m, lam, dt);
+    ens_unit_any<MODE, LAM, PACE>(smem, reals, units[i], sc, parity, c_m, lam, dt, pace);
     __syncthreads();  // the next unit rewrites the plane buffers
   }
 }
@@ -177,51 +189,18 @@ __global__ __launch_bounds__(1024) void k_ens_tb(const EnsReal *__restrict__ rea
 // meet in one L2, while the long-first order stays balanced across XCDs.
 constexpr int ENS_XCD_GROUP = 4;
 
-template <class T, bool F32C, bool LAM>
-__global__ __launch_bounds__(1024) void k_ens_tb_flat(const EnsReal *__restrict__ reals,
-                                                      const EnsUnit *__restrict__ units,
-                                                      const EnsStepCoef *__restrict__ steps, int64_t step,
-                                                      int parity, double c_m, double lam, double dt) {
-  __shared__ TbLds<T> lds;
+template <int MODE, bool LAM, bool PACE>
+__global__ __launch_bounds__(ens_threads<MODE>()) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_ens_tb_flat(
+    const EnsReal *__restrict__ reals, const EnsUnit *__restrict__ units, const EnsStepCoef *__restrict__ steps,
+    int64_t step, int parity, double c_m, double lam, double dt, int pace) {
+  __shared__ __attribute__((aligned(16))) EnsElem<MODE> smem[ens_lds<MODE>()];
   int u = blockIdx.x;
   const int total = gridDim.x;
   if (total % (8 * ENS_XCD_GROUP) == 0) {  // a bijection of [0, total); otherwise dispatch order
     const int x = u & 7, i = u >> 3;
     u = ((i / ENS_XCD_GROUP) * 8 + x) * ENS_XCD_GROUP + (i % ENS_XCD_GROUP);
   }
-  ens_unit_any<T, F32C, LAM, true, !F32C>(lds, reals, units[u], steps[step], parity, c_m, lam, dt);
-}
-
-// The same two forms for the compensated storage with the single-precision stencil
-// (CF_PREC_F32S), paced (PACE: every unit's plane iterations follow pace ticks of the
-// real-time counter from the unit's start; cf_tb_body.hpp). Occupancy is one 1024-thread
-// block per CU regardless, so the compiler may use the 128 VGPRs that allows.
-template <bool LAM, bool PACE>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_ens_tb_sa(
-    const EnsReal *__restrict__ reals, const int32_t *__restrict__ unit_off, const EnsUnit *__restrict__ units,
-    const EnsStepCoef *__restrict__ steps, int64_t step, int parity, double c_m, double lam, double dt, int pace) {
-  __shared__ TbLds<float> lds;
-  const EnsStepCoef sc = steps[step];
-  const int beg = unit_off[blockIdx.x], end = unit_off[blockIdx.x + 1];
-  for (int i = beg; i < end; ++i) {
-    ens_unit_any<float, true, LAM, false, false, true, PACE>(lds, reals, units[i], sc, parity, c_m, lam, dt, pace);
-    __syncthreads();
-  }
-}
-
-template <bool LAM, bool PACE>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_ens_tb_flat_sa(
-    const EnsReal *__restrict__ reals, const EnsUnit *__restrict__ units, const EnsStepCoef *__restrict__ steps,
-    int64_t step, int parity, double c_m, double lam, double dt, int pace) {
-  __shared__ TbLds<float> lds;
-  int u = blockIdx.x;
-  const int total = gridDim.x;
-  if (total % (8 * ENS_XCD_GROUP) == 0) {
-    const int x = u & 7, i = u >> 3;
-    u = ((i / ENS_XCD_GROUP) * 8 + x) * ENS_XCD_GROUP + (i % ENS_XCD_GROUP);
-  }
-  ens_unit_any<float, true, LAM, true, false, true, PACE>(lds, reals, units[u], steps[step], parity, c_m, lam, dt,
-                                                          pace);
+  ens_unit_any<MODE, LAM, PACE>(smem, reals, units[u], steps[step], parity, c_m, lam, dt, pace);
 }
 
 }  // namespace cf
@@ -290,7 +269,7 @@ static cf_status ens_build(cf_ensemble *e) {
     const int Tb = ens_tile_b(reg, N), Tc = ens_tile_c(reg, N);
     const int64_t ntb = cdiv(N, Tb), ntc = cdiv(N, Tc);
     const int A = e->chunk[N];
-    const int waves = reg == CF_ENS_REGION_24X40 ? (ENS_R1_B * ENS_R1_C + 63) / 64 : TBR * TBR / 64;
+    const int sites = ENS_RB[reg] * ENS_RC[reg];
     for (int64_t a0 = 0; a0 < N; a0 += A)
       for (int64_t tb = 0; tb < ntb; ++tb)
         for (int64_t tc = 0; tc < ntc; ++tc) {
@@ -304,7 +283,7 @@ static cf_status ens_build(cf_ensemble *e) {
           u.a0 = a0;
           u.a1 = std::min<int64_t>(a0 + A, N);
           units.push_back(u);
-          cost.push_back(((int)(u.a1 - u.a0) + 8) * waves);
+          cost.push_back(((int)(u.a1 - u.a0) + 2 * TBH) * sites);
         }
   }
   std::vector<int> order(units.size());
@@ -383,74 +362,27 @@ static cf_status ens_fill_steps(cf_ensemble *e, double t0, int64_t k0, int64_t n
   return CF_OK;
 }
 
-static cf_status ens_launch_sa(cf_ensemble *e, int64_t step, int parity, double dt, hipStream_t st) {
+template <int MODE, bool LAM, bool PACE>
+static void ens_launch_as(cf_ensemble *e, int64_t step, int parity, double dt, hipStream_t st) {
   const double c_m = e->m * e->m;
-  const bool lam = e->lambda != 0.0, paced = e->pace > 0;
-  const dim3 blk(1024);
-  if (e->grid == CF_ENS_GRID_FLAT) {
-    const dim3 grd(e->n_units);
-#define CF_ENS_FLAT_SA(L, P)                                                                                        \
-  hipLaunchKernelGGL((k_ens_tb_flat_sa<L, P>), grd, blk, 0, st, e->d_reals, e->d_units, e->d_steps, step, parity, \
-                     c_m, e->lambda, dt, e->pace)
-    if (lam && paced) CF_ENS_FLAT_SA(true, true);
-    else if (lam) CF_ENS_FLAT_SA(true, false);
-    else if (paced) CF_ENS_FLAT_SA(false, true);
-    else CF_ENS_FLAT_SA(false, false);
-#undef CF_ENS_FLAT_SA
-  } else {
-    const dim3 grd(e->grid);
-#define CF_ENS_SA(L, P)                                                                                            \
-  hipLaunchKernelGGL((k_ens_tb_sa<L, P>), grd, blk, 0, st, e->d_reals, e->d_unit_off, e->d_units, e->d_steps, step, \
-                     parity, c_m, e->lambda, dt, e->pace)
-    if (lam && paced) CF_ENS_SA(true, true);
-    else if (lam) CF_ENS_SA(true, false);
-    else if (paced) CF_ENS_SA(false, true);
-    else CF_ENS_SA(false, false);
-#undef CF_ENS_SA
-  }
-  CF_LAUNCHED();
-  return CF_OK;
+  const dim3 blk(ens_threads<MODE>());
+  if (e->grid == CF_ENS_GRID_FLAT)
+    hipLaunchKernelGGL((k_ens_tb_flat<MODE, LAM, PACE>), dim3(e->n_units), blk, 0, st, e->d_reals, e->d_units,
+                       e->d_steps, step, parity, c_m, e->lambda, dt, e->pace);
+  else
+    hipLaunchKernelGGL((k_ens_tb<MODE, LAM, PACE>), dim3(e->grid), blk, 0, st, e->d_reals, e->d_unit_off, e->d_units,
+                       e->d_steps, step, parity, c_m, e->lambda, dt, e->pace);
 }
 
 static cf_status ens_launch(cf_ensemble *e, int64_t step, int parity, double dt, hipStream_t st) {
-  if (e->prec == CF_PREC_F32S) return ens_launch_sa(e, step, parity, dt, st);
-  dim3 grd(e->grid), blk(1024);
-  const double c_m = e->m * e->m;
   const bool lam = e->lambda != 0.0;
-  if (e->grid == CF_ENS_GRID_FLAT) {
-    grd = dim3(e->n_units);
-    if (e->prec == CF_PREC_F32C) {
-      if (lam)
-        hipLaunchKernelGGL((k_ens_tb_flat<float, true, true>), grd, blk, 0, st, e->d_reals, e->d_units, e->d_steps,
-                           step, parity, c_m, e->lambda, dt);
-      else
-        hipLaunchKernelGGL((k_ens_tb_flat<float, true, false>), grd, blk, 0, st, e->d_reals, e->d_units, e->d_steps,
-                           step, parity, c_m, e->lambda, dt);
-    } else {
-      if (lam)
-        hipLaunchKernelGGL((k_ens_tb_flat<double, false, true>), grd, blk, 0, st, e->d_reals, e->d_units,
-                           e->d_steps, step, parity, c_m, e->lambda, dt);
-      else
-        hipLaunchKernelGGL((k_ens_tb_flat<double, false, false>), grd, blk, 0, st, e->d_reals, e->d_units,
-                           e->d_steps, step, parity, c_m, e->lambda, dt);
-    }
-    CF_LAUNCHED();
-    return CF_OK;
-  }
-  if (e->prec == CF_PREC_F32C) {
-    if (lam)
-      hipLaunchKernelGGL((k_ens_tb<float, true, true>), grd, blk, 0, st, e->d_reals, e->d_unit_off, e->d_units,
-                         e->d_steps, step, parity, c_m, e->lambda, dt);
-    else
-      hipLaunchKernelGGL((k_ens_tb<float, true, false>), grd, blk, 0, st, e->d_reals, e->d_unit_off, e->d_units,
-                         e->d_steps, step, parity, c_m, e->lambda, dt);
+  if (e->prec == CF_PREC_F32S) {
+    if (e->pace > 0) lam ? ens_launch_as<TB_F32S, true, true>(e, step, parity, dt, st) : ens_launch_as<TB_F32S, false, true>(e, step, parity, dt, st);
+    else lam ? ens_launch_as<TB_F32S, true, false>(e, step, parity, dt, st) : ens_launch_as<TB_F32S, false, false>(e, step, parity, dt, st);
+  } else if (e->prec == CF_PREC_F32C) {
+    lam ? ens_launch_as<TB_F32C, true, false>(e, step, parity, dt, st) : ens_launch_as<TB_F32C, false, false>(e, step, parity, dt, st);
   } else {
-    if (lam)
-      hipLaunchKernelGGL((k_ens_tb<double, false, true>), grd, blk, 0, st, e->d_reals, e->d_unit_off, e->d_units,
-                         e->d_steps, step, parity, c_m, e->lambda, dt);
-    else
-      hipLaunchKernelGGL((k_ens_tb<double, false, false>), grd, blk, 0, st, e->d_reals, e->d_unit_off,
-                         e->d_units, e->d_steps, step, parity, c_m, e->lambda, dt);
+    lam ? ens_launch_as<TB_F64, true, false>(e, step, parity, dt, st) : ens_launch_as<TB_F64, false, false>(e, step, parity, dt, st);
   }
   CF_LAUNCHED();
   return CF_OK;
@@ -666,8 +598,7 @@ cf_status cf_ensemble_get_plan(const cf_ensemble *e, int64_t N, int *chunk, int 
 cf_status cf_ensemble_set_region(cf_ensemble *e, int64_t N, int region) {
   CF_REQUIRE(e, "cf_ensemble_set_region: null ensemble");
   CF_REQUIRE(e->region.count(N), "cf_ensemble_set_region: no lattice of size %lld", (long long)N);
-  CF_REQUIRE(region == CF_ENS_REGION_32X32 || region == CF_ENS_REGION_24X40,
-             "cf_ensemble_set_region: unknown region shape %d", region);
+  CF_REQUIRE(region >= 0 && region < ENS_REGIONS, "cf_ensemble_set_region: unknown region shape %d", region);
   e->region[N] = region;
   return ens_build(e);
 }
@@ -701,53 +632,79 @@ cf_status cf_ensemble_tune(cf_ensemble *e, double dt, int reps, int *grid_out) {
   CF_REQUIRE(e, "cf_ensemble_tune: null ensemble");
   if (reps <= 0) reps = 3;
   CF_TRY(ens_fill_steps(e, 0.0, 0, 1, dt));
-  const int grids[] = {256, 512, 768, 1024, 2048, CF_ENS_GRID_FLAT};
   float best = 1e30f, ms = 0;
-  int best_g = e->grid;
-  for (int g : grids) {
-    e->grid = g;
-    CF_TRY(ens_build(e));
-    CF_TRY(ens_time(e, reps, dt, &ms));
-    if (ms < best) {
-      best = ms;
-      best_g = g;
+  // Flat launches first, every size at one common chunk and region shape: a start from
+  // which no size's later sweep is misled by another size's poor chunk.
+  e->grid = CF_ENS_GRID_FLAT;
+  int best_a = 0, best_r = CF_ENS_REGION_28X36;
+  for (int reg : {CF_ENS_REGION_28X36, CF_ENS_REGION_32X32})
+    for (int A : {64, 32, 16, 8}) {
+      if (reg != CF_ENS_REGION_28X36 && A != best_a) continue;  // the other shape at the first one's chunk
+      for (auto &kv : e->chunk) {
+        kv.second = (int)std::min<int64_t>(A, kv.first);
+        e->region[kv.first] = reg;
+      }
+      CF_TRY(ens_build(e));
+      CF_TRY(ens_time(e, reps, dt, &ms));
+      if (ms < best) {
+        best = ms;
+        best_a = A;
+        best_r = reg;
+      }
     }
+  for (auto &kv : e->chunk) {
+    kv.second = (int)std::min<int64_t>(best_a, kv.first);
+    e->region[kv.first] = best_r;
   }
-  e->grid = best_g;
   CF_TRY(ens_build(e));
-  // per lattice size, every (region shape, chunk) pair, the other sizes' plans held;
-  // a second sweep revisits each size once the others have their tuned plans. Chunks
-  // go longest first and a candidate must win by more than 0.5%: within the timing
-  // noise the longer chunk (fewer warm-up planes) is kept. A paced ensemble
-  // (CF_PREC_F32S) tunes its pace between the two sweeps, so the second one times the
-  // plans paced.
-  for (int sweep = 0; sweep < 2; ++sweep) {
-    if (sweep == 1 && e->prec == CF_PREC_F32S) CF_TRY(ens_tune_pace(e, reps, dt));
+  // Then per lattice size every (region shape, chunk) pair, the other sizes' plans held. A
+  // candidate must win by more than 0.5%. A paced ensemble (CF_PREC_F32S) tunes its pace
+  // between two such sweeps, so the second one times the plans paced.
+  for (int sweep = 0; sweep < (e->prec == CF_PREC_F32S ? 2 : 1); ++sweep) {
+    if (sweep == 1) CF_TRY(ens_tune_pace(e, reps, dt));
     for (auto &kv : e->chunk) {
       const int64_t N = kv.first;
-      int best_a = kv.second, best_r = e->region[N];
+      int keep_a = kv.second, keep_r = e->region[N];
+      const int was_a = keep_a, was_r = keep_r;
       CF_TRY(ens_time(e, reps, dt, &best));
       std::vector<int> chunks;
-      for (int A : {(int)N, 256, 128, 64, 32, 16, 8})
+      for (int A : {(int)N, (int)(N + 1) / 2, 256, 128, 64, 32, 16, 8})
         if (A <= N && std::find(chunks.begin(), chunks.end(), A) == chunks.end()) chunks.push_back(A);
-      for (int reg : {CF_ENS_REGION_32X32, CF_ENS_REGION_24X40})
+      for (int reg : {CF_ENS_REGION_28X36, CF_ENS_REGION_32X32})
         for (int A : chunks) {
-          if (A == best_a && reg == best_r) continue;
+          if (A == was_a && reg == was_r) continue;
           e->chunk[N] = A;
           e->region[N] = reg;
           CF_TRY(ens_build(e));
           CF_TRY(ens_time(e, reps, dt, &ms));
           if (ms < best * 0.995f) {
             best = ms;
-            best_a = A;
-            best_r = reg;
+            keep_a = A;
+            keep_r = reg;
           }
         }
-      e->chunk[N] = best_a;
-      e->region[N] = best_r;
+      e->chunk[N] = keep_a;
+      e->region[N] = keep_r;
       CF_TRY(ens_build(e));
     }
   }
+  // Last the persistent grids of fewer blocks than units (flat launches have measured
+  // faster for every mix so far; a persistent one must win by 0.5%).
+  CF_TRY(ens_time(e, reps, dt, &best));
+  const int units = e->n_units;
+  int best_g = CF_ENS_GRID_FLAT;
+  for (int g : {256, 512, 1024}) {
+    if (g >= units) continue;
+    e->grid = g;
+    CF_TRY(ens_build(e));
+    CF_TRY(ens_time(e, reps, dt, &ms));
+    if (ms < best * 0.995f) {
+      best = ms;
+      best_g = g;
+    }
+  }
+  e->grid = best_g;
+  CF_TRY(ens_build(e));
   if (grid_out) *grid_out = e->grid;
   return CF_OK;
 }

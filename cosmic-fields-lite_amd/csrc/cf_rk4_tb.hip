@@ -7,30 +7,32 @@
 // hi', lo' = 32 B (plus halo and warm-up re-reads, mostly served by L2).
 // The output goes to a second buffer (neighbouring blocks still read the old
 // state), so runs ping-pong between two state arrays.
+#include <algorithm>
+#include <atomic>
 #include <cmath>
-
 #include <map>
 #include <mutex>
 #include <tuple>
+#include <utility>
 #include <vector>
 
 #include "cf_tb_body.hpp"
-#include "cf_tb_ring.hpp"
 #include "cf_tb_run.hpp"
 
 namespace cf {
 
 struct TbGeom {
   int64_t N;
-  int Tb, Tc;        // output tile edges along b and c
-  int ntb, ntc;      // tiles along b and c
-  int A;             // planes per chunk
-  int n_ac;          // chunks
-  int total;         // ntb * ntc * n_ac
-  int64_t NA;        // planes of the state buffers along a (N, or a slab's planes + ghosts)
+  int shape;           // index of the kernel's region shape (below)
+  int rb, rc;          // its rows and columns
+  int Tb, Tc;          // output tile edges along b and c
+  int ntb, ntc;        // tiles along b and c
+  int A;               // planes per chunk
+  int n_ac;            // chunks
+  int total;           // ntb * ntc * n_ac
+  int64_t NA;          // planes of the state buffers along a (N, or a slab's planes + ghosts)
   int64_t a_lo, a_hi;  // output planes [a_lo, a_hi)
   int pace;            // ticks of the 100 MHz real-time counter per plane iteration, 0: unpaced
-  int rb, rc;          // region shape (Tb, Tc plus the halo) the launch was planned for
 };
 
 // Work unit of logical block `bid`: tile (tb, tc), chunk ac, c fastest.
@@ -52,163 +54,175 @@ __device__ __forceinline__ TbUnit tb_unit_of(const TbGeom &g, int bid) {
   return u;
 }
 
-// Region shape (b rows x c columns) of the FP32-comp single-lattice kernel. Measured
-// at N=512 (GSite*step/s, same bits): 32 x 32 (24 x 24 tiles) 87.8-88.3; 24 x 40 (16 x 32
-// tiles, whose c edges fall on 128-byte lines; 960 threads) 83.0-83.4; 25 x 40 81.4-82.1.
-constexpr int TB_F32C_RB = 32, TB_F32C_RC = 32;
-// Region shape of the single-precision-stencil kernel: 24 x 40 (16 x 32 tiles, 960 of the
-// 1024 threads; the tiles' c edges fall on 128-byte lines, and N=512 makes 512 tiles).
-// Measured at N=512 with 256-plane chunks (1024 blocks, four full rounds over 256 CUs;
-// GSite*step/s, same bits): unpaced 101.7 against 76.7 for 32 x 32, paced 107.0 (at 115
-// ticks per plane) against 97.3 (at 128).
-constexpr int TB_F32S_RB = 24, TB_F32S_RC = 40;
-
-template <class T, bool F32C, bool LAM>
-__global__ __launch_bounds__(1024) void k_rk4_tb(TbGeom g, TbStep k, const T *__restrict__ xin,
-                                                 const float *__restrict__ lin, T *__restrict__ xout,
-                                                 float *__restrict__ lout) {
-  __shared__ TbLds<T> lds;
+// One kernel per storage form, region shape and lambda = 0 / != 0. WAVES: wavefronts
+// per SIMD the registers leave room for (512 / WAVES VGPRs each). PACE: the blocks keep
+// to a common schedule of plane iterations (cf_tb_body.hpp).
+template <int MODE, bool LAM, class SH, int WAVES, bool PACE>
+__global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void k_rk4_tb(
+    TbGeom g, TbStep k, TbStepF kf, const void *__restrict__ xin, const float *__restrict__ lin,
+    void *__restrict__ xout, float *__restrict__ lout) {
+  __shared__ __attribute__((aligned(16))) TbElem<MODE, SH> smem[SH::LDS];
   // Blocks go to the 8 XCDs round robin; consecutive logical tiles are mapped
   // to one XCD so that neighbouring tiles' halos meet in its L2.
-  const TbUnit u = tb_unit_of(g, tb_xcd_order(blockIdx.x, g.total));
-  // Lane shifts for the c neighbours in FP64; LDS in the compensated mode, whose
-  // float plane buffers are cheap and whose VALU load is the larger (measured).
-  constexpr int RB = F32C ? TB_F32C_RB : TBR, RC = F32C ? TB_F32C_RC : TBR;
-  tb_unit<T, F32C, LAM, true, !F32C && RC == TBR, TB_KG, false, RB, RC>(lds, u, k, xin, lin, xout, lout);
+  tb_unit<MODE, LAM, SH, TB_KG, PACE>(smem, tb_unit_of(g, tb_xcd_order(blockIdx.x, g.total)), k, kf, xin, lin, xout,
+                                      lout);
 }
 
-// The compensated storage with the single-precision stencil (float forces, double
-// increment): the same body as the FP32-comp kernel over 24 x 40 regions; PACE: paced
-// (cf_tb_body.hpp), at g.pace ticks per plane iteration. Occupancy stays at one
-// 1024-thread block per CU, so the compiler may use the 128 VGPRs that allows: with
-// its default target it kept 84 and serialised the LDS neighbour reads (read, wait,
-// add, read), 77.6 against 80.4 GSite*step/s unpaced at N=512.
-template <bool LAM, bool PACE, int RB = TB_F32S_RB, int RC = TB_F32S_RC>
-__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_rk4_tb_sa(
-    TbGeom g, TbStep k, TbStepF kf, const float *__restrict__ xin, const float *__restrict__ lin,
-    float *__restrict__ xout, float *__restrict__ lout) {
-  __shared__ TbLds<float> lds;
-  const TbUnit u = tb_unit_of(g, tb_xcd_order(blockIdx.x, g.total));
-  tb_unit<float, true, LAM, true, false, TB_KG, false, RB, RC, true, PACE>(lds, u, k, xin, lin, xout, lout, nullptr,
-                                                                         TbPsi{}, kf);
+// The same step for the equation variants, FP64.
+template <int VAR, class SH>
+__global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_rk4_tb_var(
+    TbGeom g, TbStep k, const double *__restrict__ xin, double *__restrict__ xout, const double *__restrict__ psi,
+    TbPsi cps) {
+  __shared__ __attribute__((aligned(16))) double smem[SH::LDS];
+  tb_unit<TB_F64, false, SH, VAR>(smem, tb_unit_of(g, tb_xcd_order(blockIdx.x, g.total)), k, TbStepF{}, xin, nullptr,
+                                  xout, nullptr, psi, cps);
 }
 
-// FP64: the same step with the state streamed into an LDS ring TB_RING_DEPTH planes
-// ahead (cf_tb_ring.hpp; same bits as the register-prefetch body).
-constexpr int TB_RING_DEPTH = 4;
+// Region shapes of the single-lattice kernels, smallest first. A large region repeats
+// less of its neighbours' work and reads (26 x 64 tiles: 1.23 region sites per output
+// site, 8 x 16 ones 1.88); a small one gives a small lattice enough blocks and takes
+// less time per plane. `wave`: VGPR budget as wavefronts per SIMD.
+//
+// t1 and tau are the time of a plane iteration in us with one block on a CU and, per
+// block, with the CU full; bw the rate in bytes per us at which launches that stream
+// through HBM pass their loads (halo and warm-up included) and stores. Measured over
+// N = 32 .. 512 on 256 CUs; see tb_cost.
+struct TbShapeInfo {
+  int rb, rc, resident;
+  double t1, tau, bw;
+};
+typedef TbShape<12, 20, 2, 128> TbS12x20;
+typedef TbShape<14, 36, 2, 256> TbS14x36;
+typedef TbShape<28, 36, 2, 512> TbS28x36;
+typedef TbShape<30, 68, 2, 1024> TbS30x68;
+typedef TbShape<15, 132, 2, 1024> TbS15x132;  // floats: 128-column rows, four lines
+typedef TbShape<14, 36, 1, 512> TbC14x36;     // a column per thread (TB_F32C, variants)
+typedef TbShape<28, 36, 1, 1024> TbC28x36;
+typedef TbShape<22, 68, 2, 768> TbC22x68;     // 768 threads: 168 VGPRs for float histories and double sums
 
-template <bool LAM>
-__global__ __launch_bounds__(1024) void k_rk4_tb_ring(TbGeom g, TbStep k, const double *__restrict__ xin,
-                                                      double *__restrict__ xout) {
-  __shared__ __attribute__((aligned(16))) char smem[TbRing<TB_RING_DEPTH>::BYTES];
-  const TbUnit u = tb_unit_of(g, tb_xcd_order(blockIdx.x, g.total));
-  tb_unit_ring<LAM, TB_RING_DEPTH>(smem, u, k, xin, xout);
+static const std::vector<TbShapeInfo> &tb_shapes(int family);
+
+enum : int { TB_FAM_F64 = 0, TB_FAM_F32C = 1, TB_FAM_F32S = 2, TB_FAM_VAR = 3 };
+
+static const std::vector<TbShapeInfo> &tb_shapes(int family) {
+  static const std::vector<TbShapeInfo> t[4] = {
+      {{12, 20, 8, 0.56, 0.20, 4.9e6}, {14, 36, 4, 0.64, 0.46, 5.0e6}, {28, 36, 2, 0.96, 0.93, 5.3e6},
+       {30, 68, 1, 1.75, 1.75, 5.55e6}},
+      {{14, 36, 2, 0.75, 0.60, 4.6e6}, {28, 36, 1, 1.24, 1.24, 4.7e6}, {22, 68, 1, 1.73, 1.73, 5.1e6}},
+      {{12, 20, 8, 0.54, 0.16, 4.0e6}, {14, 36, 4, 0.56, 0.39, 4.6e6}, {28, 36, 2, 0.85, 0.81, 4.6e6},
+       {30, 68, 1, 1.55, 1.55, 4.9e6}, {15, 132, 1, 1.55, 1.55, 5.2e6}},
+      {{14, 36, 2, 0.9, 0.8, 4.6e6}, {28, 36, 1, 1.5, 1.5, 4.9e6}},
+  };
+  return t[family];
 }
 
-// The same step for the fixed-curvature (Psi, N^3) and sqrt-potential equation
-// variants, FP64.
-template <int VAR>
-__global__ __launch_bounds__(1024) void k_rk4_tb_var(TbGeom g, TbStep k, const double *__restrict__ xin,
-                                                     double *__restrict__ xout, const double *__restrict__ psi,
-                                                     TbPsi cps) {
-  __shared__ TbLds<double> lds;
-  const TbUnit u = tb_unit_of(g, tb_xcd_order(blockIdx.x, g.total));
-  tb_unit<double, false, false, true, true, VAR, true>(lds, u, k, xin, nullptr, xout, nullptr, psi, cps);
+// Compute units of the current device.
+static int tb_cus() {
+  static std::atomic<int> known[64] = {};
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if ((cus = known[dev].load(std::memory_order_relaxed)) > 0) return cus;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) return 256;
+  known[dev].store(cus, std::memory_order_relaxed);
+  return cus;
 }
 
-// Tiles of (RB - 8) x (RC - 8) sites (the whole extent when N is smaller) over the
+// Tiles of (rb - 4) x (rc - 4) sites (the whole extent when N is smaller) over the
 // output planes [a_lo, a_hi) of buffers of NA planes; a periodic lattice: 0, N, N.
-static TbGeom tb_geom(int64_t N, int A, int RB = TBR, int RC = TBR, int64_t a_lo = 0, int64_t a_hi = -1,
-                      int64_t NA = -1) {
+static TbGeom tb_geom(int family, int shape, int64_t N, int A, int64_t a_lo, int64_t a_hi, int64_t NA) {
+  const TbShapeInfo &s = tb_shapes(family)[(size_t)shape];
   TbGeom g;
   g.N = N;
+  g.shape = shape;
+  g.rb = s.rb;
+  g.rc = s.rc;
   g.a_lo = a_lo;
-  g.a_hi = a_hi < 0 ? N : a_hi;
-  g.NA = NA < 0 ? N : NA;
-  const int64_t planes = g.a_hi - g.a_lo;
-  g.Tb = N < RB - 2 * TBH ? (int)N : RB - 2 * TBH;
-  g.Tc = N < RC - 2 * TBH ? (int)N : RC - 2 * TBH;
+  g.a_hi = a_hi;
+  g.NA = NA;
+  const int64_t planes = a_hi - a_lo;
+  g.Tb = N < s.rb - 2 * TBH ? (int)N : s.rb - 2 * TBH;
+  g.Tc = N < s.rc - 2 * TBH ? (int)N : s.rc - 2 * TBH;
   g.ntb = (int)cdiv(N, g.Tb);
   g.ntc = (int)cdiv(N, g.Tc);
   g.A = (A <= 0 || A > planes) ? (int)planes : A;
   g.n_ac = (int)cdiv(planes, g.A);
   g.total = g.ntb * g.ntc * g.n_ac;
   g.pace = 0;
-  g.rb = RB;
-  g.rc = RC;
   return g;
 }
 
-// Default planes per block along a. One 1024-thread block runs per CU at a time,
-// so k chunks per tile cost about ceil(tiles k / CUs) rounds of (N/k + 8) plane
-// iterations (8 warm-up planes per chunk). Too few blocks leave CUs idle (N=256 with
-// one chunk: 121 blocks for 256 CUs), too many pay warm-ups. Among the k within 2%
-// of the cheapest, the largest is taken. Measured on MI355X (FP64 / FP32-comp
-// GSite*step/s): N=128 chunk 19 66 / 55 against 16 / 12 with one chunk; N=256 chunk
-// 128 103 / 89 against 65 / 51; N=384 one chunk 118 / 88 against 92 / 74 with 256;
-// N=512 chunk 256 (the rule's pick) and 171 within 1-3% of each other, one chunk
-// 96 / 77.
-static int tb_default_chunk(int64_t N, int RB = TBR, int RC = TBR, int64_t planes = -1,
-                            int64_t *cost_out = nullptr, std::vector<int> *near = nullptr, int near_pct = 0) {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
-  if (planes < 0) planes = N;  // output planes of the launch
-  const TbGeom g1 = tb_geom(N, 0, RB, RC);
-  const int64_t tiles = (int64_t)g1.ntb * g1.ntc;
-  const int64_t kmax = planes / 8 > 1 ? planes / 8 : 1;
-  std::vector<int64_t> cost((size_t)kmax + 1, -1);
-  int64_t best = -1;
-  for (int64_t k = 1; k <= kmax; ++k) {
-    const int64_t ch = cdiv(planes, k);
-    const int64_t kk = cdiv(planes, ch);  // chunks actually launched for this chunk length
-    if (kk != k) continue;
-    cost[k] = cdiv(tiles * k, cus) * (ch + 8);
-    if (best < 0 || cost[k] < best) best = cost[k];
+// Modelled time of a launch in us: the larger of
+//   the busiest CU's plane iterations: its n = ceil(blocks / CUs) blocks run `resident`
+//   at a time, A + 4 iterations each, at tau per block (t1 when one runs alone), and
+//   the bytes it passes: the loads of every region and iteration and the stores, at bw
+//   (20% more while both states fit the 256 MB cache).
+// Few chunks leave CUs idle, many repeat warm-up planes; small regions repeat halos.
+static double tb_cost(const TbShapeInfo &s, const TbGeom &g, int cus) {
+  const int64_t n = cdiv(g.total, cus), full = n / s.resident, rest = n % s.resident;
+  const double it = (double)(g.A + 2 * TBH);
+  const double one = std::max(s.t1, (double)rest * s.tau);
+  const double cu = it * ((double)full * s.resident * s.tau + (rest ? one : 0.0));
+  const double sites = (double)g.N * (double)g.N * (double)(g.a_hi - g.a_lo);
+  const double loads = 16.0 * (double)g.ntb * g.ntc * g.n_ac * s.rb * s.rc * it, stores = 16.0 * sites;
+  const double bw = 32.0 * sites <= 256e6 ? 1.2 * s.bw : s.bw;
+  return std::max(cu, (loads + stores) / bw);
+}
+
+// The cheapest (shape, chunk) of a launch, or the cheapest shape for a given chunk. With
+// `near`, also every chunk length whose best shape costs at most near_pct percent more,
+// cheapest first. Chunk lengths are the ceil(planes / k); there are about 2 sqrt(planes).
+// Measured on MI355X (us a step, FP64; before: one rule over 32 x 32 regions with a halo
+// of four): N=32 20.5 -> 5.2, 64 20.7 -> 7.8, 128 31.6 -> 19.5, 200 80 -> 57, 250 152 ->
+// 113, 300 258 -> 192, 384 467 -> 394, 512 1239 -> 895.
+static TbGeom tb_plan(int family, int64_t N, int chunk, int64_t a_lo, int64_t a_hi, int64_t NA,
+                      std::vector<int> *near = nullptr, int near_pct = 0) {
+  const std::vector<TbShapeInfo> &shapes = tb_shapes(family);
+  const int cus = tb_cus();
+  const int64_t planes = a_hi - a_lo;
+  TbGeom best{};
+  double best_cost = -1.0;
+  std::vector<std::pair<double, int>> costs;
+  auto try_chunk = [&](int A) {
+    double least = -1.0;
+    for (size_t i = 0; i < shapes.size(); ++i) {
+      const TbGeom g = tb_geom(family, (int)i, N, A, a_lo, a_hi, NA);
+      const double c = tb_cost(shapes[i], g, cus);
+      if (least < 0.0 || c < least) least = c;
+      if (best_cost < 0.0 || c < best_cost) {
+        best = g;
+        best_cost = c;
+      }
+    }
+    if (near) costs.emplace_back(least, A);
+  };
+  if (chunk > 0) {
+    try_chunk(chunk);
+    return best;
   }
-  int64_t pick = 1;
-  for (int64_t k = 1; k <= kmax; ++k)
-    if (cost[k] >= 0 && cost[k] * 100 <= best * 102) pick = k;
-  if (cost_out) *cost_out = best;
-  if (near)  // every chunk length within near_pct percent of the best cost, longest first
-    for (int64_t k = 1; k <= kmax; ++k)
-      if (cost[k] >= 0 && cost[k] * 100 <= best * (100 + near_pct)) near->push_back((int)cdiv(planes, k));
-  return (int)cdiv(planes, pick);
+  for (int64_t k = 1; k <= planes;) {  // every distinct ceil(planes / k)
+    const int64_t A = cdiv(planes, k);
+    try_chunk((int)A);
+    k = A > 1 ? (planes + A - 2) / (A - 1) : planes + 1;  // the first k of a shorter chunk
+  }
+  if (near) {
+    std::sort(costs.begin(), costs.end());
+    for (const auto &c : costs)
+      if (c.first * 100.0 <= best_cost * (100 + near_pct)) near->push_back(c.second);
+  }
+  return best;
 }
 
 // Where the FP32-comp run puts its second hi and lo arrays in the work buffer: at the
 // first address from `from` on with the same residue modulo TB_ALIGN_SLACK as the
-// caller's array `like`. Measured at N=512: hi, lo and the second pair at relative
-// offsets that are not multiples of 4 KB (one allocation carved 256 B - 2 KB apart)
-// ran 72-83 GSite*step/s against 84-90 at multiples of 4 KB. Matching residues keeps
-// each array's offset to its partner of the other step a multiple of 4 KB; the work
-// buffer carries the slack (cf_rk4_tb_work_bytes).
+// caller's array `like`, so that each array's offset to its partner of the other step is
+// a multiple of 4 KB (offsets that are not cost up to 20%; the work buffer carries the
+// slack, cf_rk4_tb_work_bytes).
 constexpr size_t TB_ALIGN_SLACK = 4096;
 static float *same_residue(void *from, const float *like) {
   const uintptr_t f = reinterpret_cast<uintptr_t>(from), l = reinterpret_cast<uintptr_t>(like);
   return reinterpret_cast<float *>(f + ((l - f) & (TB_ALIGN_SLACK - 1)));
 }
 
-// Geometry of the FP32-comp kernel (its region shape), chunk <= 0: the cost model's.
-static TbGeom tb_f32c_geom(int64_t N, int chunk) {
-  return tb_geom(N, chunk > 0 ? chunk : tb_default_chunk(N, TB_F32C_RB, TB_F32C_RC), TB_F32C_RB, TB_F32C_RC);
-}
-// Region shape of the single-precision-stencil kernel for `planes` output planes of an
-// N^2 cross-section: 24 x 40 unless the cost model's launch over 32 x 32 regions is more
-// than TB_F32S_SQUARE_GAIN percent cheaper (at N=192 and 384 its 8 x 8 / 16 x 16 tiles
-// fill the CUs in one round where 24 x 40 needs more rounds of shorter chunks; measured
-// at N=384: 105.7 GSite*step/s against 97.3). Elsewhere 24 x 40 is faster at equal cost
-// (N=256: 109.8 against 95.4; 768: 108.3 against 92.6, a cost ratio of 1.14).
-constexpr int TB_F32S_SQUARE_GAIN = 20;
-static void tb_f32s_shape(int64_t N, int64_t planes, int *RB, int *RC) {
-  int64_t c_strip = 0, c_square = 0;
-  tb_default_chunk(N, TB_F32S_RB, TB_F32S_RC, planes, &c_strip);
-  tb_default_chunk(N, TB_F32C_RB, TB_F32C_RC, planes, &c_square);
-  const bool square = c_square * (100 + TB_F32S_SQUARE_GAIN) < c_strip * 100;
-  *RB = square ? TB_F32C_RB : TB_F32S_RB;
-  *RC = square ? TB_F32C_RC : TB_F32S_RC;
-}
 // Default chunk of the single-precision-stencil step per device and lattice size, set by
 // cf_rk4_tb_tune_pace (chunk <= 0) or cf_rk4_tb_set_chunk; absent: the cost model's.
 static std::mutex g_chunk_mu;
@@ -222,29 +236,56 @@ static int tb_f32s_tuned_chunk(int64_t N) {
   return it == g_chunk.end() ? 0 : it->second;
 }
 
-// ... and of the single-precision-stencil kernel (sa) or the FP32-comp one.
+static TbGeom tb_f64_geom(int64_t N, int chunk) { return tb_plan(TB_FAM_F64, N, chunk, 0, N, N); }
+
+// ... of the single-precision-stencil kernel (sa) or the FP32-comp one.
 static TbGeom tb_comp_geom(bool sa, int64_t N, int chunk) {
-  if (!sa) return tb_f32c_geom(N, chunk);
-  int RB = 0, RC = 0;
-  tb_f32s_shape(N, N, &RB, &RC);
+  if (!sa) return tb_plan(TB_FAM_F32C, N, chunk, 0, N, N);
   if (chunk <= 0) chunk = tb_f32s_tuned_chunk(N);
-  return tb_geom(N, chunk > 0 ? chunk : tb_default_chunk(N, RB, RC), RB, RC);
+  return tb_plan(TB_FAM_F32S, N, chunk, 0, N, N);
 }
 
-template <class T, bool F32C>
-static cf_status tb_launch(const TbGeom &g, const TbStep &k, const T *xin, const float *lin, T *xout,
-                           float *lout, hipStream_t st) {
-  if constexpr (!F32C) {
-    if (k.lam != 0.0)
-      hipLaunchKernelGGL(k_rk4_tb_ring<true>, dim3(g.total), dim3(1024), 0, st, g, k, xin, xout);
-    else
-      hipLaunchKernelGGL(k_rk4_tb_ring<false>, dim3(g.total), dim3(1024), 0, st, g, k, xin, xout);
-  } else {
-    if (k.lam != 0.0)
-      hipLaunchKernelGGL((k_rk4_tb<T, F32C, true>), dim3(g.total), dim3(1024), 0, st, g, k, xin, lin, xout, lout);
-    else
-      hipLaunchKernelGGL((k_rk4_tb<T, F32C, false>), dim3(g.total), dim3(1024), 0, st, g, k, xin, lin, xout, lout);
+// The region class of a lattice size that cf_rk4_tb_f32s_region reports: 24 x 40 unless
+// rounds x (chunk + 8) of a launch over 32 x 32 regions with halos of four is more than
+// 20% lower. Callers file tuned settings by it; the kernel's own shapes are tb_shapes'.
+static void tb_f32s_class(int64_t N, int *rows, int *cols) {
+  const int cus = tb_cus();
+  auto least = [&](int64_t tb, int64_t tc) {
+    const int64_t tiles = cdiv(N, N < tb ? N : tb) * cdiv(N, N < tc ? N : tc);
+    int64_t best = -1;
+    for (int64_t k = 1; k <= (N / 8 > 1 ? N / 8 : 1); ++k) {
+      const int64_t ch = cdiv(N, k), c = cdiv(tiles * cdiv(N, ch), cus) * (ch + 8);
+      if (cdiv(N, ch) == k && (best < 0 || c < best)) best = c;
+    }
+    return best;
+  };
+  const bool square = least(24, 24) * 120 < least(16, 32) * 100;
+  *rows = square ? 32 : 24;
+  *cols = square ? 32 : 40;
+}
+
+template <int MODE, class SH, int WAVES>
+static void tb_launch_shape(const TbGeom &g, const TbStep &k, const TbStepF &kf, const void *xin, const float *lin,
+                            void *xout, float *lout, hipStream_t st) {
+  const dim3 grid((unsigned)g.total), block(SH::NT);
+  const bool lam = k.lam != 0.0;
+  if constexpr (MODE == TB_F32S) {
+    if (g.pace > 0) {
+      if (lam) hipLaunchKernelGGL((k_rk4_tb<MODE, true, SH, WAVES, true>), grid, block, 0, st, g, k, kf, xin, lin, xout, lout);
+      else hipLaunchKernelGGL((k_rk4_tb<MODE, false, SH, WAVES, true>), grid, block, 0, st, g, k, kf, xin, lin, xout, lout);
+      return;
+    }
   }
+  if (lam) hipLaunchKernelGGL((k_rk4_tb<MODE, true, SH, WAVES, false>), grid, block, 0, st, g, k, kf, xin, lin, xout, lout);
+  else hipLaunchKernelGGL((k_rk4_tb<MODE, false, SH, WAVES, false>), grid, block, 0, st, g, k, kf, xin, lin, xout, lout);
+}
+
+static cf_status tb_launch_f64(const TbGeom &g, const TbStep &k, const double *xin, double *xout, hipStream_t st) {
+  const TbStepF kf{};
+  if (g.shape == 0) tb_launch_shape<TB_F64, TbS12x20, 4>(g, k, kf, xin, nullptr, xout, nullptr, st);
+  else if (g.shape == 1) tb_launch_shape<TB_F64, TbS14x36, 4>(g, k, kf, xin, nullptr, xout, nullptr, st);
+  else if (g.shape == 2) tb_launch_shape<TB_F64, TbS28x36, 4>(g, k, kf, xin, nullptr, xout, nullptr, st);
+  else tb_launch_shape<TB_F64, TbS30x68, 4>(g, k, kf, xin, nullptr, xout, nullptr, st);
   CF_LAUNCHED();
   return CF_OK;
 }
@@ -264,30 +305,24 @@ static TbStepF tb_step_f32(const TbStep &k) {
   return f;
 }
 
-template <int RB, int RC>
-static void tb_launch_sa_shape(const TbGeom &g, const TbStep &k, const TbStepF &kf, const float *xin,
-                               const float *lin, float *xout, float *lout, hipStream_t st) {
-  const bool lam = k.lam != 0.0, paced = g.pace > 0;
-  const dim3 grid(g.total), block(1024);
-  if (lam && paced)
-    hipLaunchKernelGGL((k_rk4_tb_sa<true, true, RB, RC>), grid, block, 0, st, g, k, kf, xin, lin, xout, lout);
-  else if (lam)
-    hipLaunchKernelGGL((k_rk4_tb_sa<true, false, RB, RC>), grid, block, 0, st, g, k, kf, xin, lin, xout, lout);
-  else if (paced)
-    hipLaunchKernelGGL((k_rk4_tb_sa<false, true, RB, RC>), grid, block, 0, st, g, k, kf, xin, lin, xout, lout);
-  else
-    hipLaunchKernelGGL((k_rk4_tb_sa<false, false, RB, RC>), grid, block, 0, st, g, k, kf, xin, lin, xout, lout);
+static cf_status tb_launch_f32c(const TbGeom &g, const TbStep &k, const float *xin, const float *lin, float *xout,
+                                float *lout, hipStream_t st) {
+  const TbStepF kf{};
+  if (g.shape == 0) tb_launch_shape<TB_F32C, TbC14x36, 4>(g, k, kf, xin, lin, xout, lout, st);
+  else if (g.shape == 1) tb_launch_shape<TB_F32C, TbC28x36, 4>(g, k, kf, xin, lin, xout, lout, st);
+  else tb_launch_shape<TB_F32C, TbC22x68, 3>(g, k, kf, xin, lin, xout, lout, st);
+  CF_LAUNCHED();
+  return CF_OK;
 }
 
 static cf_status tb_launch_sa(const TbGeom &g, const TbStep &k, const float *xin, const float *lin, float *xout,
                               float *lout, hipStream_t st) {
   const TbStepF kf = tb_step_f32(k);
-  if (g.rb == TB_F32S_RB && g.rc == TB_F32S_RC)
-    tb_launch_sa_shape<TB_F32S_RB, TB_F32S_RC>(g, k, kf, xin, lin, xout, lout, st);
-  else if (g.rb == TB_F32C_RB && g.rc == TB_F32C_RC)
-    tb_launch_sa_shape<TB_F32C_RB, TB_F32C_RC>(g, k, kf, xin, lin, xout, lout, st);
-  else
-    CF_REQUIRE(false, "single-precision stencil: no kernel for %d x %d regions", g.rb, g.rc);
+  if (g.shape == 0) tb_launch_shape<TB_F32S, TbS12x20, 4>(g, k, kf, xin, lin, xout, lout, st);
+  else if (g.shape == 1) tb_launch_shape<TB_F32S, TbS14x36, 4>(g, k, kf, xin, lin, xout, lout, st);
+  else if (g.shape == 2) tb_launch_shape<TB_F32S, TbS28x36, 4>(g, k, kf, xin, lin, xout, lout, st);
+  else if (g.shape == 3) tb_launch_shape<TB_F32S, TbS30x68, 4>(g, k, kf, xin, lin, xout, lout, st);
+  else tb_launch_shape<TB_F32S, TbS15x132, 4>(g, k, kf, xin, lin, xout, lout, st);
   CF_LAUNCHED();
   return CF_OK;
 }
@@ -306,6 +341,17 @@ static cf_status tb_check(const cf_kg_params *p) {
   return CF_OK;
 }
 
+template <int VAR>
+static void tb_launch_var(const TbGeom &g, const TbStep &k, const double *xin, double *xout, const double *psi,
+                          const TbPsi &cp, hipStream_t st) {
+  if (g.shape == 0)
+    hipLaunchKernelGGL((k_rk4_tb_var<VAR, TbC14x36>), dim3((unsigned)g.total), dim3(TbC14x36::NT), 0, st, g, k, xin,
+                       xout, psi, cp);
+  else
+    hipLaunchKernelGGL((k_rk4_tb_var<VAR, TbC28x36>), dim3((unsigned)g.total), dim3(TbC28x36::NT), 0, st, g, k, xin,
+                       xout, psi, cp);
+}
+
 cf_status tb_step_variant(int var, const cf_kg_params *p, double f_a, const double *psi, const double *xin,
                           double *xout, double t, double dt, int chunk, hipStream_t st, const TbPsi *cps) {
   CF_TRY(tb_check(p));
@@ -316,19 +362,14 @@ cf_status tb_step_variant(int var, const cf_kg_params *p, double f_a, const doub
   const size_t n = 2 * (size_t)p->N * p->N * p->N;
   CF_REQUIRE(xin && xout && disjoint(xin, xout, n * sizeof(double)),
              "temporally blocked variant step: null or overlapping state buffers");
-  const TbGeom g = tb_geom(p->N, chunk > 0 ? chunk : tb_default_chunk(p->N));
+  const TbGeom g = tb_plan(TB_FAM_VAR, p->N, chunk, 0, p->N, p->N);
   TbStep k = tb_step_host(p, t, dt);
   k.fa2 = f_a * f_a;
   const TbPsi cp = cps ? *cps : TbPsi{};
-  if (var == TB_FIXED_CURVATURE)
-    hipLaunchKernelGGL(k_rk4_tb_var<TB_FIXED_CURVATURE>, dim3(g.total), dim3(1024), 0, st, g, k, xin, xout, psi, cp);
-  else if (var == TB_SQRT_POTENTIAL)
-    hipLaunchKernelGGL(k_rk4_tb_var<TB_SQRT_POTENTIAL>, dim3(g.total), dim3(1024), 0, st, g, k, xin, xout, psi, cp);
-  else if (var == TB_COMOVING)
-    hipLaunchKernelGGL(k_rk4_tb_var<TB_COMOVING>, dim3(g.total), dim3(1024), 0, st, g, k, xin, xout, psi, cp);
-  else
-    hipLaunchKernelGGL(k_rk4_tb_var<TB_APPROX_COMOVING>, dim3(g.total), dim3(1024), 0, st, g, k, xin, xout, psi,
-                       cp);
+  if (var == TB_FIXED_CURVATURE) tb_launch_var<TB_FIXED_CURVATURE>(g, k, xin, xout, psi, cp, st);
+  else if (var == TB_SQRT_POTENTIAL) tb_launch_var<TB_SQRT_POTENTIAL>(g, k, xin, xout, psi, cp, st);
+  else if (var == TB_COMOVING) tb_launch_var<TB_COMOVING>(g, k, xin, xout, psi, cp, st);
+  else tb_launch_var<TB_APPROX_COMOVING>(g, k, xin, xout, psi, cp, st);
   CF_LAUNCHED();
   return CF_OK;
 }
@@ -366,7 +407,7 @@ static cf_status tb_pace_store(const TbGeom &g, int pace) {
 // the single-precision stencil (sa = true).
 static cf_status tb_launch_comp(bool sa, const TbGeom &g, const TbStep &k, const float *xin, const float *lin,
                                 float *xout, float *lout, hipStream_t st) {
-  return sa ? tb_launch_sa(g, k, xin, lin, xout, lout, st) : tb_launch<float, true>(g, k, xin, lin, xout, lout, st);
+  return sa ? tb_launch_sa(g, k, xin, lin, xout, lout, st) : tb_launch_f32c(g, k, xin, lin, xout, lout, st);
 }
 
 static cf_status tb_run_comp(const char *name, bool sa, const cf_kg_params *p, float *hi, float *lo, double t0,
@@ -439,16 +480,13 @@ static cf_status tb_step_comp_slab(const char *name, bool sa, const cf_kg_params
                                    double dt, int chunk, hipStream_t st) {
   CF_TRY(tb_check(p));
   CF_REQUIRE(n_planes >= 1 && n_planes <= p->N, "%s: n_planes=%lld outside 1..N", name, (long long)n_planes);
-  const int64_t NA = n_planes + 2 * TBH;
+  const int64_t NA = n_planes + 2 * TB_GHOST;
   const size_t b = 2 * (size_t)NA * p->N * p->N * sizeof(float);
   CF_REQUIRE(hi_in && lo_in && hi_out && lo_out, "%s: null buffer", name);
   CF_REQUIRE(disjoint(hi_in, lo_in, b) && disjoint(hi_out, lo_out, b) && disjoint(hi_in, hi_out, b) &&
                  disjoint(hi_in, lo_out, b) && disjoint(lo_in, hi_out, b) && disjoint(lo_in, lo_out, b),
              "%s: overlapping buffers", name);
-  int RB = TB_F32C_RB, RC = TB_F32C_RC;
-  if (sa) tb_f32s_shape(p->N, n_planes, &RB, &RC);
-  TbGeom g = tb_geom(p->N, chunk > 0 ? chunk : tb_default_chunk(p->N, RB, RC, n_planes), RB, RC, TBH,
-                     TBH + n_planes, NA);
+  TbGeom g = tb_plan(sa ? TB_FAM_F32S : TB_FAM_F32C, p->N, chunk, TB_GHOST, TB_GHOST + n_planes, NA);
   if (sa) CF_TRY(tb_pace_lookup(g));  // the pace tuned for this lattice size and chunk, if any
   return tb_launch_comp(sa, g, tb_step_host(p, t, dt), hi_in, lo_in, hi_out, lo_out, st);
 }
@@ -471,12 +509,11 @@ cf_status cf_rk4_run_tb_f64(const cf_kg_params *p, double *x, double t0, int64_t
   CF_REQUIRE(x && work && disjoint(x, work, 2 * (size_t)p->N * p->N * p->N * sizeof(double)),
              "cf_rk4_run_tb_f64: null or overlapping buffer");
   CF_REQUIRE(n_steps >= 0, "cf_rk4_run_tb_f64: negative step count");
-  const TbGeom g = tb_geom(p->N, chunk > 0 ? chunk : tb_default_chunk(p->N));
+  const TbGeom g = tb_f64_geom(p->N, chunk);
   double *bufs[2] = {x, (double *)work};
   for (int64_t s = 0; s < n_steps; ++s) {
     const double t = t0 + static_cast<double>(k0 + s) * dt;
-    CF_TRY((tb_launch<double, false>(g, tb_step_host(p, t, dt), bufs[s & 1], nullptr, bufs[(s + 1) & 1], nullptr,
-                                      S(stream))));
+    CF_TRY(tb_launch_f64(g, tb_step_host(p, t, dt), bufs[s & 1], bufs[(s + 1) & 1], S(stream)));
   }
   if (n_steps & 1) {
     const size_t bytes = 2 * (size_t)p->N * p->N * p->N * sizeof(double);
@@ -497,12 +534,11 @@ cf_status cf_rk4_run_tb_f64_noalloc(const cf_kg_params *p, double *x, double t0,
   CF_TRY(scratch_on_current_device(&work));
   const size_t bytes = 2 * (size_t)p->N * p->N * p->N * sizeof(double);
   CF_REQUIRE(disjoint(x, work, bytes), "cf_rk4_run_tb_f64_noalloc: the state overlaps the library's buffer");
-  const TbGeom g = tb_geom(p->N, chunk > 0 ? chunk : tb_default_chunk(p->N));
+  const TbGeom g = tb_f64_geom(p->N, chunk);
   double *bufs[2] = {x, work};
   for (int64_t s = 0; s < n_steps; ++s) {
     const double t = t0 + static_cast<double>(k0 + s) * dt;
-    CF_TRY((tb_launch<double, false>(g, tb_step_host(p, t, dt), bufs[s & 1], nullptr, bufs[(s + 1) & 1], nullptr,
-                                      S(stream))));
+    CF_TRY(tb_launch_f64(g, tb_step_host(p, t, dt), bufs[s & 1], bufs[(s + 1) & 1], S(stream)));
   }
   if (n_steps & 1) CF_HIP(hipMemcpyAsync(x, work, bytes, hipMemcpyDeviceToDevice, S(stream)));
   return CF_OK;
@@ -524,8 +560,8 @@ cf_status cf_rk4_step_tb_f64(const cf_kg_params *p, const double *x_in, double *
   const size_t n = 2 * (size_t)p->N * p->N * p->N;
   CF_REQUIRE(x_in && x_out && disjoint(x_in, x_out, n * sizeof(double)),
              "cf_rk4_step_tb_f64: null or overlapping state buffers");
-  const TbGeom g = tb_geom(p->N, chunk > 0 ? chunk : tb_default_chunk(p->N));
-  return tb_launch<double, false>(g, tb_step_host(p, t, dt), x_in, nullptr, x_out, nullptr, S(stream));
+  const TbGeom g = tb_f64_geom(p->N, chunk);
+  return tb_launch_f64(g, tb_step_host(p, t, dt), x_in, x_out, S(stream));
 }
 
 cf_status cf_rk4_step_tb_f64_slab(const cf_kg_params *p, int64_t n_planes, const double *x_in, double *x_out,
@@ -533,16 +569,15 @@ cf_status cf_rk4_step_tb_f64_slab(const cf_kg_params *p, int64_t n_planes, const
   CF_TRY(tb_check(p));
   CF_REQUIRE(n_planes >= 1 && n_planes <= p->N, "cf_rk4_step_tb_f64_slab: n_planes=%lld outside 1..N",
              (long long)n_planes);
-  const int64_t NA = n_planes + 2 * TBH;  // own planes and four ghost planes on each side
+  const int64_t NA = n_planes + 2 * TB_GHOST;  // own planes and four ghost planes on each side
   const size_t bytes = 2 * (size_t)NA * p->N * p->N * sizeof(double);
   CF_REQUIRE(x_in && x_out && disjoint(x_in, x_out, bytes), "cf_rk4_step_tb_f64_slab: null or overlapping slabs");
-  // A unit reads planes a0 - 4 .. a1 + 3 of its chunk (wrapping at NA only in the ring's
-  // dead prefetches past a1 + 3), all inside the slab for chunks within [4, 4 + n_planes).
-  const TbGeom g = tb_geom(p->N, chunk > 0 ? chunk : tb_default_chunk(p->N, TBR, TBR, n_planes), TBR, TBR, TBH,
-                           TBH + n_planes, NA);
-  return tb_launch<double, false>(g, tb_step_host(p, t, dt), x_in, nullptr, x_out, nullptr, S(stream));
+  // A unit's stored sites depend on planes a0 - 2 .. a1 + 1 of its chunk, all inside the
+  // slab for chunks within [4, 4 + n_planes); it loads no plane but those and the two after
+  // them, and its lattice offsets wrap at NA.
+  const TbGeom g = tb_plan(TB_FAM_F64, p->N, chunk, TB_GHOST, TB_GHOST + n_planes, NA);
+  return tb_launch_f64(g, tb_step_host(p, t, dt), x_in, x_out, S(stream));
 }
-
 
 cf_status cf_rk4_step_tb_f32c(const cf_kg_params *p, const float *hi_in, const float *lo_in, float *hi_out,
                               float *lo_out, double t, double dt, int chunk, cf_stream stream) {
@@ -567,21 +602,18 @@ cf_status cf_rk4_step_tb_f32s_slab(const cf_kg_params *p, int64_t n_planes, cons
 }
 
 // Pacing of the single-precision-stencil step: time the step of this lattice at a
-// range of paces and keep one with margin. Below the fastest pace the rate falls (over
-// 32 x 32 regions it fell off a cliff: blocks that are not held back drift out of step;
-// over the 24 x 40 regions the kernel uses now, by 1-3% per tick) and above it declines
-// slowly, and where the fall begins moves with the clock: a pace one or two ticks above a
-// cliff measured fast while tuning and then ran 10-15% slow. So each pace P is scored by
-// the slowest of P - TB_PACE_MARGIN .. P, and the best score wins (at equal scores the
-// larger pace); unpaced wins if it is as fast.
+// range of paces and keep one with margin. Where pacing helps, the rate falls below the
+// fastest pace and declines slowly above it, and where the fall begins moves with the
+// clock, so each pace P is scored by the slowest of P - TB_PACE_MARGIN .. P, and the best
+// score wins (at equal scores the larger pace); unpaced wins if it is as fast. With the
+// 24 x 40 regions and the halo of four that the kernel had before, pacing gave 101 -> 109
+// GSite*step/s at N=512; the large regions drift less and gain little or nothing.
 constexpr int TB_PACE_MARGIN = 2;
 
 // Chunk lengths within this many percent of the cost model's best that the pace tuner
-// tries when the caller leaves the chunk to it. At N=512 (24 x 40 regions) these are 512,
-// 256, 171 and 128 planes; measured tuned: 109.0-110.4, 105.9-107.2, 108.4-109.3 and
-// 106.9-108.5 GSite*step/s: the drift of the blocks, which the cost model does not
-// see, depends on the chunk length and how the rounds of blocks line up.
+// tries when the caller leaves the chunk to it, the cheapest TB_CHUNK_NEAR_MAX of them.
 constexpr int TB_CHUNK_NEAR_PCT = 5;
+constexpr size_t TB_CHUNK_NEAR_MAX = 4;
 
 // Pace of launches over geometry g: the pick and its score (the slowest ms per step over
 // the picked pace and the TB_PACE_MARGIN paces below it; the unpaced ms for pick 0).
@@ -644,13 +676,12 @@ cf_status cf_rk4_tb_tune_pace(const cf_kg_params *p, const float *hi, const floa
                  disjoint(hi, n * sizeof(float), work, wb) && disjoint(lo, n * sizeof(float), work, wb),
              "cf_rk4_tb_tune_pace: null or overlapping buffer");
   hipStream_t st = S(stream);
-  int RB = 0, RC = 0;
-  tb_f32s_shape(p->N, p->N, &RB, &RC);
   std::vector<int> chunks;
   if (chunk > 0)
     chunks.push_back(chunk);
   else
-    tb_default_chunk(p->N, RB, RC, p->N, nullptr, &chunks, TB_CHUNK_NEAR_PCT);
+    (void)tb_plan(TB_FAM_F32S, p->N, 0, 0, p->N, p->N, &chunks, TB_CHUNK_NEAR_PCT);
+  if (chunks.size() > TB_CHUNK_NEAR_MAX) chunks.resize(TB_CHUNK_NEAR_MAX);
   float *ho = same_residue(work, hi), *lw = same_residue(ho + n, lo);
   const TbStep k = tb_step_host(p, t, dt);
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -662,7 +693,7 @@ cf_status cf_rk4_tb_tune_pace(const cf_kg_params *p, const float *hi, const floa
   cf_status rc = CF_OK;
   std::vector<TbGeom> picks;
   for (size_t i = 0; i < chunks.size() && rc == CF_OK; ++i) {
-    TbGeom g = tb_geom(p->N, chunks[i], RB, RC);
+    TbGeom g = tb_plan(TB_FAM_F32S, p->N, chunks[i], 0, p->N, p->N);
     float score = 0.0f;
     rc = tb_tune_pace_geom(g, k, hi, lo, ho, lw, st, e0, e1, &g.pace, &score);
     if (rc == CF_OK) rc = tb_pace_store(g, g.pace);
@@ -740,7 +771,7 @@ int cf_rk4_tb_get_chunk(int64_t N) {
 cf_status cf_rk4_tb_f32s_region(int64_t N, int *rows, int *cols) {
   CF_REQUIRE(valid_N(N), "cf_rk4_tb_f32s_region: unsupported lattice size N=%lld", (long long)N);
   CF_REQUIRE(rows && cols, "cf_rk4_tb_f32s_region: null output");
-  tb_f32s_shape(N, N, rows, cols);
+  tb_f32s_class(N, rows, cols);
   return CF_OK;
 }
 

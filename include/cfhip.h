@@ -157,9 +157,8 @@ cf_status cf_rk4_run_tb_f32c(const cf_kg_params *p, float *hi_dev, float *lo_dev
  * (hi + lo) + (increment + dt/6 k4) is formed in double and split into hi and lo. The
  * increment weights stay double, so the scheme has no drift from rounded step
  * lengths. Work buffer and placement as cf_rk4_run_tb_f32c
- * (cf_rk4_tb_work_bytes(N, CF_PREC_F32S)). The launch covers the lattice with 24 x 40
- * or 32 x 32 regions (16 x 32 or 24 x 24 tiles), whichever the chunk cost model favours
- * for N and the device's CU count; both give the same bits. */
+ * (cf_rk4_tb_work_bytes(N, CF_PREC_F32S)). The launch covers the lattice with tiles
+ * whose size a cost model picks for N and the device's CU count; all give the same bits. */
 cf_status cf_rk4_run_tb_f32s(const cf_kg_params *p, float *hi_dev, float *lo_dev, double t0, int64_t k0,
                              int64_t n_steps, double dt, int chunk, void *work_dev, cf_stream stream);
 /* Pacing of the single-precision-stencil step (no reference counterpart). Its blocks
@@ -174,8 +173,8 @@ cf_status cf_rk4_run_tb_f32s(const cf_kg_params *p, float *hi_dev, float *lo_dev
  * the pace P whose slowest of P-2..P is fastest (the rate falls just below the best
  * pace, so the pick keeps a margin above it; unpaced if that is as fast), and
  * returns it in *pace_out (may be null); it synchronises the stream. With chunk <= 0
- * it does so for each chunk length whose launch the cost model rates within 5% of its
- * best (at N=512 four of them, about 1400 steps in all), keeps every chunk's pace, and
+ * it does so for the chunk lengths whose launches the cost model rates within 5% of its
+ * best (at most four, about 1400 steps in all), keeps every chunk's pace, and
  * makes the chunk with the fastest score the default for N on this device (the chunk
  * that chunk <= 0 means from then on in the f32s runs, steps and pace calls), its pace
  * the one returned. Pacing and chunking change timing only, never results.
@@ -190,9 +189,10 @@ int cf_rk4_tb_get_pace(int64_t N, int chunk);
  * set or the cost model's), -1 for an unsupported N. */
 cf_status cf_rk4_tb_set_chunk(int64_t N, int chunk);
 int cf_rk4_tb_get_chunk(int64_t N);
-/* Region shape (rows along b x columns along c, halo included) over which
- * cf_rk4_run_tb_f32s and cf_rk4_step_tb_f32s cover an N^3 lattice on the current device:
- * 24 x 40 or 32 x 32 (no reference counterpart; the kernel's name carries it). */
+/* Region class of the f32s step for N on the current device, 24 x 40 or 32 x 32 (rows
+ * along b x columns along c): the shape whose launch over regions with four-site halos
+ * the chunk cost is lower for (no reference counterpart). A name to file tuned settings
+ * under; the step's own tiles are chosen per launch and may be larger. */
 cf_status cf_rk4_tb_f32s_region(int64_t N, int *rows, int *cols);
 /* cf_rk4_run_tb_f64 without a work buffer and without any allocation. No counterpart
  * in the reference: it is for callers that cannot allocate device memory (code
@@ -273,11 +273,13 @@ cf_status cf_ensemble_init_grf(cf_ensemble *e, const uint32_t *seeds, int kind, 
 cf_status cf_ensemble_set_plan(cf_ensemble *e, int64_t N, int chunk, int grid);
 cf_status cf_ensemble_get_plan(const cf_ensemble *e, int64_t N, int *chunk, int *grid);
 /* Region shape of the blocks that advance lattices of size N (rows along b x columns
- * along c): CF_ENS_REGION_32X32 (24 x 24 output tiles, the default) or
- * CF_ENS_REGION_24X40 (16 x 32 tiles, which divide N = 64 and 128; 24 x 24 tiles
- * leave 27% of the covered area outside such lattices). Same bits either way. */
+ * along c, halo of two sites included): CF_ENS_REGION_32X32 (28 x 28 output tiles, the
+ * default), CF_ENS_REGION_24X40 (20 x 36) or CF_ENS_REGION_28X36 (24 x 32 tiles, which
+ * divide N = 96 and whose rows fall on 128-byte lines for N = 64, 96 and 128). Same bits
+ * in all of them. */
 #define CF_ENS_REGION_32X32 0
 #define CF_ENS_REGION_24X40 1
+#define CF_ENS_REGION_28X36 2
 cf_status cf_ensemble_set_region(cf_ensemble *e, int64_t N, int region);
 cf_status cf_ensemble_get_region(const cf_ensemble *e, int64_t N, int *region);
 /* Autotuner: times candidate grids (persistent and flat), then per N candidate
