@@ -1,5 +1,11 @@
-// cf_spectrum.hip -- hipFFT wrapper, deterministic spectrum binning, Gaussian
+// cf_spectrum.hip -- lattice transforms, deterministic spectrum binning, Gaussian
 // random fields and the fixed-order rms rescale.
+//
+// Transforms. Sizes without a prime factor above 7 run the passes of cf_fft.hpp, which
+// read the caller's field without changing it, fold the powers of a spectrum in the last
+// pass (no half spectrum is written for one) and scale modes in the first pass of an
+// inverse transform. Other sizes go through hipFFT. One power spectrum at N=256: 209 us
+// of transform, 18 of input copy and 40 of row binning before.
 //
 // Binning without atomics. The half spectrum has N*N*(N/2+1) entries; entry
 // (a,b,c) belongs to bin s = a'^2 + b'^2 + c^2 with x' = min(x, N-x), and counts
@@ -19,18 +25,23 @@
 #include <vector>
 
 #include "cf_common.hpp"
+#include "cf_fft.hpp"
 
 struct cf_spectrum_plan {
   int64_t N = 0, H = 0, nb = 0, nhalf = 0;
+  cf::FftPlan fft;               // fft.N != 0: this size's own passes; otherwise hipFFT below
+  int64_t pitch = 0;             // complex entries per row of cbuf0 / cbuf1
   hipfftHandle d2z = 0, z2d = 0;
   bool have_d2z = false, have_z2d = false;
   void *work = nullptr;
   double *rbuf = nullptr;        // N^3 real scratch
-  double *cbuf0 = nullptr;       // half-spectrum scratch (2*nhalf doubles)
-  double *cbuf1 = nullptr;       // second half-spectrum scratch
+  double *cbuf0 = nullptr;       // half-spectrum scratch (N*N*pitch entries)
+  double *cbuf1 = nullptr;       // second half-spectrum scratch, or two fields' folded powers
   int64_t nr = 0;                // row classes r = as^2 + bs^2 <= 2 (N/2)^2
   int32_t *roff = nullptr;       // nr+1 offsets into rows
   int32_t *rows = nullptr;       // the N^2 rows (a*N + b) of the half spectrum sorted by r
+  int32_t *foff = nullptr;       // the same for the (N/2 + 1) N rows (a'*N + b) of folded powers
+  int32_t *frows = nullptr;
   double *red = nullptr;         // reduction scratch (RED_BLOCKS + 1 doubles)
   double *bins = nullptr;        // one spectrum (nb doubles) for callers inside the library
 };
@@ -58,6 +69,8 @@ constexpr int RED_BLOCKS = 1024;
 //   step B: P(s) = sum_{c ascending} Q[c][s - c^2], coalesced over consecutive s.
 // Fixed summation orders, no atomics: bit-reproducible.
 constexpr int BIN_LDS = 4096;  // doubles of the step-A tile (32 KB: several blocks per CU)
+constexpr int BIN_MAX_RB = 256;  // row classes per block
+constexpr int BIN_LIST = 1024;   // rows of a block's classes kept in LDS
 constexpr int BIN_CQ = 9;      // 64-column chunks of a row: H = N/2 + 1 <= 513
 
 // CQ: 64-column chunks per row (CQ * 64 >= H). Each wavefront keeps bin_group rows
@@ -69,19 +82,36 @@ constexpr int bin_group(bool mode, int cq) {
   return g < 1 ? 1 : (g > 4 ? 4 : g);
 }
 
-template <bool MODE, int CQ>
-__global__ __launch_bounds__(256) void k_bin_rows(const double2 *__restrict__ fk, const double2 *__restrict__ dk,
+// Rows of `pitch` entries of type E: half-spectrum values (double2) or folded powers (double).
+template <bool MODE, int CQ, class E>
+__global__ __launch_bounds__(256) void k_bin_rows(const E *__restrict__ fk, const E *__restrict__ dk,
                                                   const int32_t *__restrict__ roff, const int32_t *__restrict__ rows,
-                                                  int64_t H, int64_t nr, int lrb, double m2, double kir2, double a2,
-                                                  double *__restrict__ Q) {
+                                                  int64_t H, int64_t pitch, int64_t nr, int lrb, double m2,
+                                                  double kir2, double a2, double *__restrict__ Q) {
   __shared__ double tile[BIN_LDS];
+  __shared__ int32_t list[BIN_LIST], offs[BIN_MAX_RB + 1];
   const int RB = 1 << lrb;
   const int64_t r0 = (int64_t)blockIdx.x * RB;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  // the block's offsets and row list (contiguous) first, so that a class costs one memory
+  // latency and not three; most classes are empty (no two squares sum to r)
+  for (int i = threadIdx.x; i <= RB; i += 256) offs[i] = roff[r0 + i < nr ? r0 + i : nr];
+  __syncthreads();
+  const int32_t first = offs[0], count = offs[RB] - first;
+  if (count <= BIN_LIST)
+    for (int i = threadIdx.x; i < count; i += 256) list[i] = rows[first + i];
+  __syncthreads();
+  auto row_of = [&](int32_t j) { return count <= BIN_LIST ? list[j - first] : rows[j]; };
   for (int rl = wave; rl < RB; rl += 4) {  // each wavefront its own row classes
     const int64_t r = r0 + rl;
     if (r >= nr) break;
-    const int32_t beg = roff[r], end = roff[r + 1];
+    const int32_t beg = offs[rl], end = offs[rl + 1];
+    if (beg == end) {
+#pragma unroll
+      for (int q = 0; q < CQ; ++q)
+        if (lane + 64 * q < H) tile[rl * H + lane + 64 * q] = 0.0;
+      continue;
+    }
     // lane holds columns c = lane + 64 q
     double acc[CQ];
     double denom[CQ];
@@ -92,20 +122,24 @@ __global__ __launch_bounds__(256) void k_bin_rows(const double2 *__restrict__ fk
       // fdm3d.cpp:64: m*m + (2*pi/L)*(2*pi/L)*s/(a_t*a_t)
       denom[q] = MODE ? m2 + (kir2 * (double)(r + c * c)) / a2 : 1.0;
     }
-    auto add = [&](int q, double2 u, double2 w) {
+    auto power = [](const E &u) {
+      if constexpr (sizeof(E) == sizeof(double2)) return u.x * u.x + u.y * u.y;
+      else return u;
+    };
+    auto add = [&](int q, E u, E w) {
       const int64_t c = lane + 64 * q;
-      double p = u.x * u.x + u.y * u.y;
-      if constexpr (MODE) p = p + (w.x * w.x + w.y * w.y) / denom[q];
+      double p = power(u);
+      if constexpr (MODE) p = p + power(w) / denom[q];
       acc[q] += (c == 0 || c == H - 1) ? p : 2.0 * p;
     };
-    const double2 zero = make_double2(0.0, 0.0);
+    const E zero{};
     constexpr int BIN_G = bin_group(MODE, CQ);
     int32_t j = beg;
     for (; j + BIN_G <= end; j += BIN_G) {
       int64_t base[BIN_G];
 #pragma unroll
-      for (int g = 0; g < BIN_G; ++g) base[g] = (int64_t)rows[j + g] * H;
-      double2 u[BIN_G][CQ], w[BIN_G][CQ];
+      for (int g = 0; g < BIN_G; ++g) base[g] = (int64_t)row_of(j + g) * pitch;
+      E u[BIN_G][CQ], w[BIN_G][CQ];
 #pragma unroll
       for (int g = 0; g < BIN_G; ++g)
 #pragma unroll
@@ -122,7 +156,7 @@ __global__ __launch_bounds__(256) void k_bin_rows(const double2 *__restrict__ fk
           if (lane + 64 * q < H) add(q, u[g][q], w[g][q]);
     }
     for (; j < end; ++j) {
-      const int64_t base = (int64_t)rows[j] * H;
+      const int64_t base = (int64_t)row_of(j) * pitch;
 #pragma unroll
       for (int q = 0; q < CQ; ++q) {
         const int64_t c = lane + 64 * q;
@@ -147,10 +181,18 @@ __global__ __launch_bounds__(256) void k_bin_cols(const double *__restrict__ Q, 
                                                   double *__restrict__ bins) {
   const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nb) return;
+  // sixteen entries in flight, added in order of c (one at a time the loop waits out the
+  // memory latency for each: 48 us at N=256 for 34 MB)
   double acc = 0.0;
-  for (int64_t c = 0; c < H && c * c <= s; ++c) {
-    const int64_t r = s - c * c;
-    if (r < nr) acc += Q[c * nr + r];
+  for (int64_t c0 = 0; c0 < H && c0 * c0 <= s; c0 += 16) {
+    double v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int64_t c = c0 + i, r = s - c * c;
+      v[i] = (c < H && r >= 0 && r < nr) ? Q[c * nr + r] : 0.0;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc += v[i];
   }
   bins[s] = acc;
 }
@@ -273,16 +315,23 @@ static cf_status plan_check(const cf_spectrum_plan *p) {
   return CF_OK;
 }
 
-static cf_status d2z_exec(cf_spectrum_plan *p, double *in, double *out, hipStream_t st) {
+// Transforms of sizes without own passes. hipFFT may use either's input as scratch.
+static cf_status d2z_lib(cf_spectrum_plan *p, double *in, double *out, hipStream_t st) {
   CF_FFT(hipfftSetStream(p->d2z, st));
   CF_FFT(hipfftExecD2Z(p->d2z, (hipfftDoubleReal *)in, (hipfftDoubleComplex *)out));
   return CF_OK;
 }
 
-static cf_status z2d_exec(cf_spectrum_plan *p, double *in, double *out, hipStream_t st) {
+static cf_status z2d_lib(cf_spectrum_plan *p, double *in, double *out, hipStream_t st) {
   CF_FFT(hipfftSetStream(p->z2d, st));
   CF_FFT(hipfftExecZ2D(p->z2d, (hipfftDoubleComplex *)in, (hipfftDoubleReal *)out));
   return CF_OK;
+}
+
+// out = inverse transform of `in` (rows of N/2 + 1, or cbuf0 itself), which may be destroyed.
+static cf_status z2d_exec(cf_spectrum_plan *p, double *in, double *out, hipStream_t st) {
+  if (p->fft.N) return fft_inverse(p->fft, (const double2 *)in, (double2 *)p->cbuf0, FftScale{}, out, st);
+  return z2d_lib(p, in, out, st);
 }
 
 // Spectrum factories over s, |k| = sqrt(s)*2*pi/L (random_field.cpp:67,212-254).
@@ -342,7 +391,8 @@ cf_status cf_spectrum_plan_destroy(cf_spectrum_plan *p) {
   if (!p) return CF_OK;
   if (p->have_d2z) hipfftDestroy(p->d2z);
   if (p->have_z2d) hipfftDestroy(p->z2d);
-  void *bufs[] = {p->work, p->rbuf, p->cbuf0, p->cbuf1, p->roff, p->rows, p->red, p->bins};
+  p->fft.release();
+  void *bufs[] = {p->work, p->rbuf, p->cbuf0, p->cbuf1, p->roff, p->rows, p->foff, p->frows, p->red, p->bins};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   delete p;
@@ -363,27 +413,37 @@ cf_status cf_spectrum_plan_create(int64_t N, cf_spectrum_plan **out) {
     cf_spectrum_plan_destroy(p);
     return s;
   };
-  // hipFFT plans sharing one work area (cuda_wrapper.cu:202-222)
   size_t ws1 = 0, ws2 = 0;
-  if (hipfftCreate(&p->d2z) != HIPFFT_SUCCESS) { set_error("hipfftCreate failed"); return fail(CF_E_FFT); }
-  p->have_d2z = true;
-  if (hipfftCreate(&p->z2d) != HIPFFT_SUCCESS) { set_error("hipfftCreate failed"); return fail(CF_E_FFT); }
-  p->have_z2d = true;
-  hipfftSetAutoAllocation(p->d2z, 0);
-  hipfftSetAutoAllocation(p->z2d, 0);
-  if (hipfftMakePlan3d(p->d2z, (int)N, (int)N, (int)N, HIPFFT_D2Z, &ws1) != HIPFFT_SUCCESS ||
-      hipfftMakePlan3d(p->z2d, (int)N, (int)N, (int)N, HIPFFT_Z2D, &ws2) != HIPFFT_SUCCESS) {
-    set_error("hipfftMakePlan3d(N=%lld) failed", (long long)N);
-    return fail(CF_E_FFT);
+  const bool own = FftPlan::supports(N);
+  p->pitch = own ? fft_pitch(N) : p->H;
+  if (own) {
+    const cf_status rc = p->fft.init(N);
+    if (rc != CF_OK) return fail(rc);
+  } else {
+    // hipFFT plans sharing one work area (cuda_wrapper.cu:202-222)
+    if (hipfftCreate(&p->d2z) != HIPFFT_SUCCESS) { set_error("hipfftCreate failed"); return fail(CF_E_FFT); }
+    p->have_d2z = true;
+    if (hipfftCreate(&p->z2d) != HIPFFT_SUCCESS) { set_error("hipfftCreate failed"); return fail(CF_E_FFT); }
+    p->have_z2d = true;
+    hipfftSetAutoAllocation(p->d2z, 0);
+    hipfftSetAutoAllocation(p->z2d, 0);
+    if (hipfftMakePlan3d(p->d2z, (int)N, (int)N, (int)N, HIPFFT_D2Z, &ws1) != HIPFFT_SUCCESS ||
+        hipfftMakePlan3d(p->z2d, (int)N, (int)N, (int)N, HIPFFT_Z2D, &ws2) != HIPFFT_SUCCESS) {
+      set_error("hipfftMakePlan3d(N=%lld) failed", (long long)N);
+      return fail(CF_E_FFT);
+    }
   }
   const size_t ws = ws1 > ws2 ? ws1 : ws2;
   const size_t n3 = (size_t)N * N * N;
+  const size_t cbytes = 2 * (size_t)N * N * p->pitch * sizeof(double);
   if ((ws && hipMalloc(&p->work, ws) != hipSuccess) ||
       hipMalloc((void **)&p->rbuf, n3 * sizeof(double)) != hipSuccess ||
-      hipMalloc((void **)&p->cbuf0, 2 * (size_t)p->nhalf * sizeof(double)) != hipSuccess ||
-      hipMalloc((void **)&p->cbuf1, 2 * (size_t)p->nhalf * sizeof(double)) != hipSuccess ||
+      hipMalloc((void **)&p->cbuf0, cbytes) != hipSuccess ||
+      hipMalloc((void **)&p->cbuf1, cbytes) != hipSuccess ||
       hipMalloc((void **)&p->roff, ((size_t)p->nr + 1) * sizeof(int32_t)) != hipSuccess ||
       hipMalloc((void **)&p->rows, (size_t)(N * N) * sizeof(int32_t)) != hipSuccess ||
+      hipMalloc((void **)&p->foff, ((size_t)p->nr + 1) * sizeof(int32_t)) != hipSuccess ||
+      hipMalloc((void **)&p->frows, (size_t)((N / 2 + 1) * N) * sizeof(int32_t)) != hipSuccess ||
       hipMalloc((void **)&p->red, (RED_BLOCKS + 1) * sizeof(double)) != hipSuccess ||
       hipMalloc((void **)&p->bins, (size_t)p->nb * sizeof(double)) != hipSuccess) {
     set_error("cf_spectrum_plan_create(N=%lld): device allocation failed", (long long)N);
@@ -396,24 +456,26 @@ cf_status cf_spectrum_plan_create(int64_t N, cf_spectrum_plan **out) {
       return fail(CF_E_FFT);
     }
   }
-  // Row table: stable counting sort of the N^2 rows (a, b) by r = as^2 + bs^2 (the
-  // binning's step A; its output Q, H * nr <= N^3 doubles, lives in rbuf).
-  {
+  // Row tables: stable counting sort of the rows (a, b) by r = as^2 + bs^2, of all N^2 rows
+  // and of those with a <= N/2 (folded powers). The binning's step A output Q, H * nr <=
+  // N^3 doubles, lives in rbuf.
+  auto row_table = [&](int64_t na, int32_t *off_dev, int32_t *rows_dev) {
     const int64_t nr = p->nr;
     std::vector<int32_t> off((size_t)nr + 1, 0);
     auto fold = [&](int64_t v) { return (v <= N / 2) ? v : N - v; };
-    for (int64_t a = 0; a < N; ++a)
+    for (int64_t a = 0; a < na; ++a)
       for (int64_t b = 0; b < N; ++b) off[fold(a) * fold(a) + fold(b) * fold(b) + 1]++;
     for (int64_t q = 0; q < nr; ++q) off[q + 1] += off[q];
     std::vector<int32_t> pos(off.begin(), off.end() - 1);
-    std::vector<int32_t> rws((size_t)(N * N));
-    for (int64_t a = 0; a < N; ++a)
+    std::vector<int32_t> rws((size_t)(na * N));
+    for (int64_t a = 0; a < na; ++a)
       for (int64_t b = 0; b < N; ++b) rws[pos[fold(a) * fold(a) + fold(b) * fold(b)]++] = (int32_t)(a * N + b);
-    if (hipMemcpy(p->roff, off.data(), off.size() * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(p->rows, rws.data(), rws.size() * sizeof(int32_t), hipMemcpyHostToDevice) != hipSuccess) {
-      set_error("cf_spectrum_plan_create: bin table upload failed");
-      return fail(CF_E_HIP);
-    }
+    return hipMemcpy(off_dev, off.data(), off.size() * sizeof(int32_t), hipMemcpyHostToDevice) == hipSuccess &&
+           hipMemcpy(rows_dev, rws.data(), rws.size() * sizeof(int32_t), hipMemcpyHostToDevice) == hipSuccess;
+  };
+  if (!row_table(N, p->roff, p->rows) || (own && !row_table(N / 2 + 1, p->foff, p->frows))) {
+    set_error("cf_spectrum_plan_create: bin table upload failed");
+    return fail(CF_E_HIP);
   }
   *out = p;
   return CF_OK;
@@ -422,9 +484,10 @@ cf_status cf_spectrum_plan_create(int64_t N, cf_spectrum_plan **out) {
 cf_status cf_fft_d2z(cf_spectrum_plan *p, const double *in, double *out, cf_stream stream) {
   CF_TRY(plan_check(p));
   CF_REQUIRE(in && out, "cf_fft_d2z: null buffer");
+  if (p->fft.N) return fft_forward(p->fft, in, (double2 *)p->cbuf0, (double2 *)out, S(stream));
   const size_t n3 = (size_t)p->N * p->N * p->N;
   CF_HIP(hipMemcpyAsync(p->rbuf, in, n3 * sizeof(double), hipMemcpyDeviceToDevice, S(stream)));
-  return d2z_exec(p, p->rbuf, out, S(stream));
+  return d2z_lib(p, p->rbuf, out, S(stream));
 }
 
 cf_status cf_fft_z2d(cf_spectrum_plan *p, double *in, double *out, cf_stream stream) {
@@ -446,16 +509,21 @@ cf_status cf_fft_z2d_inplace(cf_spectrum_plan *p, double *inout, cf_stream strea
 }
 
 // Step A into the plan's real scratch (free once the transform has run), step B into bins.
-static cf_status bin_launch(cf_spectrum_plan *p, const double *fk, const double *dk, double m2, double kir2,
-                            double a2, double *bins, hipStream_t st) {
+// fk, dk: half spectra (fold false, rows of H) or folded powers (rows of the plan's pitch).
+static cf_status bin_launch(cf_spectrum_plan *p, const double *fk, const double *dk, bool fold, double m2,
+                            double kir2, double a2, double *bins, hipStream_t st) {
   CF_REQUIRE(p->H <= 64 * BIN_CQ, "binning: N=%lld exceeds the row chunking", (long long)p->N);
   int lrb = 0;  // RB = 2^lrb row classes per block: the largest power of two with RB * H <= BIN_LDS
   while ((2 << lrb) * p->H <= BIN_LDS && lrb < 8) ++lrb;
   const dim3 gA((unsigned)cdiv(p->nr, (int64_t)1 << lrb)), b256(256);
   auto rows_kernel = [&](auto mode, auto cq) {
-    hipLaunchKernelGGL((k_bin_rows<decltype(mode)::value, decltype(cq)::value>), gA, b256, 0, st,
-                       (const double2 *)fk, (const double2 *)dk, p->roff, p->rows, p->H, p->nr, lrb, m2, kir2, a2,
-                       p->rbuf);
+    if (fold)
+      hipLaunchKernelGGL((k_bin_rows<decltype(mode)::value, decltype(cq)::value, double>), gA, b256, 0, st, fk, dk,
+                         p->foff, p->frows, p->H, p->pitch, p->nr, lrb, m2, kir2, a2, p->rbuf);
+    else
+      hipLaunchKernelGGL((k_bin_rows<decltype(mode)::value, decltype(cq)::value, double2>), gA, b256, 0, st,
+                         (const double2 *)fk, (const double2 *)dk, p->roff, p->rows, p->H, p->H, p->nr, lrb, m2, kir2,
+                         a2, p->rbuf);
   };
   auto by_cq = [&](auto mode) {
     const int64_t cq = cdiv(p->H, 64);  // H <= 64 * BIN_CQ (checked above)
@@ -477,20 +545,33 @@ static cf_status bin_launch(cf_spectrum_plan *p, const double *fk, const double 
 cf_status cf_bin_power(cf_spectrum_plan *p, const double *fk, double *bins, cf_stream stream) {
   CF_TRY(plan_check(p));
   CF_REQUIRE(fk && bins, "cf_bin_power: null buffer");
-  return bin_launch(p, fk, nullptr, 0.0, 0.0, 1.0, bins, S(stream));
+  return bin_launch(p, fk, nullptr, false, 0.0, 0.0, 1.0, bins, S(stream));
+}
+
+// m^2 + (2 pi / L)^2 s / a^2 of the mode power (fdm3d.cpp:64).
+static double mode_kir2(double L) {
+  const double pi = 3.14159265358979323846;
+  return (2 * pi / L) * (2 * pi / L);
 }
 
 cf_status cf_bin_mode_power(cf_spectrum_plan *p, const double *phik, const double *dphik, double L,
                             double m, double a_t, double *bins, cf_stream stream) {
   CF_TRY(plan_check(p));
   CF_REQUIRE(phik && dphik && bins, "cf_bin_mode_power: null buffer");
-  const double pi = 3.14159265358979323846;
-  const double kir2 = (2 * pi / L) * (2 * pi / L);
-  return bin_launch(p, phik, dphik, m * m, kir2, a_t * a_t, bins, S(stream));
+  return bin_launch(p, phik, dphik, false, m * m, mode_kir2(L), a_t * a_t, bins, S(stream));
 }
+
+// Folded powers of a field into slot 0 or 1 of cbuf1 (two fields' worth fit: 2 (N/2 + 1) N
+// pitch <= 2 N^2 pitch doubles). cbuf0 holds the spectrum on the way.
+static double *fold_slot(cf_spectrum_plan *p, int slot) { return p->cbuf1 + slot * (p->N / 2 + 1) * p->N * p->pitch; }
 
 cf_status cf_power_spectrum(cf_spectrum_plan *p, const double *f, double *bins, cf_stream stream) {
   CF_TRY(plan_check(p));
+  if (p->fft.N) {
+    CF_REQUIRE(f && bins, "cf_power_spectrum: null buffer");
+    CF_TRY(fft_forward_fold(p->fft, f, (double2 *)p->cbuf0, fold_slot(p, 0), S(stream)));
+    return bin_launch(p, fold_slot(p, 0), nullptr, true, 0.0, 0.0, 1.0, bins, S(stream));
+  }
   CF_TRY(cf_fft_d2z(p, f, p->cbuf0, stream));
   return cf_bin_power(p, p->cbuf0, bins, stream);
 }
@@ -498,7 +579,8 @@ cf_status cf_power_spectrum(cf_spectrum_plan *p, const double *f, double *bins, 
 cf_status cf_power_spectrum_consume(cf_spectrum_plan *p, double *f, double *bins, cf_stream stream) {
   CF_TRY(plan_check(p));
   CF_REQUIRE(f && bins, "cf_power_spectrum_consume: null buffer");
-  CF_TRY(d2z_exec(p, f, p->cbuf0, S(stream)));
+  if (p->fft.N) return cf_power_spectrum(p, f, bins, stream);
+  CF_TRY(d2z_lib(p, f, p->cbuf0, S(stream)));
   return cf_bin_power(p, p->cbuf0, bins, stream);
 }
 
@@ -507,6 +589,11 @@ cf_status cf_mode_power_spectrum(cf_spectrum_plan *p, const double *state, doubl
   CF_TRY(plan_check(p));
   CF_REQUIRE(state && bins, "cf_mode_power_spectrum: null buffer");
   const int64_t N3 = p->N * p->N * p->N;
+  if (p->fft.N) {
+    for (int q = 0; q < 2; ++q)
+      CF_TRY(fft_forward_fold(p->fft, state + q * N3, (double2 *)p->cbuf0, fold_slot(p, q), S(stream)));
+    return bin_launch(p, fold_slot(p, 0), fold_slot(p, 1), true, m * m, mode_kir2(L), a_t * a_t, bins, S(stream));
+  }
   CF_TRY(cf_fft_d2z(p, state, p->cbuf0, stream));
   CF_TRY(cf_fft_d2z(p, state + N3, p->cbuf1, stream));
   return cf_bin_mode_power(p, p->cbuf0, p->cbuf1, L, m, a_t, bins, stream);
@@ -549,11 +636,16 @@ cf_status cf_grf(cf_spectrum_plan *p, double *w, const double *sqrtP, const doub
     hipLaunchKernelGGL(k_mul_exp, dim3(grid_cap(N3, 256)), dim3(256), 0, st, w, Psi, N3);
     CF_LAUNCHED();
   }
-  CF_TRY(d2z_exec(p, w, p->cbuf0, st));
+  if (p->fft.N) {
+    double2 *spec = (double2 *)p->cbuf0;
+    CF_TRY(fft_forward(p->fft, w, spec, spec, st));
+    return fft_inverse(p->fft, spec, spec, FftScale{sqrtP, 1.0, 0.0}, out, st);
+  }
+  CF_TRY(d2z_lib(p, w, p->cbuf0, st));
   hipLaunchKernelGGL(k_grf_scale, dim3(grid_cap(p->nhalf, 256)), dim3(256), 0, st, (double2 *)p->cbuf0,
                      sqrtP, p->N, p->H);
   CF_LAUNCHED();
-  return z2d_exec(p, p->cbuf0, out, st);
+  return z2d_lib(p, p->cbuf0, out, st);
 }
 
 cf_status cf_scaled_fourier_modes(cf_spectrum_plan *p, const double *f, const double *kernel_by_s, double *out,
@@ -562,12 +654,17 @@ cf_status cf_scaled_fourier_modes(cf_spectrum_plan *p, const double *f, const do
   CF_REQUIRE(f && kernel_by_s && out, "cf_scaled_fourier_modes: null buffer");
   hipStream_t st = S(stream);
   const size_t n3 = (size_t)p->N * p->N * p->N;
+  if (p->fft.N) {
+    double2 *spec = (double2 *)p->cbuf0;
+    CF_TRY(fft_forward(p->fft, f, spec, spec, st));
+    return fft_inverse(p->fft, spec, spec, FftScale{kernel_by_s, 1.0, (double)n3}, out, st);
+  }
   CF_HIP(hipMemcpyAsync(p->rbuf, f, n3 * sizeof(double), hipMemcpyDeviceToDevice, st));
-  CF_TRY(d2z_exec(p, p->rbuf, p->cbuf0, st));
+  CF_TRY(d2z_lib(p, p->rbuf, p->cbuf0, st));
   hipLaunchKernelGGL(k_scale_modes, dim3(grid_cap(p->nhalf, 256)), dim3(256), 0, st, (double2 *)p->cbuf0,
                      kernel_by_s, p->N, p->H);
   CF_LAUNCHED();
-  return z2d_exec(p, p->cbuf0, out, st);
+  return z2d_lib(p, p->cbuf0, out, st);
 }
 
 }  // extern "C"

@@ -33,6 +33,7 @@
 
 #include <cmath>
 
+#include "cf_fft.hpp"
 #include "cf_march.hpp"
 #include "cf_tb_run.hpp"
 
@@ -232,18 +233,50 @@ __global__ void k_comoving_transfer(int64_t G, const double *__restrict__ R, dou
   }
 }
 
+// The same transfer as a table: the factors of Psi^ and dPsi^/dt for every pair a' >= b' of
+// folded indices (block x: the pair's row) and every c.
+__global__ void k_comoving_table(int64_t pitch, double g3, double2 *__restrict__ tab, double factor, double H) {
+  const int row = blockIdx.x;
+  int a = (int)((sqrtf(8.0f * (float)row + 1.0f) - 1.0f) * 0.5f);
+  while (a * (a + 1) / 2 > row) --a;
+  while ((a + 1) * (a + 2) / 2 <= row) ++a;
+  const int b = row - a * (a + 1) / 2;
+  for (int c = threadIdx.x; c < pitch; c += blockDim.x) {
+    const int s = a * a + b * b + c * c;
+    double2 v = make_double2(0.0, 0.0);
+    if (s != 0) {
+      const double w = sqrt((double)s) * factor;
+      double sv, cv;
+      sincos(w, &sv, &cv);
+      const double cf = 2.0 / ((w * w) * w) / g3;
+      v = make_double2((sv - w * cv) * cf, (H * ((3.0 * w) * cv + ((w * w) - 3.0) * sv)) * cf);
+    }
+    tab[row * pitch + c] = v;
+  }
+}
+
 // Half spectrum of N^3 -> half spectrum of M^3 (compute_cutoff_fouriers,
 // fdm3d.cpp:105-130): low |k| modes kept, divided by (N/M)^3.
-__global__ void k_cutoff(int64_t N, int64_t M, const double *__restrict__ in, double *__restrict__ out,
-                         double scale3) {
-  const int64_t HM = M / 2 + 1, HN = N / 2 + 1, n = M * M * HM;
+__global__ void k_cutoff(int64_t N, int64_t M, const double *__restrict__ in, int64_t pitch_in,
+                         double *__restrict__ out, int64_t pitch_out, double scale3) {
+  const int64_t HM = M / 2 + 1, n = M * M * HM;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
     const int64_t c = e % HM, b = (e / HM) % M, a = e / (HM * M);
     const int64_t aN = (a < M / 2) ? a : N - (M - a), bN = (b < M / 2) ? b : N - (M - b);
-    const int64_t f = (aN * N + bN) * HN + c;
-    out[2 * e] = in[2 * f] / scale3;
-    out[2 * e + 1] = in[2 * f + 1] / scale3;
+    const int64_t f = (aN * N + bN) * pitch_in + c, o = (a * M + b) * pitch_out + c;
+    out[2 * o] = in[2 * f] / scale3;
+    out[2 * o + 1] = in[2 * f + 1] / scale3;
   }
+}
+
+static unsigned grid_for(int64_t n);
+static cf_status launch_cutoff(int64_t N, int64_t M, const double *in, int64_t pitch_in, double *out,
+                               int64_t pitch_out, hipStream_t st) {
+  const double sd = static_cast<double>(N) / static_cast<double>(M);
+  hipLaunchKernelGGL(k_cutoff, dim3(grid_for(M * M * (M / 2 + 1))), dim3(256), 0, st, N, M, in, pitch_in, out,
+                     pitch_out, pow(sd, 3));
+  CF_LAUNCHED();
+  return CF_OK;
 }
 
 static unsigned grid_for(int64_t n) {
@@ -252,10 +285,16 @@ static unsigned grid_for(int64_t n) {
 }
 
 // Psi and dPsi/dt on one grid, rebuilt from the stored spectrum R at a stage
-// time, with a two-slot cache keyed by that time.
+// time, with a three-slot cache keyed by that time. Grids without a prime factor above 7
+// take the own transform passes: the first one multiplies R by both fields' transfer
+// factors (a table) as it reads it, so the two spectra are never formed before it.
+// At N=384 the transfer kernel and hipFFT's three passes took 2040 us for the pair.
 struct PsiGrid {
   int64_t G = 0;
-  double *R = nullptr;     // 2*G*G*(G/2+1): comoving curvature, half spectrum
+  FftPlan fft;             // fft.N != 0: own passes
+  int64_t pitch = 0;       // entries per row of R and spec
+  double2 *tab = nullptr;  // transfer factors (own passes)
+  double *R = nullptr;     // comoving curvature, half spectrum (rows of `pitch`)
   double *spec = nullptr;  // 2 half spectra: Psi^, dPsi^
   // Psi | dPsi (2*G^3 each) at up to three times, least recently used replaced: a
   // temporally blocked step needs t, t + dt/2 and t + dt at once, and the next step
@@ -275,9 +314,14 @@ struct PsiGrid {
   cf_status init(int64_t g) {
     G = g;
     CF_REQUIRE(G <= 1024, "comoving curvature variants support grids up to 1024^3 (got %lld)", (long long)G);
-    CF_HIP(hipMalloc(&R, half() * sizeof(double)));
-    CF_HIP(hipMalloc(&spec, 2 * half() * sizeof(double)));
+    pitch = FftPlan::supports(G) ? fft_pitch(G) : G / 2 + 1;
+    CF_HIP(hipMalloc(&R, 2 * (size_t)G * G * pitch * sizeof(double)));
+    CF_HIP(hipMalloc(&spec, 4 * (size_t)G * G * pitch * sizeof(double)));
     for (int s = 0; s < NS; ++s) CF_HIP(hipMalloc(&slot[s], 2 * cube() * sizeof(double)));
+    if (FftPlan::supports(G)) {
+      CF_HIP(hipMalloc(&tab, (size_t)fft_pair_rows(G) * pitch * sizeof(double2)));
+      return fft.init(G);
+    }
     int n[3] = {(int)G, (int)G, (int)G};
     hipfftResult r = hipfftPlanMany(&plan, 3, n, nullptr, 1, (int)(G * G * (G / 2 + 1)), nullptr, 1, (int)cube(),
                                     HIPFFT_Z2D, 2);
@@ -288,9 +332,19 @@ struct PsiGrid {
     have_plan = true;
     return CF_OK;
   }
+  // R from a half spectrum without padding.
+  cf_status set_R(const double *field, hipStream_t st) {
+    const size_t row = (size_t)(G / 2 + 1) * sizeof(double2);
+    CF_HIP(hipMemcpy2DAsync(R, (size_t)pitch * sizeof(double2), field, row, row, (size_t)(G * G),
+                            hipMemcpyDeviceToDevice, st));
+    return CF_OK;
+  }
   void release() {
     if (have_plan) hipfftDestroy(plan);
     have_plan = false;
+    fft.release();
+    (void)hipFree(tab);
+    tab = nullptr;
     (void)hipFree(R);
     (void)hipFree(spec);
     for (int s = 0; s < NS; ++s) {
@@ -312,6 +366,17 @@ struct PsiGrid {
     for (int q = 1; q < NS; ++q)
       if (used[q] < used[s]) s = q;
     valid[s] = false;
+    if (fft.N) {
+      hipLaunchKernelGGL(k_comoving_table, dim3((unsigned)fft_pair_rows(G)), dim3(64), 0, st, pitch,
+                         (double)(G * G * G), tab, factor, H);
+      CF_LAUNCHED();
+      CF_TRY(fft_inverse_pair(fft, (const double2 *)R, tab, (double2 *)spec, pitch, slot[s], st));
+      slot_t[s] = t;
+      valid[s] = true;
+      used[s] = ++clock;
+      *out = slot[s];
+      return CF_OK;
+    }
     hipLaunchKernelGGL(k_comoving_transfer, dim3(grid_for((int64_t)(half() / 2))), dim3(256), 0, st, G, R, spec,
                        spec + half(), factor, H);
     CF_LAUNCHED();
@@ -417,11 +482,7 @@ cf_status cf_cutoff_fouriers(int64_t N, int64_t M, const double *in, double *out
   CF_REQUIRE(valid_N(N) && valid_N(M) && M <= N, "cf_cutoff_fouriers: need even 4 <= M <= N <= 2048 (N=%lld M=%lld)",
              (long long)N, (long long)M);
   CF_REQUIRE(in && out && (const void *)in != (const void *)out, "cf_cutoff_fouriers: null or aliased buffers");
-  const double sd = static_cast<double>(N) / static_cast<double>(M);
-  const int64_t n = M * M * (M / 2 + 1);
-  hipLaunchKernelGGL(k_cutoff, dim3(grid_for(n)), dim3(256), 0, S(stream), N, M, in, out, pow(sd, 3));
-  CF_LAUNCHED();
-  return CF_OK;
+  return launch_cutoff(N, M, in, N / 2 + 1, out, M / 2 + 1, S(stream));
 }
 
 cf_status cf_comoving_psi_fft(int64_t G, const double *R_fft, double *psi_fft, double *dpsi_fft, double factor,
@@ -456,7 +517,7 @@ cf_status cf_variant_create(const cf_kg_params *p, int kind, double f_a, int64_t
   v->M = (kind == V_APPROX) ? M : 0;
   hipStream_t st = S(stream);
   cf_status rc = CF_OK;
-  const size_t N3 = (size_t)N * N * N, halfN = 2 * (size_t)N * N * (N / 2 + 1);
+  const size_t N3 = (size_t)N * N * N;
   if (kind == V_FIXED) {
     if (hipMalloc(&v->psi_fixed, N3 * sizeof(double)) != hipSuccess ||
         hipMemcpyAsync(v->psi_fixed, field, N3 * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess) {
@@ -465,18 +526,12 @@ cf_status cf_variant_create(const cf_kg_params *p, int kind, double f_a, int64_t
     }
   } else if (kind == V_COMOVING) {
     rc = v->grid.init(N);
-    if (rc == CF_OK && hipMemcpyAsync(v->grid.R, field, halfN * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess) {
-      set_error("cf_variant_create: copy of the R spectrum failed");
-      rc = CF_E_HIP;
-    }
+    if (rc == CF_OK) rc = v->grid.set_R(field, st);
   } else if (kind == V_APPROX) {
     rc = v->grid.init(M);
     if (rc == CF_OK) rc = v->full.init(N);
-    if (rc == CF_OK && hipMemcpyAsync(v->full.R, field, halfN * sizeof(double), hipMemcpyDeviceToDevice, st) != hipSuccess) {
-      set_error("cf_variant_create: copy of the R spectrum failed");
-      rc = CF_E_HIP;
-    }
-    if (rc == CF_OK) rc = cf_cutoff_fouriers(N, M, v->full.R, v->grid.R, stream);
+    if (rc == CF_OK) rc = v->full.set_R(field, st);
+    if (rc == CF_OK) rc = launch_cutoff(N, M, v->full.R, v->full.pitch, v->grid.R, v->grid.pitch, st);
     v->full_ready = (rc == CF_OK);
   }
   if (rc == CF_OK && hipStreamSynchronize(st) != hipSuccess) {

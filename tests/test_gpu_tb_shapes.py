@@ -66,3 +66,27 @@ def test_ensemble_28x36_keeps_bits(cfl, prec, grid):
             x = cfl.join_f64(hi, lo)
         torch.cuda.synchronize()
         assert torch.equal(ens.state(r), x), f"realisation {r}"
+
+
+@pytest.mark.parametrize("N", [18, 98])
+def test_odd_alignment(cfl, N):
+    """States that start on an odd double / float (the step moves two columns a lane)."""
+    print(f"case tb odd alignment N={N}", flush=True)
+    n = 2 * N ** 3
+    p = cfl.kg_params(N, float(N), 1.0, 0.1, cfl.radiation(**FRW))
+    x = dev(rand_state(N, 33, amp=0.5))
+    a = torch.empty(n + 1, dtype=torch.float64, device="cuda")
+    b = torch.empty_like(a)
+    a[1:] = x
+    ref = torch.empty_like(x)
+    cfl.rk4_step_tb_f64(p, x, ref, 1.0, 0.05)
+    cfl.rk4_step_tb_f64(p, a[1:], b[1:], 1.0, 0.05)
+    assert torch.equal(b[1:], ref)
+    hi, lo = cfl.split_f64(x)
+    h2, l2 = torch.empty_like(hi), torch.empty_like(lo)
+    bufs = [torch.empty(n + 1, dtype=torch.float32, device="cuda") for _ in range(4)]
+    bufs[0][1:], bufs[1][1:] = hi, lo
+    for step in (cfl.rk4_step_tb_f32s, cfl.rk4_step_tb_f32c):
+        step(p, hi, lo, h2, l2, 1.0, 0.05)
+        step(p, *[t[1:] for t in bufs], 1.0, 0.05)
+        assert torch.equal(bufs[2][1:], h2) and torch.equal(bufs[3][1:], l2)
