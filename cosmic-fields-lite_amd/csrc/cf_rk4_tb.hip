@@ -59,8 +59,7 @@ __device__ __forceinline__ TbUnit tb_unit_of(const TbGeom &g, int bid) {
 // to a common schedule of plane iterations (cf_tb_body.hpp).
 template <int MODE, bool LAM, class SH, int WAVES, bool PACE>
 __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void k_rk4_tb(
-    TbGeom g, TbStep k, TbStepF kf, const void *__restrict__ xin, const float *__restrict__ lin,
-    void *__restrict__ xout, float *__restrict__ lout) {
+    TbGeom g, TbStep k, TbStepF kf, const void *xin, const float *lin, void *xout, float *lout) {
   __shared__ __attribute__((aligned(16))) TbElem<MODE, SH> smem[SH::LDS];
   // Blocks go to the 8 XCDs round robin; consecutive logical tiles are mapped
   // to one XCD so that neighbouring tiles' halos meet in its L2.
@@ -81,12 +80,12 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(4, 4))) 
 // Region shapes of the single-lattice kernels, smallest first. A large region repeats
 // less of its neighbours' work and reads (26 x 64 tiles: 1.23 region sites per output
 // site, 8 x 16 ones 1.88); a small one gives a small lattice enough blocks and takes
-// less time per plane. `wave`: VGPR budget as wavefronts per SIMD.
+// less time per plane.
 //
 // t1 and tau are the time of a plane iteration in us with one block on a CU and, per
-// block, with the CU full; bw the rate in bytes per us at which launches that stream
-// through HBM pass their loads (halo and warm-up included) and stores. Measured over
-// N = 32 .. 512 on 256 CUs; see tb_cost.
+// block, with `resident` blocks, the CU full; bw the rate in bytes per us at which
+// launches that stream through HBM pass their loads (halo and warm-up included) and
+// stores. Measured over N = 32 .. 512 on 256 CUs; see tb_cost.
 struct TbShapeInfo {
   int rb, rc, resident;
   double t1, tau, bw;
@@ -100,17 +99,15 @@ typedef TbShape<14, 36, 1, 512> TbC14x36;     // a column per thread (TB_F32C, v
 typedef TbShape<28, 36, 1, 1024> TbC28x36;
 typedef TbShape<22, 68, 2, 768> TbC22x68;     // 768 threads: 168 VGPRs for float histories and double sums
 
-static const std::vector<TbShapeInfo> &tb_shapes(int family);
-
 enum : int { TB_FAM_F64 = 0, TB_FAM_F32C = 1, TB_FAM_F32S = 2, TB_FAM_VAR = 3 };
 
 static const std::vector<TbShapeInfo> &tb_shapes(int family) {
   static const std::vector<TbShapeInfo> t[4] = {
-      {{12, 20, 8, 0.56, 0.20, 4.9e6}, {14, 36, 4, 0.64, 0.46, 5.0e6}, {28, 36, 2, 0.96, 0.93, 5.3e6},
-       {30, 68, 1, 1.75, 1.75, 5.55e6}},
-      {{14, 36, 2, 0.75, 0.60, 4.6e6}, {28, 36, 1, 1.24, 1.24, 4.7e6}, {22, 68, 1, 1.73, 1.73, 5.1e6}},
-      {{12, 20, 8, 0.54, 0.16, 4.0e6}, {14, 36, 4, 0.56, 0.39, 4.6e6}, {28, 36, 2, 0.85, 0.81, 4.6e6},
-       {30, 68, 1, 1.55, 1.55, 4.9e6}, {15, 132, 1, 1.55, 1.55, 5.2e6}},
+      {{12, 20, 8, 0.68, 0.26, 4.9e6}, {14, 36, 4, 0.70, 0.47, 5.0e6}, {28, 36, 2, 1.00, 0.92, 5.1e6},
+       {30, 68, 1, 2.00, 2.00, 5.55e6}},
+      {{14, 36, 2, 0.75, 0.58, 4.6e6}, {28, 36, 1, 1.22, 1.22, 4.4e6}, {22, 68, 1, 1.73, 1.73, 5.0e6}},
+      {{12, 20, 8, 0.60, 0.18, 3.9e6}, {14, 36, 4, 0.65, 0.39, 4.6e6}, {28, 36, 2, 0.84, 0.78, 4.65e6},
+       {30, 68, 1, 1.65, 1.65, 5.2e6}, {15, 132, 1, 1.55, 1.55, 5.8e6}},
       {{14, 36, 2, 0.9, 0.8, 4.6e6}, {28, 36, 1, 1.5, 1.5, 4.9e6}},
   };
   return t[family];
@@ -152,28 +149,32 @@ static TbGeom tb_geom(int family, int shape, int64_t N, int A, int64_t a_lo, int
 }
 
 // Modelled time of a launch in us: the larger of
-//   the busiest CU's plane iterations: its n = ceil(blocks / CUs) blocks run `resident`
-//   at a time, A + 4 iterations each, at tau per block (t1 when one runs alone), and
+//   the launch itself and the busiest CU's plane iterations: its n = ceil(blocks / CUs)
+//   blocks run `resident` at a time, A + 4 iterations each at tau per block (t1 when one
+//   runs alone), of which the two that only load and the two without k3 and k4 cost two;
 //   the bytes it passes: the loads of every region and iteration and the stores, at bw
-//   (20% more while both states fit the 256 MB cache).
+//   (60% more while both states fit the 256 MB cache). Beyond it blocks of long chunks
+//   drift apart and find less of their neighbours' planes in L2: 5% per 100 planes.
 // Few chunks leave CUs idle, many repeat warm-up planes; small regions repeat halos.
+// Within 4% of the best of 6 to 12 measured (shape, chunk) pairs at each of N = 32, 64,
+// 96, 128, 160, 200, 250, 300, 384, 512 and storage form, in half of them the best.
 static double tb_cost(const TbShapeInfo &s, const TbGeom &g, int cus) {
   const int64_t n = cdiv(g.total, cus), full = n / s.resident, rest = n % s.resident;
-  const double it = (double)(g.A + 2 * TBH);
   const double one = std::max(s.t1, (double)rest * s.tau);
-  const double cu = it * ((double)full * s.resident * s.tau + (rest ? one : 0.0));
+  const double cu = 1.8 + (double)(g.A + 2) * ((double)full * s.resident * s.tau + (rest ? one : 0.0));
   const double sites = (double)g.N * (double)g.N * (double)(g.a_hi - g.a_lo);
-  const double loads = 16.0 * (double)g.ntb * g.ntc * g.n_ac * s.rb * s.rc * it, stores = 16.0 * sites;
-  const double bw = 32.0 * sites <= 256e6 ? 1.2 * s.bw : s.bw;
-  return std::max(cu, (loads + stores) / bw);
+  const bool cached = 32.0 * sites <= 256e6;
+  const double drift = cached ? 1.0 : 1.0 + 5e-4 * (double)g.A;
+  const double loads = 16.0 * (double)g.ntb * g.ntc * g.n_ac * s.rb * s.rc * (double)(g.A + 2 * TBH) * drift;
+  return std::max(cu, (loads + 16.0 * sites) / (cached ? 1.6 * s.bw : s.bw));
 }
 
 // The cheapest (shape, chunk) of a launch, or the cheapest shape for a given chunk. With
 // `near`, also every chunk length whose best shape costs at most near_pct percent more,
 // cheapest first. Chunk lengths are the ceil(planes / k); there are about 2 sqrt(planes).
 // Measured on MI355X (us a step, FP64; before: one rule over 32 x 32 regions with a halo
-// of four): N=32 20.5 -> 5.2, 64 20.7 -> 7.8, 128 31.6 -> 19.5, 200 80 -> 57, 250 152 ->
-// 113, 300 258 -> 192, 384 467 -> 394, 512 1239 -> 895.
+// of four): N=32 20.5 -> 3.5, 64 20.7 -> 6.0, 128 31.6 -> 17.8, 200 80 -> 55, 250 152 ->
+// 110, 300 258 -> 189, 384 467 -> 392, 512 1239 -> 886.
 static TbGeom tb_plan(int family, int64_t N, int chunk, int64_t a_lo, int64_t a_hi, int64_t NA,
                       std::vector<int> *near = nullptr, int near_pct = 0) {
   const std::vector<TbShapeInfo> &shapes = tb_shapes(family);

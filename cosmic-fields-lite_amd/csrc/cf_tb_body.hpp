@@ -16,9 +16,13 @@
 //
 //   iteration j takes x at plane P = a0 - 2 + j (loaded two iterations ahead) and y1.phi
 //     A at P-1 (needs x.phi, y1.phi at P-2..P)     -> k1, k2; y2.phi, y3.phi, partial sums
-//     B at P-2 (needs y2.phi, y3.phi at P-3..P-1)  -> k3, k4; new state at P-2 (for j >= 4)
+//     B at P-2 (needs y2.phi, y3.phi at P-3..P-1)  -> k3, k4; new state at P-2
 //
-// so a chunk of A planes takes A + 4 iterations. The in-plane neighbours come from four
+// The first stored plane is that of j = 4 and needs A from j = 2 on: the loop starts there,
+// with the first two planes taken straight from their loads, and iterations 2 and 3 leave
+// B out. So a chunk of A planes takes A + 2 iterations, two of them half. (Running all
+// stages from j = 0: A + 4 full iterations; N=32 5.6 against 3.6 us, N=64 7.8 / 6.0,
+// N=128 19.4 / 17.7.) The in-plane neighbours come from four
 // plane buffers in LDS (x.phi, y1.phi of P-1; y2.phi, y3.phi of P-2), all known when the
 // iteration starts: they are written together, and with two sets of buffers one barrier
 // per plane suffices. The histories are three planes deep; the loop is unrolled by six
@@ -29,9 +33,9 @@
 //
 // Memory. Loads and stores go through buffer resources over one plane, VC values each
 // (16 bytes in FP64), with per-lane offsets that never change: lanes outside the tile
-// hold an offset past the plane's end, and the stores of the first four iterations use
-// an empty resource, so no branch surrounds a memory operation. N is even, so a pair of
-// columns never straddles the periodic wrap. The plane loads are issued two iterations
+// hold an offset past the plane's end, so no branch surrounds a memory operation (before
+// j = 4 the lo parts are read through an empty resource). N is even, so a pair of columns
+// never straddles the periodic wrap. The plane loads are issued two iterations
 // ahead; the barrier is a bare s_barrier after a wait for this wavefront's LDS operations,
 // so it waits for no load. What bounds it: at N=512 the bytes moved, 4.8 TB/s of the 32
 // it cannot do without (a plain copy reaches 4.8-5.0 on this part); below N=200 vector
@@ -304,8 +308,8 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
     off += NN;
     return off == N3 ? 0 : off;
   };
-  int64_t off_ld = wrap(u.a0 - TBH);      // next plane to load
-  int64_t off_st = wrap(u.a0 - TBH - 2);  // plane P-2
+  int64_t off_ld = wrap(u.a0 - TBH);  // next plane to load
+  int64_t off_st = off_ld;            // plane P-2 of the first iteration, j = 2
   int64_t off_lo = off_st;
   const int iters = (int)(u.a1 - u.a0) + 4;
   auto load = [&](int s) {
@@ -320,11 +324,19 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
     LP[s] = tb_load<float, VC>(tb_plane(lin + N3 + off_lo, nb), st_off);
     off_lo = next_plane(off_lo);
   };
+  // x at the planes of j = 0 and 1, then the prefetches of j = 2 and 3
+  V first[2][2];
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    load(q);
+    first[q][0] = LDF[q];
+    first[q][1] = LDP[q];
+  }
   load(0);
   load(1);
   if constexpr (MODE != TB_F64) {
-    load_lo(0, 0);
-    load_lo(1, 1);
+    load_lo(0, 2);
+    load_lo(1, 3);
   }
   // Variants: Psi (and dPsi) of A's plane at the stage times of k1 and k2 and of B's plane
   // at that of k4, loaded one iteration ahead; what k3 needs is what k2 had.
@@ -337,8 +349,8 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
   double psA[2] = {0.0, 0.0}, dpA[2] = {0.0, 0.0}, psB = 0.0, dpB = 0.0;
   TbSite site_mid = {0.0, 0.0, 0.0};   // of B's plane, from the iteration before
   if constexpr (CURV || COM) {
-    off_a = wrap(u.a0 - TBH - 1);
-    off_b = wrap(u.a0 - TBH - 2);
+    off_a = wrap(u.a0 - 1);
+    off_b = wrap(u.a0 - 2);
   } else if constexpr (APX) {
     const int sd = (int)cps.sd, hs = (int)cps.hs;
     ps_off = (uint32_t)((((b + hs) % N) / sd) * (int)cps.G + ((c + hs) % N) / sd) * 8u;
@@ -347,8 +359,8 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
       off = (int64_t)(q / sd) * cps.G * cps.G;
       rem = q % sd;
     };
-    cell(u.a0 - TBH - 1, off_a, rem_a);
-    cell(u.a0 - TBH - 2, off_b, rem_b);
+    cell(u.a0 - 1, off_a, rem_a);
+    cell(u.a0 - 2, off_b, rem_b);
   }
   auto field = [&](const double *f, int64_t off) {
     return tb_load<double, 1>(tb_plane(f + off, field_bytes), ps_off).v[0];
@@ -411,8 +423,16 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
   };
   const Av dh = MODE == TB_F32S ? (Av)kf.dh : (Av)k.dh, dt = MODE == TB_F32S ? (Av)kf.dt : (Av)k.dt;
 
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+#pragma unroll
+    for (int v = 0; v < VC; ++v) {
+      XF[q].v[v] = (H)first[q][0].v[v];
+      XP[q].v[v] = (H)first[q][1].v[v];
+      Y1F[q].v[v] = input(XF[q].v[v], dh, (Av)XP[q].v[v]);
+    }
   const uint64_t t_begin = PACE ? __builtin_amdgcn_s_memrealtime() : 0;
-  auto iteration = [&](auto phase, auto set, const int j) {
+  auto iteration = [&](auto phase, auto set, auto with_b, const int j) {
     // the value of plane P - d sits at [(phase - d) mod 3] of its history
     constexpr int p0 = decltype(phase)::value, p1 = (p0 + 2) % 3, p2 = (p0 + 1) % 3;
     constexpr int S = decltype(set)::value;  // j & 1: buffer set, prefetch slot
@@ -478,64 +498,67 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
     }
     // ---- B at P-2: k3 = f(y2), k4 = f(y3); new state (AF, AP, Y2P: from A of the
     // iteration before)
-    HV y3p;
-    force(Y2F[p2], Y2F[p1], Y2F[p0], Y2P, bs + 2 * PL, 2, CURV || COM || APX ? site_mid : site_2, kp);
-#pragma unroll
-    for (int v = 0; v < VC; ++v) {
-      y3p.v[v] = input(XP[p2].v[v], dt, kp[v]);
-      AP.v[v] = add(AP.v[v], k.dt3, (double)kp[v]);
-    }
-    force(Y3F[p2], Y3F[p1], Y3F[p0], y3p, bs + 3 * PL, 3, CURV ? site_mid : site_4, kp);
-    const int nb = j >= 4 ? plane_bytes : 0;
-    V of, op;
-    if constexpr (MODE == TB_F64) {
+    if constexpr (decltype(with_b)::value != 0) {
+      HV y3p;
+      force(Y2F[p2], Y2F[p1], Y2F[p0], Y2P, bs + 2 * PL, 2, CURV || COM || APX ? site_mid : site_2, kp);
 #pragma unroll
       for (int v = 0; v < VC; ++v) {
-        of.v[v] = AF.v[v] + k.dt6 * y3p.v[v];
-        op.v[v] = AP.v[v] + k.dt6 * kp[v];
+        y3p.v[v] = input(XP[p2].v[v], dt, kp[v]);
+        AP.v[v] = add(AP.v[v], k.dt3, (double)kp[v]);
       }
-    } else {
-      TbVec<float, VC> olf, olp;
+      force(Y3F[p2], Y3F[p1], Y3F[p0], y3p, bs + 3 * PL, 3, CURV ? site_mid : site_4, kp);
+      V of, op;
+      if constexpr (MODE == TB_F64) {
 #pragma unroll
-      for (int v = 0; v < VC; ++v) {
-        double i0, i1;
-        if constexpr (MODE == TB_F32S) {
-          i0 = __builtin_fma(k.dt6, (double)y3p.v[v], AF.v[v]);
-          i1 = __builtin_fma(k.dt6, (double)kp[v], AP.v[v]);
-        } else {
-          i0 = (double)AF.v[v] + k.dt6 * (double)y3p.v[v];
-          i1 = (double)AP.v[v] + k.dt6 * kp[v];
+        for (int v = 0; v < VC; ++v) {
+          of.v[v] = AF.v[v] + k.dt6 * y3p.v[v];
+          op.v[v] = AP.v[v] + k.dt6 * kp[v];
         }
-        const double s0 = ((double)XF[p2].v[v] + (double)lf.v[v]) + i0;
-        const double s1 = ((double)XP[p2].v[v] + (double)lp.v[v]) + i1;
-        of.v[v] = (float)s0;
-        op.v[v] = (float)s1;
-        olf.v[v] = (float)(s0 - (double)of.v[v]);
-        olp.v[v] = (float)(s1 - (double)op.v[v]);
+      } else {
+        TbVec<float, VC> olf, olp;
+#pragma unroll
+        for (int v = 0; v < VC; ++v) {
+          double i0, i1;
+          if constexpr (MODE == TB_F32S) {
+            i0 = __builtin_fma(k.dt6, (double)y3p.v[v], AF.v[v]);
+            i1 = __builtin_fma(k.dt6, (double)kp[v], AP.v[v]);
+          } else {
+            i0 = (double)AF.v[v] + k.dt6 * (double)y3p.v[v];
+            i1 = (double)AP.v[v] + k.dt6 * kp[v];
+          }
+          const double s0 = ((double)XF[p2].v[v] + (double)lf.v[v]) + i0;
+          const double s1 = ((double)XP[p2].v[v] + (double)lp.v[v]) + i1;
+          of.v[v] = (float)s0;
+          op.v[v] = (float)s1;
+          olf.v[v] = (float)(s0 - (double)of.v[v]);
+          olp.v[v] = (float)(s1 - (double)op.v[v]);
+        }
+        tb_store<float, VC>(olf, tb_plane(lout + off_st, plane_bytes), st_off);
+        tb_store<float, VC>(olp, tb_plane(lout + N3 + off_st, plane_bytes), st_off);
       }
-      tb_store<float, VC>(olf, tb_plane(lout + off_st, nb), st_off);
-      tb_store<float, VC>(olp, tb_plane(lout + N3 + off_st, nb), st_off);
+      tb_store<T, VC>(of, tb_plane(xout + off_st, plane_bytes), st_off);
+      tb_store<T, VC>(op, tb_plane(xout + N3 + off_st, plane_bytes), st_off);
     }
-    tb_store<T, VC>(of, tb_plane(xout + off_st, nb), st_off);
-    tb_store<T, VC>(op, tb_plane(xout + N3 + off_st, nb), st_off);
     off_st = next_plane(off_st);
     Y2P = y2p;
     AF = af;
     AP = ap;
     site_mid = site_2;
   };
-  for (int j = 0;;) {
-    iteration(tb_ic<0>{}, tb_ic<0>{}, j);
+  iteration(tb_ic<2>{}, tb_ic<0>{}, tb_ic<0>{}, 2);
+  iteration(tb_ic<0>{}, tb_ic<1>{}, tb_ic<0>{}, 3);
+  for (int j = 4;;) {
+    iteration(tb_ic<1>{}, tb_ic<0>{}, tb_ic<1>{}, j);
     if (++j >= iters) break;
-    iteration(tb_ic<1>{}, tb_ic<1>{}, j);
+    iteration(tb_ic<2>{}, tb_ic<1>{}, tb_ic<1>{}, j);
     if (++j >= iters) break;
-    iteration(tb_ic<2>{}, tb_ic<0>{}, j);
+    iteration(tb_ic<0>{}, tb_ic<0>{}, tb_ic<1>{}, j);
     if (++j >= iters) break;
-    iteration(tb_ic<0>{}, tb_ic<1>{}, j);
+    iteration(tb_ic<1>{}, tb_ic<1>{}, tb_ic<1>{}, j);
     if (++j >= iters) break;
-    iteration(tb_ic<1>{}, tb_ic<0>{}, j);
+    iteration(tb_ic<2>{}, tb_ic<0>{}, tb_ic<1>{}, j);
     if (++j >= iters) break;
-    iteration(tb_ic<2>{}, tb_ic<1>{}, j);
+    iteration(tb_ic<0>{}, tb_ic<1>{}, tb_ic<1>{}, j);
     if (++j >= iters) break;
   }
 }
