@@ -39,6 +39,7 @@
 #include <vector>
 
 #include "cf_march.hpp"
+#include "cf_tb_body.hpp"
 
 namespace cf {
 
@@ -75,55 +76,23 @@ struct AdjStep {
   double two_m;             // 2m
 };
 
-// Tile of the v-th slot of the fixed grid's walk. Blocks go to the 8 XCDs round
-// robin (block mod 8), and a block's slots keep its residue, so when the tile
-// count allows, each XCD is given one contiguous range of tiles: the halo rows
-// and planes that neighbouring tiles share meet in one L2.
-__device__ __forceinline__ int adj_tile(int v, int total) {
-  return (total & 7) == 0 ? (v & 7) * (total >> 3) + (v >> 3) : v;
-}
-
 // The transposed Jacobian applied to a at a site, phi component:
 // (-m^2 - 3 lambda phi_y^2) a_pi + inv (sum of the six neighbours' a_pi - 6 a_pi).
 __device__ __forceinline__ double jt_phi(double c_m, double lam, double phi_y, double inv, double a0, double nb) {
   return (-c_m - 3.0 * lam * phi_y * phi_y) * a0 + inv * (nb - 6.0 * a0);
 }
 
-// Geometry of the backward step: a block of ADJ_R x ADJ_R threads, one per (b,c)
-// column of a region, marches planes [a0, a1) of one tile; the tile is the region
-// without a border of two columns (ADJ_T = ADJ_R - 4).
-constexpr int ADJ_R = 32;
-constexpr int ADJ_T = ADJ_R - 4;
-constexpr int ADJ_FT = ADJ_R * ADJ_R;  // threads per block
-
+// Geometry of the backward step: output tiles of Tb x Tc columns (the region of a shape
+// without a border of two on every side, or the whole extent of a smaller lattice) over
+// chunks of A planes, one work unit each.
 struct AdjGeom {
   int64_t N;
-  int nt;     // tiles per side (b and c)
-  int A;      // planes per chunk
-  int total;  // nt * nt * chunks
+  int shape;     // index into adj_shapes
+  int Tb, Tc;    // tile edges along b and c
+  int ntb, ntc;  // tiles along b and c
+  int A;         // planes per chunk
+  int total;     // ntb * ntc * chunks
 };
-
-// Plane slots of the step in LDS (112 KB: one block per CU).
-struct AdjLds {
-  double q[2][4][ADJ_FT];  // per column: x.phi, y1.phi, a4.pi, a3.pi of one plane; two planes
-  double w[3][2][ADJ_FT];  // per column: a2.pi, a1.pi of one plane; three planes
-  double red[ADJ_FT];      // block sums of the dL/dm partials
-};
-
-// s_waitcnt immediate (gfx9 encoding) that waits for the wave's LDS operations
-// (lgkmcnt 0) and for no vector-memory or export counter (vmcnt 63, expcnt 7).
-constexpr int ADJ_WAIT_LDS = 15 | (3 << 14) | (7 << 4);
-
-// Workgroup barrier for LDS plane slots only: every wave's LDS writes complete, then
-// s_barrier. Global loads in flight (the next plane's prefetch) stay in flight; a
-// __syncthreads() fence would wait for them too. The empty asm statements keep the
-// compiler from moving memory operations across the barrier.
-__device__ __forceinline__ void adj_barrier() {
-  asm volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(ADJ_WAIT_LDS);
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-}
 
 // Backward step, fused.
 //
@@ -147,149 +116,286 @@ __device__ __forceinline__ void adj_barrier() {
 //   half ((lambda' + ybar4 + ybar3) + ybar2 + ybar1).pi + (J(x)^T a1).pi
 // (the order of the running sum s).
 //
-// Per plane j of the march, every thread loads x and lambda' at its own site of
-// plane j+2 (used one iteration later, so the load overlaps a whole iteration) and
-//   A(j) on the region minus its outer ring: half A at plane j. The in-plane
-//        neighbours' x.phi, y1.phi, a4.pi and a3.pi come from the LDS slot of plane
-//        j (written by their owners one iteration earlier), the a-neighbours from the
-//        thread's own registers. w(j) goes to a ring of three LDS plane slots, s(j)
-//        stays in registers.
-//   barrier
-//   B(j-1) on the tile: half B at plane j-1, with w's in-plane neighbours from the
-//        slot of plane j-1 and its a-neighbours (j-2, j) from registers; writes lambda.
-// One barrier per plane suffices: A(j) rewrites the q slot that A(j-1) read and the w
-// slot that B(j-3) read, both before the previous barrier. s and w never reach HBM;
-// the step reads x and lambda' (2 x 16 B/site, times the region/tile area ratio) and
-// writes lambda (16 B/site). part: the dL/dm partials of stages 4, 3, 2, 1 of this
-// block, ADJ_BLOCKS apart (block 0 zeroes the slots of blocks beyond the grid). lo
-// must not overlap x or lp.
-template <bool LAM>
-__global__ __launch_bounds__(ADJ_FT) void k_adj_step(AdjGeom g, AdjStep k, const double *__restrict__ x,
-                                                     const double *__restrict__ lp, double *__restrict__ lo,
-                                                     double *__restrict__ part) {
-  __shared__ AdjLds S;
-  const int64_t N = g.N, NN = N * N, N3 = NN * N;
-  const int me = (int)threadIdx.x, tx = me & (ADJ_R - 1), ty = me / ADJ_R;
+// The march is that of the blocked forward step (cf_tb_body.hpp): each thread owns two
+// neighbouring columns of a row of the region, takes x and lambda' at plane P = a0 - 2 + j
+// in iteration j (loaded two iterations ahead through buffer resources over one plane)
+// and runs, side by side,
+//   A at P-1 (x.phi, y1.phi, a4.pi, a3.pi at P-2..P): half A; w and the sum s stay in registers
+//   B at P-2 (w at P-3..P-1): half B; writes lambda
+// The in-plane neighbours come from six LDS plane buffers (the four of A at P-1, w of P-2),
+// written together at the start of the iteration; with two sets of them one barrier per
+// plane suffices. The first output needs A from j = 2 on, so planes 0 and 1 come straight
+// from their loads and iterations 2 and 3 have no B. Results of region edges reach no
+// stored site and no sum. s and w never reach HBM; the step reads x and lambda'
+// (2 x 16 B/site, times the region/tile area ratio) and writes lambda (16 B/site).
+//
+// What bounds it: of the 1.7 us a plane of a 28 x 36 region takes, FP64 issue is 0.8 and
+// LDS 0.65 (two wavefronts per SIMD in step with the barrier overlap them only in part).
+// One column per thread (1024 threads, 128 VGPRs) took 32.1 us at N=128 against 27.9, 22 x
+// 68 regions spill. Before, with 28 x 28 tiles that share 128-byte lines with their
+// neighbours, one column per thread and half A masked per lane: 44 us.
+//
+// part: 4 ADJ_BLOCKS slots of which a block fills one with its dL/dm (all four stages) and
+// block 0 clears those of blocks beyond the grid. lo must not overlap x or lp.
+template <bool LAM, class SH>
+__global__ __launch_bounds__(SH::NT) void k_adj_step(AdjGeom g, AdjStep k, const double *x, const double *lp,
+                                                     double *lo, double *part) {
+  constexpr int VC = SH::VC, RC = SH::RC, PL = SH::PLANE;
+  typedef TbVec<double, VC> V;
+  __shared__ __attribute__((aligned(16))) double lds[12 * PL + 2 * RC];
+  const int N = (int)g.N;
+  const int64_t NN = g.N * g.N, N3 = NN * g.N;
+  const int plane_bytes = (int)(NN * 8);
+  const int tid = (int)threadIdx.x, r = tid / SH::TPR, cc = (tid % SH::TPR) * VC;
   const double c_m = k.r1.c_m, lam = k.r1.lam;
-  const bool in_a = tx >= 1 && tx <= ADJ_R - 2 && ty >= 1 && ty <= ADJ_R - 2;
-  // in-plane neighbours in a slot, in the rhs_pi argument order: b+1, b-1, c+1, c-1
-  const int o0 = me + ADJ_R, o1 = me - ADJ_R, o2 = me + 1, o3 = me - 1;
-  auto y1phi = [&](double f, double p) { return f + k.dh * p; };
-  auto a4pi = [&](double lpi) { return k.dt6 * lpi; };
-  auto a3pi = [&](double lphi, double lpi) {
-    const double yb4pi = k.dt6 * lphi + k.ch4 * a4pi(lpi);
-    return k.dt3 * lpi + k.dt * yb4pi;
-  };
-  double dm4 = 0.0, dm3 = 0.0, dm2 = 0.0, dm1 = 0.0;
-  for (int v = blockIdx.x; v < g.total; v += gridDim.x) {
-    const int t = adj_tile(v, g.total);
-    const int ct = t % g.nt, r = t / g.nt, bt = r % g.nt, ac = r / g.nt;
-    const int64_t b0 = (int64_t)bt * ADJ_T, c0 = (int64_t)ct * ADJ_T;
-    const int64_t a0 = (int64_t)ac * g.A, a1 = (a0 + g.A < N) ? a0 + g.A : N;
-    const int64_t nb_ = (N - b0 < ADJ_T) ? N - b0 : ADJ_T, nc_ = (N - c0 < ADJ_T) ? N - c0 : ADJ_T;
-    const bool out = ty >= 2 && ty < 2 + nb_ && tx >= 2 && tx < 2 + nc_;
-    const int64_t b = ((b0 - 2 + ty) % N + N) % N, c = ((c0 - 2 + tx) % N + N) % N;
-    const int64_t col = b * N + c;
-    auto site = [&](int64_t a) { return (a < 0 ? a + N : (a >= N ? a - N : a)) * NN + col; };
-    // own column: plane j-1 (p), j (c), j+1 (n, loaded), j+2 (loading)
-    int64_t i = site(a0 - 2);
-    double xp = x[i], yp = y1phi(xp, x[N3 + i]);
-    double fp = a4pi(lp[N3 + i]), gp = a3pi(lp[i], lp[N3 + i]);
-    i = site(a0 - 1);
-    double xc = x[i], xpic = x[N3 + i], lphic = lp[i], lpic = lp[N3 + i];
-    double yc = y1phi(xc, xpic), fc = a4pi(lpic), gc = a3pi(lphic, lpic);
-    i = site(a0);
-    double nx = x[i], npi = x[N3 + i], nlphi = lp[i], nlpi = lp[N3 + i];
-    S.q[0][0][me] = xc;
-    S.q[0][1][me] = yc;
-    S.q[0][2][me] = fc;
-    S.q[0][3][me] = gc;
-    // B's history: w at j-2, j-1 and s, lambda'.phi at j-1
-    double um2 = 0.0, um1 = 0.0, vm2 = 0.0, vm1 = 0.0, sphi_p = 0.0, spi_p = 0.0, lphi_p = 0.0;
-    adj_barrier();
-    int sq = 0, sw = 0, sw_p = 2;  // slot of plane j in q and w; w slot of plane j-1
-    for (int64_t j = a0 - 1; j <= a1; ++j) {
-      const double xn = nx, xpin = npi, lphin = nlphi, lpin = nlpi;
-      if (j + 2 <= a1 + 1) {  // plane j+2
-        i = site(j + 2);
-        nx = x[i];
-        npi = x[N3 + i];
-        nlphi = lp[i];
-        nlpi = lp[N3 + i];
+  double *me = lds + RC + r * RC + cc;
+  double dm = 0.0;
+  for (int q = blockIdx.x; q < g.total; q += gridDim.x) {
+    const int u = tb_xcd_order(q, g.total);
+    const int tc = u % g.ntc, rest = u / g.ntc, tb = rest % g.ntb, ac = rest / g.ntb;
+    const int b0 = tb * g.Tb, c0 = tc * g.Tc;
+    const int64_t a0 = (int64_t)ac * g.A, a1 = (a0 + g.A < g.N) ? a0 + g.A : g.N;
+    int b = (b0 - TBH + r) % N, c = (c0 - TBH + cc) % N;
+    if (b < 0) b += N;
+    if (c < 0) c += N;
+    const bool out = r >= TBH && r < TBH + g.Tb && b0 + (r - TBH) < N && cc >= TBH && cc < TBH + g.Tc &&
+                     c0 + (cc - TBH) < N;
+    const uint32_t ld_off = (uint32_t)(b * N + c) * 8u, st_off = out ? ld_off : TB_OOB;
+    auto next_plane = [&](int64_t off) -> int64_t {
+      off += NN;
+      return off == N3 ? 0 : off;
+    };
+    int64_t off_ld = ((a0 - TBH) % g.N + g.N) % g.N * NN, off_st = off_ld;
+    V LX[2], LXP[2], LL[2], LLP[2];
+    auto load = [&](int s) {
+      LX[s] = tb_load<double, VC>(tb_plane(x + off_ld, plane_bytes), ld_off);
+      LXP[s] = tb_load<double, VC>(tb_plane(x + N3 + off_ld, plane_bytes), ld_off);
+      LL[s] = tb_load<double, VC>(tb_plane(lp + off_ld, plane_bytes), ld_off);
+      LLP[s] = tb_load<double, VC>(tb_plane(lp + N3 + off_ld, plane_bytes), ld_off);
+      off_ld = next_plane(off_ld);
+    };
+    // histories: the value of plane P - d at [(phase - d) mod 3]
+    V X[3], XP[3], Y1[3], F4[3], G3[3], LF[3], LP[3], W0[3] = {}, W1[3] = {}, SF = {}, SI = {}, D = {};
+    auto take = [&](int h, int s) {
+#pragma unroll
+      for (int v = 0; v < VC; ++v) {
+        const double xf = LX[s].v[v], xp = LXP[s].v[v], lf = LL[s].v[v], li = LLP[s].v[v];
+        X[h].v[v] = xf;
+        XP[h].v[v] = xp;
+        LF[h].v[v] = lf;
+        LP[h].v[v] = li;
+        Y1[h].v[v] = xf + k.dh * xp;
+        F4[h].v[v] = k.dt6 * li;                                                  // a4.pi
+        G3[h].v[v] = k.dt3 * li + k.dt * (k.dt6 * lf + k.ch4 * F4[h].v[v]);       // a3.pi
       }
-      const double yn = y1phi(xn, xpin), fn = a4pi(lpin), gn = a3pi(lphin, lpin);
-      S.q[sq ^ 1][0][me] = xn;
-      S.q[sq ^ 1][1][me] = yn;
-      S.q[sq ^ 1][2][me] = fn;
-      S.q[sq ^ 1][3][me] = gn;
-      double sphi = 0.0, spi = 0.0, w0 = 0.0, w1 = 0.0;
-      if (in_a) {  // A(j)
-        const double *Q = S.q[sq][0];
-        const double *Y = S.q[sq][1];
-        const double *F4 = S.q[sq][2];
-        const double *G3 = S.q[sq][3];
-        // stage states at the site
-        const double y1pi = xpic + k.dh * rhs_pi(xc, xn, xp, Q[o0], Q[o1], Q[o2], Q[o3], xpic, k.r1, LAM);
-        const double y2pi = xpic + k.dh * rhs_pi(yc, yn, yp, Y[o0], Y[o1], Y[o2], Y[o3], y1pi, k.r2, LAM);
-        const double y2phi = xc + k.dh * y1pi;
-        const double y3phi = xc + k.dt * y2pi;
-        // stage 4 at y3 (t + dt)
-        const double nb4 = fn + fp + F4[o0] + F4[o1] + F4[o2] + F4[o3];
-        const double yb4phi = jt_phi(c_m, lam, y3phi, k.inv4, fc, nb4);
-        const double yb4pi = k.dt6 * lphic + k.ch4 * fc;
-        // stage 3 at y2 (t + dt/2)
-        const double nb3 = gn + gp + G3[o0] + G3[o1] + G3[o2] + G3[o3];
-        const double yb3phi = jt_phi(c_m, lam, y2phi, k.r2.inv, gc, nb3);
-        const double yb3pi = (k.dt3 * lphic + k.dt * yb4phi) + k.r2.c_h * gc;
-        // stage 2 at y1 (t + dt/2): the local part
-        const double a2pi = k.dt3 * lpic + k.dh * yb3pi;
-        const double a2phi = k.dt3 * lphic + k.dh * yb3phi;
-        const double yb2pi = a2phi + k.r2.c_h * a2pi;
-        if (out && j >= a0 && j < a1) {
-          dm4 += (-k.two_m * y3phi) * fc;
-          dm3 += (-k.two_m * y2phi) * gc;
-          dm2 += (-k.two_m * yc) * a2pi;
+    };
+    load(0);
+    load(1);
+    take(0, 0);
+    load(0);
+    take(1, 1);
+    load(1);
+    // the sum of a field's neighbours at column v; o its own plane, hi and lw those above
+    // and below, p its own slot in the plane buffer
+    struct Nb {
+      V up, dn;
+      double nx, pv;
+    };
+    auto in_plane = [&](const double *p) {
+      Nb n;
+      n.nx = p[VC];
+      n.pv = p[-1];
+      n.up = *(const V *)(p + RC);
+      n.dn = *(const V *)(p - RC);
+      return n;
+    };
+    auto cn = [&](const V &o, const Nb &n, int v) { return v + 1 < VC ? o.v[v + 1 < VC ? v + 1 : v] : n.nx; };
+    auto cp = [&](const V &o, const Nb &n, int v) { return v > 0 ? o.v[v > 0 ? v - 1 : v] : n.pv; };
+    auto iteration = [&](auto phase, auto set, auto with_b) {
+      constexpr int p0 = decltype(phase)::value, p1 = (p0 + 2) % 3, p2 = (p0 + 1) % 3;
+      constexpr int S = decltype(set)::value;
+      double *bs = me + S * 6 * PL;
+      take(p0, S);
+      *(V *)(bs) = X[p1];
+      *(V *)(bs + PL) = Y1[p1];
+      *(V *)(bs + 2 * PL) = F4[p1];
+      *(V *)(bs + 3 * PL) = G3[p1];
+      if constexpr (decltype(with_b)::value != 0) {
+        *(V *)(bs + 4 * PL) = W0[p2];
+        *(V *)(bs + 5 * PL) = W1[p2];
+      }
+      load(S);  // plane P+2
+      tb_barrier();
+      // ---- A at P-1
+      V y1pi, y2phi, y3phi, sf, si, d;
+      {
+        const Nb n = in_plane(bs);
+#pragma unroll
+        for (int v = 0; v < VC; ++v)
+          y1pi.v[v] = XP[p1].v[v] + k.dh * rhs_pi(X[p1].v[v], X[p0].v[v], X[p2].v[v], n.up.v[v], n.dn.v[v],
+                                                  cn(X[p1], n, v), cp(X[p1], n, v), XP[p1].v[v], k.r1, LAM);
+      }
+      {
+        const Nb n = in_plane(bs + PL);
+#pragma unroll
+        for (int v = 0; v < VC; ++v) {
+          const double y2pi = XP[p1].v[v] + k.dh * rhs_pi(Y1[p1].v[v], Y1[p0].v[v], Y1[p2].v[v], n.up.v[v],
+                                                          n.dn.v[v], cn(Y1[p1], n, v), cp(Y1[p1], n, v), y1pi.v[v],
+                                                          k.r2, LAM);
+          y2phi.v[v] = X[p1].v[v] + k.dh * y1pi.v[v];
+          y3phi.v[v] = X[p1].v[v] + k.dt * y2pi;
         }
-        sphi = (lphic + yb4phi) + yb3phi;
-        spi = ((lpic + yb4pi) + yb3pi) + yb2pi;
-        w0 = a2pi;
-        w1 = k.dt6 * lpic + k.dh * yb2pi;
-        S.w[sw][0][me] = w0;
-        S.w[sw][1][me] = w1;
       }
-      adj_barrier();
-      if (out && j > a0) {  // B(j-1): x.phi = xp, y1.phi = yp at j-1
-        const double *U = S.w[sw_p][0];
-        const double *V = S.w[sw_p][1];
-        const double nb2 = w0 + um2 + U[o0] + U[o1] + U[o2] + U[o3];
-        const double yb2phi = jt_phi(c_m, lam, yp, k.r2.inv, um1, nb2);
-        const double nb1 = w1 + vm2 + V[o0] + V[o1] + V[o2] + V[o3];
-        const double outphi = jt_phi(c_m, lam, xp, k.r1.inv, vm1, nb1);
-        const double outpi = (k.dt6 * lphi_p + k.dh * yb2phi) + k.r1.c_h * vm1;
-        const int64_t io = site(j - 1);
-        lo[io] = (sphi_p + yb2phi) + outphi;
-        lo[N3 + io] = spi_p + outpi;
-        dm1 += (-k.two_m * xp) * vm1;
+      V yb4phi;
+      {  // stage 4 at y3 (t + dt)
+        const Nb n = in_plane(bs + 2 * PL);
+#pragma unroll
+        for (int v = 0; v < VC; ++v) {
+          const double nb = F4[p0].v[v] + F4[p2].v[v] + n.up.v[v] + n.dn.v[v] + cn(F4[p1], n, v) + cp(F4[p1], n, v);
+          yb4phi.v[v] = jt_phi(c_m, lam, y3phi.v[v], k.inv4, F4[p1].v[v], nb);
+        }
       }
-      um2 = um1; um1 = w0;
-      vm2 = vm1; vm1 = w1;
-      sphi_p = sphi; spi_p = spi; lphi_p = lphic;
-      xp = xc; xc = xn; xpic = xpin; lphic = lphin; lpic = lpin;
-      yp = yc; yc = yn;
-      fp = fc; fc = fn;
-      gp = gc; gc = gn;
-      sq ^= 1;
-      sw_p = sw;
-      sw = (sw == 2) ? 0 : sw + 1;
+      {  // stage 3 at y2 and the local part of stage 2 at y1 (t + dt/2)
+        const Nb n = in_plane(bs + 3 * PL);
+#pragma unroll
+        for (int v = 0; v < VC; ++v) {
+          const double fc = F4[p1].v[v], gc = G3[p1].v[v], lf = LF[p1].v[v], li = LP[p1].v[v];
+          const double nb = G3[p0].v[v] + G3[p2].v[v] + n.up.v[v] + n.dn.v[v] + cn(G3[p1], n, v) + cp(G3[p1], n, v);
+          const double yb3phi = jt_phi(c_m, lam, y2phi.v[v], k.r2.inv, gc, nb);
+          const double yb4pi = k.dt6 * lf + k.ch4 * fc;
+          const double yb3pi = (k.dt3 * lf + k.dt * yb4phi.v[v]) + k.r2.c_h * gc;
+          const double a2pi = k.dt3 * li + k.dh * yb3pi;
+          const double a2phi = k.dt3 * lf + k.dh * yb3phi;
+          const double yb2pi = a2phi + k.r2.c_h * a2pi;
+          d.v[v] = y3phi.v[v] * fc + y2phi.v[v] * gc + Y1[p1].v[v] * a2pi;
+          sf.v[v] = (lf + yb4phi.v[v]) + yb3phi;
+          si.v[v] = ((li + yb4pi) + yb3pi) + yb2pi;
+          W0[p1].v[v] = a2pi;
+          W1[p1].v[v] = k.dt6 * li + k.dh * yb2pi;
+        }
+      }
+      // ---- B at P-2 (SF, SI, D: from A of the iteration before)
+      if constexpr (decltype(with_b)::value != 0) {
+        const Nb nu = in_plane(bs + 4 * PL), nv = in_plane(bs + 5 * PL);
+        V of, op;
+#pragma unroll
+        for (int v = 0; v < VC; ++v) {
+          const double xf = X[p2].v[v], um1 = W0[p2].v[v], vm1 = W1[p2].v[v];
+          const double nb2 = W0[p1].v[v] + W0[p0].v[v] + nu.up.v[v] + nu.dn.v[v] + cn(W0[p2], nu, v) + cp(W0[p2], nu, v);
+          const double yb2phi = jt_phi(c_m, lam, Y1[p2].v[v], k.r2.inv, um1, nb2);
+          const double nb1 = W1[p1].v[v] + W1[p0].v[v] + nv.up.v[v] + nv.dn.v[v] + cn(W1[p2], nv, v) + cp(W1[p2], nv, v);
+          const double outphi = jt_phi(c_m, lam, xf, k.r1.inv, vm1, nb1);
+          const double outpi = (k.dt6 * LF[p2].v[v] + k.dh * yb2phi) + k.r1.c_h * vm1;
+          of.v[v] = (SF.v[v] + yb2phi) + outphi;
+          op.v[v] = SI.v[v] + outpi;
+          const double s = D.v[v] + xf * vm1;
+          dm += out ? -k.two_m * s : 0.0;
+        }
+        tb_store<double, VC>(of, tb_plane(lo + off_st, plane_bytes), st_off);
+        tb_store<double, VC>(op, tb_plane(lo + N3 + off_st, plane_bytes), st_off);
+      }
+      off_st = next_plane(off_st);
+      SF = sf;
+      SI = si;
+      D = d;
+    };
+    const int iters = (int)(a1 - a0) + 4;
+    iteration(tb_ic<2>{}, tb_ic<0>{}, tb_ic<0>{});
+    iteration(tb_ic<0>{}, tb_ic<1>{}, tb_ic<0>{});
+    for (int j = 4;;) {
+      iteration(tb_ic<1>{}, tb_ic<0>{}, tb_ic<1>{});
+      if (++j >= iters) break;
+      iteration(tb_ic<2>{}, tb_ic<1>{}, tb_ic<1>{});
+      if (++j >= iters) break;
+      iteration(tb_ic<0>{}, tb_ic<0>{}, tb_ic<1>{});
+      if (++j >= iters) break;
+      iteration(tb_ic<1>{}, tb_ic<1>{}, tb_ic<1>{});
+      if (++j >= iters) break;
+      iteration(tb_ic<2>{}, tb_ic<0>{}, tb_ic<1>{});
+      if (++j >= iters) break;
+      iteration(tb_ic<0>{}, tb_ic<1>{}, tb_ic<1>{});
+      if (++j >= iters) break;
+    }
+    tb_barrier();  // the plane buffers are read until here: the next unit, or the sum below
+  }
+  // fixed-order sum over the block: within the wavefronts, then over them
+#pragma unroll
+  for (int s = 32; s > 0; s >>= 1) dm += __shfl_xor(dm, s);
+  if ((tid & 63) == 0) lds[tid >> 6] = dm;
+  __syncthreads();
+  if (tid == 0) {
+    double t = 0.0;
+    for (int w = 0; w < SH::NT / 64; ++w) t += lds[w];
+    part[blockIdx.x] = t;
+  }
+  if (blockIdx.x == 0)
+    for (int sl = (int)gridDim.x + tid; sl < 4 * ADJ_BLOCKS; sl += SH::NT) part[sl] = 0.0;
+}
+
+// Region shapes of the backward step, smallest first: blocks that a CU holds at a time (the
+// two-column kernels take 230-245 VGPRs, two wavefronts per SIMD), the time of a plane
+// iteration in us with one block on the CU and, per block, with all of them.
+typedef TbShape<12, 20, 2, 128> AdjS12x20;
+typedef TbShape<14, 36, 1, 512> AdjS14x36;
+typedef TbShape<28, 36, 2, 512> AdjS28x36;
+struct AdjShapeInfo {
+  int rb, rc, resident;
+  double t1, tau;
+};
+
+// Shape and chunk of the backward step: the least modelled time, the larger of the busiest
+// CU's plane iterations (chunk + 2 each, as in tb_cost) and the bytes passed at 5.5 TB/s
+// (8.8 while they fit the 256 MB cache). Measured (us a step; one rule over 32 x 32 regions
+// of 28 x 28 tiles / here; the same N with the other shapes): N=32 14 / 5.6 (6.1, 7.6),
+// 64 23 / 8.8 (10.5, 10.0), 128 44 / 27.9 (32.6, 30.6), 256 290 / 200 (-, 225).
+static AdjGeom adj_geom(int64_t N) {
+  static const AdjShapeInfo shapes[3] = {
+      {12, 20, 4, 0.80, 0.43}, {14, 36, 1, 0.87, 0.87}, {28, 36, 1, 1.75, 1.75}};
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+    cus = 256;
+  AdjGeom best{};
+  double best_cost = -1.0;
+  for (int s = 0; s < 3; ++s) {
+    const AdjShapeInfo &sh = shapes[s];
+    AdjGeom g;
+    g.N = N;
+    g.shape = s;
+    g.Tb = N < sh.rb - 2 * TBH ? (int)N : sh.rb - 2 * TBH;
+    g.Tc = N < sh.rc - 2 * TBH ? (int)N : sh.rc - 2 * TBH;
+    g.ntb = (int)cdiv(N, g.Tb);
+    g.ntc = (int)cdiv(N, g.Tc);
+    for (int64_t k = 1; k <= N;) {  // every distinct ceil(N / k)
+      g.A = (int)cdiv(N, k);
+      g.total = g.ntb * g.ntc * (int)cdiv(N, g.A);
+      const int64_t n = cdiv(g.total, cus), full = n / sh.resident, rest = n % sh.resident;
+      const double one = std::max(sh.t1, (double)rest * sh.tau);
+      const double cu = 3.2 + (double)(g.A + 2) * ((double)full * sh.resident * sh.tau + (rest ? one : 0.0));
+      const double loads = 32.0 * (double)g.total * sh.rb * sh.rc * (double)(g.A + 2 * TBH);
+      const double sites = (double)N * (double)N * (double)N;
+      const double bw = 48.0 * sites <= 256e6 ? 8.8e6 : 5.5e6;
+      const double cost = std::max(cu, (loads + 16.0 * sites) / bw);
+      if (best_cost < 0.0 || cost < best_cost) {
+        best = g;
+        best_cost = cost;
+      }
+      k = g.A > 1 ? (N + g.A - 2) / (g.A - 1) : N + 1;
     }
   }
-  block_partial<ADJ_FT>(dm4, part + blockIdx.x, me, S.red);
-  block_partial<ADJ_FT>(dm3, part + ADJ_BLOCKS + blockIdx.x, me, S.red);
-  block_partial<ADJ_FT>(dm2, part + 2 * ADJ_BLOCKS + blockIdx.x, me, S.red);
-  block_partial<ADJ_FT>(dm1, part + 3 * ADJ_BLOCKS + blockIdx.x, me, S.red);
-  if (blockIdx.x == 0)
-    for (int sl = (int)gridDim.x + me; sl < ADJ_BLOCKS; sl += ADJ_FT)
-      for (int st = 0; st < 4; ++st) part[st * ADJ_BLOCKS + sl] = 0.0;
+  return best;
+}
+
+template <bool LAM>
+static void adj_launch(const AdjGeom &g, const AdjStep &k, const double *x, const double *li, double *lo, double *part,
+                       hipStream_t st) {
+  const dim3 grid(g.total < 4 * ADJ_BLOCKS ? g.total : 4 * ADJ_BLOCKS);
+  if (g.shape == 0)
+    hipLaunchKernelGGL((k_adj_step<LAM, AdjS12x20>), grid, dim3(AdjS12x20::NT), 0, st, g, k, x, li, lo, part);
+  else if (g.shape == 1)
+    hipLaunchKernelGGL((k_adj_step<LAM, AdjS14x36>), grid, dim3(AdjS14x36::NT), 0, st, g, k, x, li, lo, part);
+  else
+    hipLaunchKernelGGL((k_adj_step<LAM, AdjS28x36>), grid, dim3(AdjS28x36::NT), 0, st, g, k, x, li, lo, part);
 }
 
 // Half-spectrum fk *= 2 w[s].
@@ -404,36 +510,6 @@ cf_status cf_loss_spectrum_adjoint(cf_spectrum_plan *plan, const cf_kg_params *p
   return CF_OK;
 }
 
-// Chunk of the backward step's march. One 1024-thread block runs per CU at a time
-// (112 KB of LDS), so k chunks per tile cost about ceil(tiles k / CUs) rounds of
-// (N/k + 3) plane iterations (two extra planes of half A and the prologue's loads);
-// among the k within 2% of the cheapest the largest is taken (N=128: 25 tiles x 10
-// chunks of 13 planes, one round on 256 CUs).
-static AdjGeom adj_geom(int64_t N) {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
-    cus = 256;
-  AdjGeom g;
-  g.N = N;
-  g.nt = (int)cdiv(N, ADJ_T);
-  const int64_t tiles = (int64_t)g.nt * g.nt;
-  std::vector<int64_t> cost((size_t)N + 1, -1);
-  int64_t best = -1;
-  for (int64_t k = 1; k <= N; ++k) {
-    const int64_t ch = cdiv(N, k);
-    if (cdiv(N, ch) != k) continue;  // chunks actually launched for this chunk length
-    cost[k] = cdiv(tiles * k, cus) * (ch + 3);
-    if (best < 0 || cost[k] < best) best = cost[k];
-  }
-  int64_t pick = 1;
-  for (int64_t k = 1; k <= N; ++k)
-    if (cost[k] >= 0 && cost[k] * 100 <= best * 102) pick = k;
-  g.A = (int)cdiv(N, pick);
-  g.total = (int)(tiles * cdiv(N, g.A));
-  return g;
-}
-
 // One backward step from state x at time t: lo = dL/dx_n from li = dL/dx_{n+1};
 // part: 4*ADJ_BLOCKS partials of dL/dm (stages 4, 3, 2, 1). lo overlaps neither x
 // nor li.
@@ -461,11 +537,8 @@ static cf_status adj_step(const cf_kg_params *p, const double *x, double t, doub
   k.dt6 = dt / 6.0;
   k.two_m = 2.0 * p->m;
   const AdjGeom g = adj_geom(N);
-  const dim3 grid(g.total < ADJ_BLOCKS ? g.total : ADJ_BLOCKS), blk(ADJ_FT);
-  if (p->lambda != 0.0)
-    hipLaunchKernelGGL(k_adj_step<true>, grid, blk, 0, st, g, k, x, li, lo, part);
-  else
-    hipLaunchKernelGGL(k_adj_step<false>, grid, blk, 0, st, g, k, x, li, lo, part);
+  if (p->lambda != 0.0) adj_launch<true>(g, k, x, li, lo, part, st);
+  else adj_launch<false>(g, k, x, li, lo, part, st);
   CF_LAUNCHED();
   return CF_OK;
 }

@@ -125,6 +125,32 @@ def test_step_adjoint_partial_tiles_vs_torch(cfl, O, N, lam):
     assert abs(host(part).sum() - gm.item()) <= 1e-12 * abs(gm.item())
 
 
+@pytest.mark.parametrize("N,lam", [(8, 0.2), (16, 0.0), (18, 0.2), (32, 0.0), (66, 0.2), (90, 0.0), (130, 0.2)])
+def test_step_adjoint_tile_edges_vs_torch(cfl, O, N, lam):
+    """One step back at the edges of the backward kernel's tiles and chunks (8 x 16, 10 x
+    32 and 24 x 32 sites): whole tiles, a remainder of two, chunks that end early. The
+    step's few hundred roundings per site stay below 1e-13 of the largest value."""
+    import ctypes as C
+    print(f"case step adjoint edges N={N} lam={lam}", flush=True)
+    L, m, t, dt = float(N), 1.1, 1.3, 0.06
+    cosmo_o = O.Cosmo.radiation(**FRW)
+    rng = np.random.default_rng(N)
+    x = np.concatenate([0.5 * rng.standard_normal(N ** 3), 0.3 * rng.standard_normal(N ** 3)])
+    lamv = rng.standard_normal(2 * N ** 3)
+    p = cfl.kg_params(N, L, m, lam, cfl.radiation(**FRW))
+    ld = torch.from_numpy(lamv.copy()).cuda()
+    part = torch.full((4 * 512,), float("nan"), dtype=torch.float64, device="cuda")
+    work = torch.empty(2 * N ** 3, dtype=torch.float64, device="cuda")
+    cfl.check(cfl.lib.cf_rk4_step_adjoint_f64(C.byref(p), cfl._ptr(torch.from_numpy(x).cuda()), t, dt, cfl._ptr(ld),
+                                              cfl._ptr(part), cfl._ptr(work), cfl._stream()))
+    xt = torch.tensor(x, requires_grad=True)
+    mt = torch.tensor(m, dtype=torch.float64, requires_grad=True)
+    y = t_step(xt, N, L, mt, lam, cosmo_o, t, dt, O)
+    gx, gm = torch.autograd.grad(y, (xt, mt), grad_outputs=torch.from_numpy(lamv))
+    assert rel(host(ld), gx.numpy()) < 1e-13
+    assert abs(host(part).sum() - gm.item()) <= 1e-12 * max(abs(gm.item()), 1.0)
+
+
 @pytest.mark.parametrize("n_steps,ckpt,lam", [(24, 8, 0.0), (23, 5, 0.2), (7, 16, 0.0), (1, 1, 0.2)])
 def test_full_chain_vs_torch(cfl, O, n_steps, ckpt, lam):
     """Checkpointed forward + backward through n_steps equals torch autograd of the
