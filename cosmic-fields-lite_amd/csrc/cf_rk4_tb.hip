@@ -68,10 +68,9 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(WAVES, W
 }
 
 // The same step for the equation variants, FP64.
-template <int VAR, class SH>
-__global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_rk4_tb_var(
-    TbGeom g, TbStep k, const double *__restrict__ xin, double *__restrict__ xout, const double *__restrict__ psi,
-    TbPsi cps) {
+template <int VAR, class SH, int WAVES>
+__global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void k_rk4_tb_var(
+    TbGeom g, TbStep k, const double *xin, double *xout, const double *psi, TbPsi cps) {
   __shared__ __attribute__((aligned(16))) double smem[SH::LDS];
   tb_unit<TB_F64, false, SH, VAR>(smem, tb_unit_of(g, tb_xcd_order(blockIdx.x, g.total)), k, TbStepF{}, xin, nullptr,
                                   xout, nullptr, psi, cps);
@@ -99,16 +98,24 @@ typedef TbShape<14, 36, 1, 512> TbC14x36;     // a column per thread (TB_F32C, v
 typedef TbShape<28, 36, 1, 1024> TbC28x36;
 typedef TbShape<22, 68, 2, 768> TbC22x68;     // 768 threads: 168 VGPRs for float histories and double sums
 
-enum : int { TB_FAM_F64 = 0, TB_FAM_F32C = 1, TB_FAM_F32S = 2, TB_FAM_VAR = 3 };
+enum : int { TB_FAM_F64 = 0, TB_FAM_F32C = 1, TB_FAM_F32S = 2, TB_FAM_CURV = 3, TB_FAM_SQRT = 4, TB_FAM_COM = 5,
+             TB_FAM_APX = 6 };
+
+// Bytes a launch loads per region site and plane iteration: the state, and Psi (fixed
+// curvature) or Psi and dPsi/dt at three stage times (comoving; the coarse grid's 1/8).
+static const double tb_load_bytes[7] = {16.0, 16.0, 16.0, 24.0, 16.0, 64.0, 22.0};
 
 static const std::vector<TbShapeInfo> &tb_shapes(int family) {
-  static const std::vector<TbShapeInfo> t[4] = {
+  static const std::vector<TbShapeInfo> t[7] = {
       {{12, 20, 8, 0.68, 0.26, 4.9e6}, {14, 36, 4, 0.70, 0.47, 5.0e6}, {28, 36, 2, 1.00, 0.92, 5.1e6},
        {30, 68, 1, 2.00, 2.00, 5.55e6}},
       {{14, 36, 2, 0.75, 0.58, 4.6e6}, {28, 36, 1, 1.22, 1.22, 4.4e6}, {22, 68, 1, 1.73, 1.73, 5.0e6}},
       {{12, 20, 8, 0.60, 0.18, 3.9e6}, {14, 36, 4, 0.65, 0.39, 4.6e6}, {28, 36, 2, 0.84, 0.78, 4.65e6},
        {30, 68, 1, 1.65, 1.65, 5.2e6}, {15, 132, 1, 1.55, 1.55, 5.8e6}},
-      {{14, 36, 2, 0.9, 0.8, 4.6e6}, {28, 36, 1, 1.5, 1.5, 4.9e6}},
+      {{14, 36, 2, 0.82, 0.68, 5.3e6}, {28, 36, 1, 1.44, 1.44, 5.1e6}, {22, 68, 1, 1.99, 1.99, 5.5e6}},
+      {{14, 36, 2, 1.22, 1.13, 5.0e6}, {28, 36, 1, 2.29, 2.29, 5.0e6}, {22, 68, 1, 3.40, 3.40, 5.2e6}},
+      {{14, 36, 2, 1.25, 1.09, 6.1e6}, {28, 36, 1, 2.28, 2.28, 5.9e6}},
+      {{14, 36, 2, 1.05, 0.85, 4.0e6}, {28, 36, 1, 1.77, 1.77, 3.8e6}},
   };
   return t[family];
 }
@@ -153,19 +160,21 @@ static TbGeom tb_geom(int family, int shape, int64_t N, int A, int64_t a_lo, int
 //   blocks run `resident` at a time, A + 4 iterations each at tau per block (t1 when one
 //   runs alone), of which the two that only load and the two without k3 and k4 cost two;
 //   the bytes it passes: the loads of every region and iteration and the stores, at bw
-//   (60% more while both states fit the 256 MB cache). Beyond it blocks of long chunks
+//   (60% more while all of it fits the 256 MB cache). Beyond it blocks of long chunks
 //   drift apart and find less of their neighbours' planes in L2: 5% per 100 planes.
 // Few chunks leave CUs idle, many repeat warm-up planes; small regions repeat halos.
 // Within 4% of the best of 6 to 12 measured (shape, chunk) pairs at each of N = 32, 64,
-// 96, 128, 160, 200, 250, 300, 384, 512 and storage form, in half of them the best.
-static double tb_cost(const TbShapeInfo &s, const TbGeom &g, int cus) {
+// 96, 128, 160, 200, 250, 300, 384, 512 and storage form, in half of them the best (the
+// variants, to N=384: mostly the best, within 11%).
+static double tb_cost(int family, const TbShapeInfo &s, const TbGeom &g, int cus) {
   const int64_t n = cdiv(g.total, cus), full = n / s.resident, rest = n % s.resident;
   const double one = std::max(s.t1, (double)rest * s.tau);
   const double cu = 1.8 + (double)(g.A + 2) * ((double)full * s.resident * s.tau + (rest ? one : 0.0));
   const double sites = (double)g.N * (double)g.N * (double)(g.a_hi - g.a_lo);
-  const bool cached = 32.0 * sites <= 256e6;
+  const double lb = tb_load_bytes[family];
+  const bool cached = (lb + 16.0) * sites <= 256e6;
   const double drift = cached ? 1.0 : 1.0 + 5e-4 * (double)g.A;
-  const double loads = 16.0 * (double)g.ntb * g.ntc * g.n_ac * s.rb * s.rc * (double)(g.A + 2 * TBH) * drift;
+  const double loads = lb * (double)g.ntb * g.ntc * g.n_ac * s.rb * s.rc * (double)(g.A + 2 * TBH) * drift;
   return std::max(cu, (loads + 16.0 * sites) / (cached ? 1.6 * s.bw : s.bw));
 }
 
@@ -187,7 +196,7 @@ static TbGeom tb_plan(int family, int64_t N, int chunk, int64_t a_lo, int64_t a_
     double least = -1.0;
     for (size_t i = 0; i < shapes.size(); ++i) {
       const TbGeom g = tb_geom(family, (int)i, N, A, a_lo, a_hi, NA);
-      const double c = tb_cost(shapes[i], g, cus);
+      const double c = tb_cost(family, shapes[i], g, cus);
       if (least < 0.0 || c < least) least = c;
       if (best_cost < 0.0 || c < best_cost) {
         best = g;
@@ -342,15 +351,20 @@ static cf_status tb_check(const cf_kg_params *p) {
   return CF_OK;
 }
 
+// The variants' kernels. 22 x 68 regions of two columns per thread for those whose site
+// factors fit the registers so (168 of them; fixed curvature, N=300: 296 -> 230 us a step,
+// N=256: 173 -> 154); the comoving ones would spill a hundred.
 template <int VAR>
 static void tb_launch_var(const TbGeom &g, const TbStep &k, const double *xin, double *xout, const double *psi,
                           const TbPsi &cp, hipStream_t st) {
-  if (g.shape == 0)
-    hipLaunchKernelGGL((k_rk4_tb_var<VAR, TbC14x36>), dim3((unsigned)g.total), dim3(TbC14x36::NT), 0, st, g, k, xin,
-                       xout, psi, cp);
-  else
-    hipLaunchKernelGGL((k_rk4_tb_var<VAR, TbC28x36>), dim3((unsigned)g.total), dim3(TbC28x36::NT), 0, st, g, k, xin,
-                       xout, psi, cp);
+  const dim3 grid((unsigned)g.total);
+  if (g.shape == 0) {
+    hipLaunchKernelGGL((k_rk4_tb_var<VAR, TbC14x36, 4>), grid, dim3(TbC14x36::NT), 0, st, g, k, xin, xout, psi, cp);
+  } else if (g.shape == 1) {
+    hipLaunchKernelGGL((k_rk4_tb_var<VAR, TbC28x36, 4>), grid, dim3(TbC28x36::NT), 0, st, g, k, xin, xout, psi, cp);
+  } else if constexpr (VAR == TB_FIXED_CURVATURE || VAR == TB_SQRT_POTENTIAL) {
+    hipLaunchKernelGGL((k_rk4_tb_var<VAR, TbC22x68, 3>), grid, dim3(TbC22x68::NT), 0, st, g, k, xin, xout, psi, cp);
+  }
 }
 
 cf_status tb_step_variant(int var, const cf_kg_params *p, double f_a, const double *psi, const double *xin,
@@ -363,7 +377,11 @@ cf_status tb_step_variant(int var, const cf_kg_params *p, double f_a, const doub
   const size_t n = 2 * (size_t)p->N * p->N * p->N;
   CF_REQUIRE(xin && xout && disjoint(xin, xout, n * sizeof(double)),
              "temporally blocked variant step: null or overlapping state buffers");
-  const TbGeom g = tb_plan(TB_FAM_VAR, p->N, chunk, 0, p->N, p->N);
+  const int family = var == TB_FIXED_CURVATURE  ? TB_FAM_CURV
+                     : var == TB_SQRT_POTENTIAL ? TB_FAM_SQRT
+                     : var == TB_COMOVING       ? TB_FAM_COM
+                                                : TB_FAM_APX;
+  const TbGeom g = tb_plan(family, p->N, chunk, 0, p->N, p->N);
   TbStep k = tb_step_host(p, t, dt);
   k.fa2 = f_a * f_a;
   const TbPsi cp = cps ? *cps : TbPsi{};

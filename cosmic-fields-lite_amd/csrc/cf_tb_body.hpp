@@ -266,7 +266,7 @@ template <int MODE, bool LAM, class SH, int VAR = TB_KG, bool PACE = false>
 __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbStep &k, const TbStepF &kf,
                                         const void *xin_, const float *lin, void *xout_, float *lout,
                                         const double *psi = nullptr, const TbPsi cps = TbPsi{}) {
-  static_assert(VAR == TB_KG || (MODE == TB_F64 && SH::VC == 1), "the equation variants are FP64, a column per thread");
+  static_assert(VAR == TB_KG || MODE == TB_F64, "the equation variants are FP64");
   constexpr int VC = SH::VC, RC = SH::RC, PL = SH::PLANE;
   typedef std::conditional_t<MODE == TB_F64, double, float> T;   // storage
   typedef TbElem<MODE, SH> H;                                    // histories, plane buffers
@@ -343,17 +343,19 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
   constexpr bool CURV = VAR == TB_FIXED_CURVATURE, COM = VAR == TB_COMOVING, APX = VAR == TB_APPROX_COMOVING;
   const int64_t G3 = APX ? cps.G * cps.G * cps.G : N3;
   const int field_bytes = APX ? (int)(cps.G * cps.G * 8) : plane_bytes;
-  uint32_t ps_off = ld_off;
+  uint32_t ps_off[VC] = {};
   int64_t off_a = 0, off_b = 0;        // plane offsets of the next iteration's A and B in Psi's grid
   int rem_a = 0, rem_b = 0;            // APX: planes passed within the coarse plane
-  double psA[2] = {0.0, 0.0}, dpA[2] = {0.0, 0.0}, psB = 0.0, dpB = 0.0;
-  TbSite site_mid = {0.0, 0.0, 0.0};   // of B's plane, from the iteration before
+  TbVec<double, VC> psA[2] = {}, dpA[2] = {}, psB = {}, dpB = {};
+  TbSite site_mid[VC] = {};            // of B's plane, from the iteration before
   if constexpr (CURV || COM) {
     off_a = wrap(u.a0 - 1);
     off_b = wrap(u.a0 - 2);
   } else if constexpr (APX) {
     const int sd = (int)cps.sd, hs = (int)cps.hs;
-    ps_off = (uint32_t)((((b + hs) % N) / sd) * (int)cps.G + ((c + hs) % N) / sd) * 8u;
+#pragma unroll
+    for (int v = 0; v < VC; ++v)
+      ps_off[v] = (uint32_t)((((b + hs) % N) / sd) * (int)cps.G + ((c + v + hs) % N) / sd) * 8u;
     auto cell = [&](int64_t P, int64_t &off, int &rem) {
       const int q = (int)(((P + 2 * u.NA) % u.NA + hs) % u.NA);
       off = (int64_t)(q / sd) * cps.G * cps.G;
@@ -362,8 +364,12 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
     cell(u.a0 - 1, off_a, rem_a);
     cell(u.a0 - 2, off_b, rem_b);
   }
-  auto field = [&](const double *f, int64_t off) {
-    return tb_load<double, 1>(tb_plane(f + off, field_bytes), ps_off).v[0];
+  auto field = [&](const double *f, int64_t off, uint32_t lane) {
+    if constexpr (!APX) return tb_load<double, VC>(tb_plane(f + off, field_bytes), lane);
+    TbVec<double, VC> r;
+#pragma unroll
+    for (int v = 0; v < VC; ++v) r.v[v] = tb_load<double, 1>(tb_plane(f + off, field_bytes), ps_off[v]).v[0];
+    return r;
   };
   auto step_cell = [&](int64_t &off, int &rem) {
     if (++rem == (int)cps.sd) {
@@ -374,15 +380,15 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
   };
   auto load_psi = [&]() {
     if constexpr (CURV) {
-      psA[0] = field(psi, off_a);
+      psA[0] = field(psi, off_a, ld_off);
       off_a = next_plane(off_a);
     } else if constexpr (COM || APX) {
-      psA[0] = field(cps.f[0], off_a);
-      dpA[0] = field(cps.f[0] + G3, off_a);
-      psA[1] = field(cps.f[1], off_a);
-      dpA[1] = field(cps.f[1] + G3, off_a);
-      psB = field(cps.f[2], off_b);
-      dpB = field(cps.f[2] + G3, off_b);
+      psA[0] = field(cps.f[0], off_a, ld_off);
+      dpA[0] = field(cps.f[0] + G3, off_a, ld_off);
+      psA[1] = field(cps.f[1], off_a, ld_off);
+      dpA[1] = field(cps.f[1] + G3, off_a, ld_off);
+      psB = field(cps.f[2], off_b, st_off);
+      dpB = field(cps.f[2] + G3, off_b, st_off);
       if constexpr (COM) {
         off_a = next_plane(off_a);
         off_b = next_plane(off_b);
@@ -396,8 +402,8 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
 
   // k of one stage at the thread's columns: x0 the stage input's phi at the plane, xa and
   // xm at the planes above and below, pi its pi; bp its own slot in the plane buffer.
-  auto force = [&](const HV &x0, const HV &xa, const HV &xm, const HV &pi, const H *bp, int stage, const TbSite &s,
-                   Av(&out)[VC]) {
+  auto force = [&](const HV &x0, const HV &xa, const HV &xm, const HV &pi, const H *bp, int stage,
+                   const TbSite (&s)[VC], Av (&out)[VC]) {
     const H nx = bp[VC], pv = bp[-1];
     const HV up = *(const HV *)(bp + RC), dn = *(const HV *)(bp - RC);
 #pragma unroll
@@ -409,7 +415,7 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
       else
         out[v] = tb_force<VAR, LAM>((double)x0.v[v], (double)xa.v[v], (double)xm.v[v], (double)up.v[v],
                                     (double)dn.v[v], (double)cn, (double)cp, (double)pi.v[v], k.c_h[stage],
-                                    k.inv[stage], k, s);
+                                    k.inv[stage], k, s[v]);
     }
   };
   // a stage input x + c k (rounded to the storage type) and the increment d + c k
@@ -453,13 +459,16 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
       lp = LP[S];
       load_lo(S, j + 2);
     }
-    TbSite site_1 = {}, site_2 = {}, site_4 = {};
-    if constexpr (CURV) {
-      site_1 = site_2 = tb_site<VAR>(psA[0], 0.0, k.m);
-    } else if constexpr (COM || APX) {
-      site_1 = tb_site<VAR>(psA[0], dpA[0], k.m);
-      site_2 = tb_site<VAR>(psA[1], dpA[1], k.m);
-      site_4 = tb_site<VAR>(psB, dpB, k.m);
+    TbSite site_1[VC] = {}, site_2[VC] = {}, site_4[VC] = {};
+#pragma unroll
+    for (int v = 0; v < VC; ++v) {
+      if constexpr (CURV) {
+        site_1[v] = site_2[v] = tb_site<VAR>(psA[0].v[v], 0.0, k.m);
+      } else if constexpr (COM || APX) {
+        site_1[v] = tb_site<VAR>(psA[0].v[v], dpA[0].v[v], k.m);
+        site_2[v] = tb_site<VAR>(psA[1].v[v], dpA[1].v[v], k.m);
+        site_4[v] = tb_site<VAR>(psB.v[v], dpB.v[v], k.m);
+      }
     }
     load_psi();
 #pragma unroll
@@ -543,7 +552,8 @@ __device__ __forceinline__ void tb_unit(void *smem, const TbUnit &u, const TbSte
     Y2P = y2p;
     AF = af;
     AP = ap;
-    site_mid = site_2;
+#pragma unroll
+    for (int v = 0; v < VC; ++v) site_mid[v] = site_2[v];
   };
   iteration(tb_ic<2>{}, tb_ic<0>{}, tb_ic<0>{}, 2);
   iteration(tb_ic<0>{}, tb_ic<1>{}, tb_ic<0>{}, 3);

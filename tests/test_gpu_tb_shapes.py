@@ -90,3 +90,27 @@ def test_odd_alignment(cfl, N):
         step(p, hi, lo, h2, l2, 1.0, 0.05)
         step(p, *[t[1:] for t in bufs], 1.0, 0.05)
         assert torch.equal(bufs[2][1:], h2) and torch.equal(bufs[3][1:], l2)
+
+
+@pytest.mark.parametrize("kind,N,chunk", [(1, 66, 3), (1, 130, 0), (1, 260, 0), (2, 130, 0), (2, 302, 0), (3, 98, 0)])
+def test_variant_step_equals_stage_kernels(cfl, O, kind, N, chunk):
+    """The variants' region shapes (10 x 32, 24 x 32, 18 x 64 tiles with remainders): two
+    blocked steps give the bits of the stage kernels, from a state on an odd double too."""
+    print(f"case tb shapes variant {kind} N={N} chunk={chunk}", flush=True)
+    p = cfl.kg_params(N, float(N), 1.0, 0.0, cfl.radiation(**FRW))
+    if kind == 3:
+        g = torch.Generator(device="cuda").manual_seed(5)
+        field = 1e-2 * torch.randn(2 * N * N * (N // 2 + 1), dtype=torch.float64, device="cuda", generator=g)
+    else:
+        field = dev(0.02 * rand_state(N, 34)[: N ** 3]) if kind == 1 else None
+    v = cfl.Variant(p, kind, field, f_a=1.3)
+    x = dev(rand_state(N, 35, amp=0.3))
+    ref = x.clone()
+    v.rk4_run(ref, 1.0, 0, 2, 0.05)
+    odd = torch.empty(2 * N ** 3 + 1, dtype=torch.float64, device="cuda")
+    odd[1:] = x
+    y, z = torch.full_like(x, float("nan")), torch.full_like(x, float("nan"))
+    v.rk4_step_tb(odd[1:], y, 1.0, 0.05, chunk=chunk)
+    v.rk4_step_tb(y, z, 1.05, 0.05, chunk=chunk)
+    assert torch.equal(z, ref)
+    v.close()
