@@ -151,7 +151,7 @@ __global__ __launch_bounds__(SH::NT) void k_adj_step(AdjGeom g, AdjStep k, const
   double *me = lds + RC + r * RC + cc;
   double dm = 0.0;
   for (int q = blockIdx.x; q < g.total; q += gridDim.x) {
-    const int u = tb_xcd_order(q, g.total);
+    const int u = xcd_order(q, g.total);
     const int tc = u % g.ntc, rest = u / g.ntc, tb = rest % g.ntb, ac = rest / g.ntb;
     const int b0 = tb * g.Tb, c0 = tc * g.Tc;
     const int64_t a0 = (int64_t)ac * g.A, a1 = (a0 + g.A < g.N) ? a0 + g.A : g.N;

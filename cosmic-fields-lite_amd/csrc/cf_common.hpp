@@ -58,4 +58,13 @@ double *plan_red(cf_spectrum_plan *p);
 double *plan_bins(cf_spectrum_plan *p);
 int64_t plan_size(const cf_spectrum_plan *p);  // its lattice size N
 
+// Logical block of hardware block b of a grid of `total` blocks. The dispatcher deals
+// blocks to the 8 XCDs in turn (b -> XCD b % 8, its (b / 8)-th block); XCD x is given
+// the contiguous logical range [x q + min(x, r), ...) of q or q + 1 blocks (q, r =
+// total / 8, total % 8), so neighbours share one L2. A bijection for any total.
+__device__ __forceinline__ int xcd_order(int b, int total) {
+  const int x = b & 7, i = b >> 3, q = total >> 3, r = total & 7;
+  return x * q + (x < r ? x : r) + i;
+}
+
 }  // namespace cf

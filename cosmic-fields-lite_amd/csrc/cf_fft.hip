@@ -63,17 +63,11 @@ __device__ __forceinline__ void fft_front(const FftLen &p, double2 *d, FftTables
   __syncthreads();
 }
 
-// Logical block of hardware block b: each of the 8 XCDs (b mod 8) gets a contiguous range,
-// so that blocks whose rows share 128-byte lines meet in one L2: packed rows of N/2 + 1
-// entries, and the folded powers' half lines. Dealt out in turn, each XCD wrote its part of
-// such a line by itself (pass along a into packed rows: N=384 350 -> 264 us, N=512 855 ->
-// 644; folded: 200 -> 179, 416 -> 373).
-__device__ __forceinline__ int fft_xcd_order(int b, int total) {
-  const int x = b & 7, q = total >> 3, r = total & 7;
-  return x * q + (x < r ? x : r) + (b >> 3);
-}
-
-// Pass along a or b, in place or from `in` to `out`. SCALE: times the scale at s. FOLD:
+// Pass along a or b, in place or from `in` to `out`. Contiguous blocks on an XCD: those whose
+// rows share 128-byte lines (packed rows of N/2 + 1 entries, the folded powers' half lines)
+// meet in one L2. Dealt out in turn, each XCD wrote its part of such a line by itself (pass
+// along a into packed rows: N=384 350 -> 264 us, N=512 855 -> 644; folded: 200 -> 179, 416
+// -> 373). SCALE: times the scale at s. FOLD:
 // powers folded over the pass's axis instead of the spectrum.
 template <int DIR, bool SCALE, bool FOLD>
 __global__ __launch_bounds__(512) void k_fft_cols(FftLen p, ColGeom gi, ColGeom go, const double2 *in, double2 *out,
@@ -83,7 +77,7 @@ __global__ __launch_bounds__(512) void k_fft_cols(FftLen p, ColGeom gi, ColGeom 
   const int last = p.stages - 1, nbl = p.n / p.rad[last];
   FftTables tb(p, data, FOLD ? p.pos : p.rev, FOLD ? p.n : nbl);
   const int l = threadIdx.x & (FFT_CW - 1), q = threadIdx.x / FFT_CW, dq = blockDim.x / FFT_CW;
-  const int block = fft_xcd_order((int)blockIdx.x, (int)gridDim.x), ct = block % gi.nct, row = block / gi.nct;
+  const int block = xcd_order((int)blockIdx.x, (int)gridDim.x), ct = block % gi.nct, row = block / gi.nct;
   const int c = ct * FFT_CW + l;
   const bool rd = c < gi.ncol, wr = c < go.ncol;
   const double2 *src = in + (int64_t)row * gi.row_stride + c;

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(WAVES, W
   __shared__ __attribute__((aligned(16))) TbElem<MODE, SH> smem[SH::LDS];
   // Blocks go to the 8 XCDs round robin; consecutive logical tiles are mapped
   // to one XCD so that neighbouring tiles' halos meet in its L2.
-  tb_unit<MODE, LAM, SH, TB_KG, PACE>(smem, tb_unit_of(g, tb_xcd_order(blockIdx.x, g.total)), k, kf, xin, lin, xout,
+  tb_unit<MODE, LAM, SH, TB_KG, PACE>(smem, tb_unit_of(g, xcd_order(blockIdx.x, g.total)), k, kf, xin, lin, xout,
                                       lout);
 }
 
@@ -72,7 +72,7 @@ template <int VAR, class SH, int WAVES>
 __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(WAVES, WAVES))) void k_rk4_tb_var(
     TbGeom g, TbStep k, const double *xin, double *xout, const double *psi, TbPsi cps) {
   __shared__ __attribute__((aligned(16))) double smem[SH::LDS];
-  tb_unit<TB_F64, false, SH, VAR>(smem, tb_unit_of(g, tb_xcd_order(blockIdx.x, g.total)), k, TbStepF{}, xin, nullptr,
+  tb_unit<TB_F64, false, SH, VAR>(smem, tb_unit_of(g, xcd_order(blockIdx.x, g.total)), k, TbStepF{}, xin, nullptr,
                                   xout, nullptr, psi, cps);
 }
 

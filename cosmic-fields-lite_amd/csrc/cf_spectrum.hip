@@ -38,7 +38,10 @@ struct cf_spectrum_plan {
   double *cbuf0 = nullptr;       // half-spectrum scratch (N*N*pitch entries)
   double *cbuf1 = nullptr;       // second half-spectrum scratch, or two fields' folded powers
   int64_t nr = 0;                // row classes r = as^2 + bs^2 <= 2 (N/2)^2
-  int32_t *roff = nullptr;       // nr+1 offsets into rows
+  int64_t nc = 0;                // ... of which this many have rows
+  int32_t *cls = nullptr;        // their r, ascending
+  int32_t *cidx = nullptr;       // class of r (nr entries), -1: no rows
+  int32_t *roff = nullptr;       // nc+1 offsets into rows
   int32_t *rows = nullptr;       // the N^2 rows (a*N + b) of the half spectrum sorted by r
   int32_t *foff = nullptr;       // the same for the (N/2 + 1) N rows (a'*N + b) of folded powers
   int32_t *frows = nullptr;
@@ -63,14 +66,18 @@ constexpr int RED_BLOCKS = 1024;
 // Binning (fdm3d.cpp:11-28 sums |f_k|^2 over the full k-cube by s = |n|^2; the half
 // spectrum counts interior c columns twice). With r = as^2 + bs^2 of a row (a, b),
 // s = r + c^2, so
-//   step A: Q[c][r] = sum over the rows of class r (in sorted order) of w(c)|f|^2 --
-//           whole c-rows are read, coalesced; RB consecutive r of one block are
-//           summed into an LDS tile and written out transposed;
-//   step B: P(s) = sum_{c ascending} Q[c][s - c^2], coalesced over consecutive s.
+//   step A: Q[c][k] = sum over the rows of the k-th class that has any (in sorted order) of
+//           w(c)|f|^2 -- whole c-rows are read, coalesced; RB consecutive classes of one
+//           block are summed into an LDS tile and written out transposed;
+//   step B: P(s) = sum_{c ascending} Q[c][class of s - c^2], over consecutive s.
+// Three of four r are no sum of two squares; with a slot of Q for each of them too, step A
+// wrote 269 MB at N=512 where 70 hold a sum (both steps: N=256 39 -> 25 us, N=384 99 -> 69,
+// N=512 229 -> 134).
 // Fixed summation orders, no atomics: bit-reproducible.
 constexpr int BIN_LDS = 4096;  // doubles of the step-A tile (32 KB: several blocks per CU)
 constexpr int BIN_MAX_RB = 256;  // row classes per block
 constexpr int BIN_LIST = 1024;   // rows of a block's classes kept in LDS
+constexpr int BIN_SPLIT = 8;     // wavefronts per 64 bins in step B
 constexpr int BIN_CQ = 9;      // 64-column chunks of a row: H = N/2 + 1 <= 513
 
 // CQ: 64-column chunks per row (CQ * 64 >= H). Each wavefront keeps bin_group rows
@@ -85,17 +92,18 @@ constexpr int bin_group(bool mode, int cq) {
 // Rows of `pitch` entries of type E: half-spectrum values (double2) or folded powers (double).
 template <bool MODE, int CQ, class E>
 __global__ __launch_bounds__(256) void k_bin_rows(const E *__restrict__ fk, const E *__restrict__ dk,
-                                                  const int32_t *__restrict__ roff, const int32_t *__restrict__ rows,
-                                                  int64_t H, int64_t pitch, int64_t nr, int lrb, double m2,
-                                                  double kir2, double a2, double *__restrict__ Q) {
+                                                  const int32_t *__restrict__ cls, const int32_t *__restrict__ roff,
+                                                  const int32_t *__restrict__ rows, int64_t H, int64_t pitch,
+                                                  int64_t nc, int lrb, double m2, double kir2, double a2,
+                                                  double *__restrict__ Q) {
   __shared__ double tile[BIN_LDS];
   __shared__ int32_t list[BIN_LIST], offs[BIN_MAX_RB + 1];
   const int RB = 1 << lrb;
-  const int64_t r0 = (int64_t)blockIdx.x * RB;
+  const int64_t r0 = (int64_t)xcd_order((int)blockIdx.x, (int)gridDim.x) * RB;
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   // the block's offsets and row list (contiguous) first, so that a class costs one memory
-  // latency and not three; most classes are empty (no two squares sum to r)
-  for (int i = threadIdx.x; i <= RB; i += 256) offs[i] = roff[r0 + i < nr ? r0 + i : nr];
+  // latency and not three
+  for (int i = threadIdx.x; i <= RB; i += 256) offs[i] = roff[r0 + i < nc ? r0 + i : nc];
   __syncthreads();
   const int32_t first = offs[0], count = offs[RB] - first;
   if (count <= BIN_LIST)
@@ -103,15 +111,9 @@ __global__ __launch_bounds__(256) void k_bin_rows(const E *__restrict__ fk, cons
   __syncthreads();
   auto row_of = [&](int32_t j) { return count <= BIN_LIST ? list[j - first] : rows[j]; };
   for (int rl = wave; rl < RB; rl += 4) {  // each wavefront its own row classes
-    const int64_t r = r0 + rl;
-    if (r >= nr) break;
+    if (r0 + rl >= nc) break;
     const int32_t beg = offs[rl], end = offs[rl + 1];
-    if (beg == end) {
-#pragma unroll
-      for (int q = 0; q < CQ; ++q)
-        if (lane + 64 * q < H) tile[rl * H + lane + 64 * q] = 0.0;
-      continue;
-    }
+    [[maybe_unused]] const int64_t r = MODE ? cls[r0 + rl] : 0;
     // lane holds columns c = lane + 64 q
     double acc[CQ];
     double denom[CQ];
@@ -170,30 +172,44 @@ __global__ __launch_bounds__(256) void k_bin_rows(const E *__restrict__ fk, cons
     }
   }
   __syncthreads();
-  const int64_t nrb = (r0 + RB <= nr) ? RB : nr - r0;
+  const int64_t nrb = (r0 + RB <= nc) ? RB : nc - r0;
   for (int64_t q = threadIdx.x; q < (int64_t)RB * H; q += blockDim.x) {
     const int64_t c = q >> lrb, rl = q & (RB - 1);
-    if (rl < nrb) Q[c * nr + r0 + rl] = tile[rl * H + c];
+    if (rl < nrb) Q[c * nc + r0 + rl] = tile[rl * H + c];
   }
 }
 
-__global__ __launch_bounds__(256) void k_bin_cols(const double *__restrict__ Q, int64_t H, int64_t nr, int64_t nb,
-                                                  double *__restrict__ bins) {
-  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nb) return;
-  // sixteen entries in flight, added in order of c (one at a time the loop waits out the
-  // memory latency for each: 48 us at N=256 for 34 MB)
+__global__ __launch_bounds__(64 * BIN_SPLIT) void k_bin_cols(const double *__restrict__ Q,
+                                                             const int32_t *__restrict__ cidx, int64_t H, int64_t nr,
+                                                             int64_t nc, int64_t nb, double *__restrict__ bins) {
+  // A wavefront takes 64 bins over a BIN_SPLIT-th of the columns, in order of c, the parts
+  // are added in order: N=256 leaves three wavefronts a CU otherwise, each waiting out the
+  // memory latency group by group (16 entries in flight: 16 us with a slot for every r, 21
+  // with classes to look up; split 10.8).
+  constexpr int G = 16;
+  __shared__ double part[BIN_SPLIT][64];
+  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int64_t s = (int64_t)blockIdx.x * 64 + lane, per = (H + BIN_SPLIT - 1) / BIN_SPLIT;
+  const int64_t beg = w * per, end = beg + per < H ? beg + per : H;
   double acc = 0.0;
-  for (int64_t c0 = 0; c0 < H && c0 * c0 <= s; c0 += 16) {
-    double v[16];
+  for (int64_t c0 = beg; c0 < end && c0 * c0 <= s; c0 += G) {
+    double v[G];
+    int32_t k[G];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
+    for (int i = 0; i < G; ++i) {
       const int64_t c = c0 + i, r = s - c * c;
-      v[i] = (c < H && r >= 0 && r < nr) ? Q[c * nr + r] : 0.0;
+      k[i] = (c < end && r >= 0 && r < nr) ? cidx[r] : -1;
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc += v[i];
+    for (int i = 0; i < G; ++i) v[i] = k[i] >= 0 ? Q[(c0 + i) * nc + k[i]] : 0.0;
+#pragma unroll
+    for (int i = 0; i < G; ++i) acc += v[i];
   }
+  part[w][lane] = acc;
+  __syncthreads();
+  if (w != 0 || s >= nb) return;
+#pragma unroll
+  for (int i = 1; i < BIN_SPLIT; ++i) acc += part[i][lane];
   bins[s] = acc;
 }
 
@@ -392,7 +408,7 @@ cf_status cf_spectrum_plan_destroy(cf_spectrum_plan *p) {
   if (p->have_d2z) hipfftDestroy(p->d2z);
   if (p->have_z2d) hipfftDestroy(p->z2d);
   p->fft.release();
-  void *bufs[] = {p->work, p->rbuf, p->cbuf0, p->cbuf1, p->roff, p->rows, p->foff, p->frows, p->red, p->bins};
+  void *bufs[] = {p->work, p->rbuf, p->cbuf0, p->cbuf1, p->cls, p->cidx, p->roff, p->rows, p->foff, p->frows, p->red, p->bins};
   for (void *b : bufs)
     if (b) (void)hipFree(b);
   delete p;
@@ -440,6 +456,8 @@ cf_status cf_spectrum_plan_create(int64_t N, cf_spectrum_plan **out) {
       hipMalloc((void **)&p->rbuf, n3 * sizeof(double)) != hipSuccess ||
       hipMalloc((void **)&p->cbuf0, cbytes) != hipSuccess ||
       hipMalloc((void **)&p->cbuf1, cbytes) != hipSuccess ||
+      hipMalloc((void **)&p->cls, (size_t)p->nr * sizeof(int32_t)) != hipSuccess ||
+      hipMalloc((void **)&p->cidx, (size_t)p->nr * sizeof(int32_t)) != hipSuccess ||
       hipMalloc((void **)&p->roff, ((size_t)p->nr + 1) * sizeof(int32_t)) != hipSuccess ||
       hipMalloc((void **)&p->rows, (size_t)(N * N) * sizeof(int32_t)) != hipSuccess ||
       hipMalloc((void **)&p->foff, ((size_t)p->nr + 1) * sizeof(int32_t)) != hipSuccess ||
@@ -457,8 +475,8 @@ cf_status cf_spectrum_plan_create(int64_t N, cf_spectrum_plan **out) {
     }
   }
   // Row tables: stable counting sort of the rows (a, b) by r = as^2 + bs^2, of all N^2 rows
-  // and of those with a <= N/2 (folded powers). The binning's step A output Q, H * nr <=
-  // N^3 doubles, lives in rbuf.
+  // and of those with a <= N/2 (folded powers), which have the same classes. The binning's
+  // step A output Q, H * nc <= N^3 doubles, lives in rbuf.
   auto row_table = [&](int64_t na, int32_t *off_dev, int32_t *rows_dev) {
     const int64_t nr = p->nr;
     std::vector<int32_t> off((size_t)nr + 1, 0);
@@ -470,7 +488,18 @@ cf_status cf_spectrum_plan_create(int64_t N, cf_spectrum_plan **out) {
     std::vector<int32_t> rws((size_t)(na * N));
     for (int64_t a = 0; a < na; ++a)
       for (int64_t b = 0; b < N; ++b) rws[pos[fold(a) * fold(a) + fold(b) * fold(b)]++] = (int32_t)(a * N + b);
-    return hipMemcpy(off_dev, off.data(), off.size() * sizeof(int32_t), hipMemcpyHostToDevice) == hipSuccess &&
+    std::vector<int32_t> cls, cidx((size_t)nr, -1), coff;  // the classes that have rows
+    for (int64_t q = 0; q < nr; ++q)
+      if (off[q + 1] > off[q]) {
+        cidx[q] = (int32_t)cls.size();
+        cls.push_back((int32_t)q);
+        coff.push_back(off[q]);
+      }
+    coff.push_back(off[nr]);
+    p->nc = (int64_t)cls.size();
+    return hipMemcpy(p->cls, cls.data(), cls.size() * sizeof(int32_t), hipMemcpyHostToDevice) == hipSuccess &&
+           hipMemcpy(p->cidx, cidx.data(), cidx.size() * sizeof(int32_t), hipMemcpyHostToDevice) == hipSuccess &&
+           hipMemcpy(off_dev, coff.data(), coff.size() * sizeof(int32_t), hipMemcpyHostToDevice) == hipSuccess &&
            hipMemcpy(rows_dev, rws.data(), rws.size() * sizeof(int32_t), hipMemcpyHostToDevice) == hipSuccess;
   };
   if (!row_table(N, p->roff, p->rows) || (own && !row_table(N / 2 + 1, p->foff, p->frows))) {
@@ -513,17 +542,19 @@ cf_status cf_fft_z2d_inplace(cf_spectrum_plan *p, double *inout, cf_stream strea
 static cf_status bin_launch(cf_spectrum_plan *p, const double *fk, const double *dk, bool fold, double m2,
                             double kir2, double a2, double *bins, hipStream_t st) {
   CF_REQUIRE(p->H <= 64 * BIN_CQ, "binning: N=%lld exceeds the row chunking", (long long)p->N);
-  int lrb = 0;  // RB = 2^lrb row classes per block: the largest power of two with RB * H <= BIN_LDS
-  while ((2 << lrb) * p->H <= BIN_LDS && lrb < 8) ++lrb;
-  const dim3 gA((unsigned)cdiv(p->nr, (int64_t)1 << lrb)), b256(256);
+  // RB = 2^lrb classes per block: as many as fit BIN_LDS, but two for each of its wavefronts
+  // where that leaves fewer than 1024 blocks
+  int lrb = 0;
+  while ((2 << lrb) * p->H <= BIN_LDS && lrb < 8 && (lrb < 3 || (p->nc >> (lrb + 1)) >= 1024)) ++lrb;
+  const dim3 gA((unsigned)cdiv(p->nc, (int64_t)1 << lrb)), b256(256);
   auto rows_kernel = [&](auto mode, auto cq) {
     if (fold)
       hipLaunchKernelGGL((k_bin_rows<decltype(mode)::value, decltype(cq)::value, double>), gA, b256, 0, st, fk, dk,
-                         p->foff, p->frows, p->H, p->pitch, p->nr, lrb, m2, kir2, a2, p->rbuf);
+                         p->cls, p->foff, p->frows, p->H, p->pitch, p->nc, lrb, m2, kir2, a2, p->rbuf);
     else
       hipLaunchKernelGGL((k_bin_rows<decltype(mode)::value, decltype(cq)::value, double2>), gA, b256, 0, st,
-                         (const double2 *)fk, (const double2 *)dk, p->roff, p->rows, p->H, p->H, p->nr, lrb, m2, kir2,
-                         a2, p->rbuf);
+                         (const double2 *)fk, (const double2 *)dk, p->cls, p->roff, p->rows, p->H, p->H, p->nc, lrb,
+                         m2, kir2, a2, p->rbuf);
   };
   auto by_cq = [&](auto mode) {
     const int64_t cq = cdiv(p->H, 64);  // H <= 64 * BIN_CQ (checked above)
@@ -537,7 +568,8 @@ static cf_status bin_launch(cf_spectrum_plan *p, const double *fk, const double 
   if (dk) by_cq(std::true_type());
   else by_cq(std::false_type());
   CF_LAUNCHED();
-  hipLaunchKernelGGL(k_bin_cols, dim3((unsigned)cdiv(p->nb, 256)), b256, 0, st, p->rbuf, p->H, p->nr, p->nb, bins);
+  hipLaunchKernelGGL(k_bin_cols, dim3((unsigned)cdiv(p->nb, 64)), dim3(64 * BIN_SPLIT), 0, st, p->rbuf, p->cidx, p->H, p->nr,
+                     p->nc, p->nb, bins);
   CF_LAUNCHED();
   return CF_OK;
 }
