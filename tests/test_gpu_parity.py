@@ -229,3 +229,17 @@ def test_scale_sum_ops(cfl):
             ref = ref + al[k] * vs[k]
         assert_bitwise(host(out), ref, f"scale_sum{K}")
     assert cfl.norm_inf(dev(vs[3])) == np.max(np.abs(vs[3]))
+
+
+@pytest.mark.parametrize("N,lam", [(4, 0.2), (10, 0.0), (126, 0.2), (130, 0.0)])
+def test_energy_density_tile_edges_bitwise(cfl, O, N, lam):
+    """The energy density where its tiles (128 columns, 4 rows, 8 planes) end early or one
+    past, from a state on an odd double."""
+    print(f"case rho edges N={N} lam={lam}", flush=True)
+    x = rand_state(N, 3)
+    ref = O.energy_density(N, x, 0.9, lam, 0.44)
+    odd = torch.empty(2 * N ** 3 + 1, dtype=torch.float64, device="cuda")
+    odd[1:] = dev(x)
+    rho = torch.full((N ** 3 + 1,), float("nan"), dtype=torch.float64, device="cuda")
+    cfl.energy_density_f64(N, odd[1:], rho[1:], 0.9, lam, 0.44)
+    assert_bitwise(host(rho[1:].clone()), ref, "rho")
