@@ -49,6 +49,27 @@ __global__ void k_scale_sum(double *v0, SumArgs args, int64_t n) {  // v0 may al
   }
 }
 
+// The same for one or two vectors, a pair of elements (16 bytes; the arrays are only known to
+// start on a double) per thread. Memory-bound: N=128 (100 MB, in cache) 16.7 -> 13.7 us,
+// N=256 139 -> 133; five vectors already have enough loads in flight and lose (N=256 268 ->
+// 292).
+typedef double SumPair __attribute__((ext_vector_type(2), aligned(8)));
+template <int K>
+__global__ __launch_bounds__(256) void k_scale_sum_pairs(double *v0, SumArgs args, int64_t n) {
+  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 2;
+  if (i + 1 < n) {
+    SumPair acc = args.a[0] * *reinterpret_cast<const SumPair *>(args.v[0] + i);
+#pragma unroll
+    for (int k = 1; k < K; ++k) acc = acc + args.a[k] * *reinterpret_cast<const SumPair *>(args.v[k] + i);
+    *reinterpret_cast<SumPair *>(v0 + i) = acc;
+  } else if (i < n) {
+    double acc = args.a[0] * args.v[0][i];
+#pragma unroll
+    for (int k = 1; k < K; ++k) acc = acc + args.a[k] * args.v[k][i];
+    v0[i] = acc;
+  }
+}
+
 __global__ void k_absmax_partial(const double *__restrict__ v, int64_t n, double *__restrict__ part) {
   __shared__ double sm[256];
   double m = 0.0;
@@ -213,10 +234,13 @@ cf_status cf_scale_sum(int K, double *v0, const double *const *v, const double *
     args.a[k] = alpha[k];
   }
   dim3 g(grid_for(n, 256, 1 << 20)), b(256);
+  const dim3 pairs((unsigned)((n + 511) / 512));
   switch (K) {
+    case 1: hipLaunchKernelGGL(k_scale_sum_pairs<1>, pairs, b, 0, S(stream), v0, args, n); break;
+    case 2: hipLaunchKernelGGL(k_scale_sum_pairs<2>, pairs, b, 0, S(stream), v0, args, n); break;
 #define CF_CASE(k) \
   case k: hipLaunchKernelGGL(k_scale_sum<k>, g, b, 0, S(stream), v0, args, n); break;
-    CF_CASE(1) CF_CASE(2) CF_CASE(3) CF_CASE(4) CF_CASE(5) CF_CASE(6) CF_CASE(7)
+    CF_CASE(3) CF_CASE(4) CF_CASE(5) CF_CASE(6) CF_CASE(7)
     CF_CASE(8) CF_CASE(9) CF_CASE(10) CF_CASE(11) CF_CASE(12) CF_CASE(13) CF_CASE(14)
 #undef CF_CASE
   }

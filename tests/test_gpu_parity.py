@@ -243,3 +243,24 @@ def test_energy_density_tile_edges_bitwise(cfl, O, N, lam):
     rho = torch.full((N ** 3 + 1,), float("nan"), dtype=torch.float64, device="cuda")
     cfl.energy_density_f64(N, odd[1:], rho[1:], 0.9, lam, 0.44)
     assert_bitwise(host(rho[1:].clone()), ref, "rho")
+
+
+@pytest.mark.parametrize("K", [1, 2])
+@pytest.mark.parametrize("n", [1, 2, 511, 512, 513, 4097])
+def test_scale_sum_pairs_edges(cfl, K, n):
+    """Short sums where the pairs of elements end, on even and odd doubles and in place."""
+    rng = np.random.default_rng(n)
+    a, v = rng.standard_normal(K), rng.standard_normal((K, n))
+    ref = a[0] * v[0]
+    for k in range(1, K):
+        ref = ref + a[k] * v[k]
+    for off in (0, 1):
+        bufs = [torch.full((n + 3,), float("nan"), dtype=torch.float64, device="cuda") for _ in range(K + 1)]
+        for k in range(K):
+            bufs[k][off:off + n] = dev(v[k])
+        ins = [b[off:off + n] for b in bufs]
+        cfl.scale_sum(ins[K], ins[:K], list(a))
+        assert np.array_equal(host(ins[K].clone()), ref)
+        assert torch.isnan(bufs[K][off + n:]).all() and torch.isnan(bufs[K][:off]).all()
+        cfl.scale_sum(ins[0], ins[:K], list(a))
+        assert np.array_equal(host(ins[0].clone()), ref)
