@@ -53,10 +53,11 @@ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 // Scratch owned by a spectrum plan (cf_spectrum.hip), for library code that runs
 // with a plan: a reduction buffer of 1025 doubles and one spectrum of
-// cf_spectrum_bins(N) doubles. Calls that share a plan are ordered on one stream.
+// cf_spectrum_bins(N) doubles with three more behind it. Calls that share a plan are ordered on one stream.
 double *plan_red(cf_spectrum_plan *p);
 double *plan_bins(cf_spectrum_plan *p);
 int64_t plan_size(const cf_spectrum_plan *p);  // its lattice size N
+cf_status plan_z2d_weighted(cf_spectrum_plan *p, double *fk, const double *w, double *out, hipStream_t st);
 
 // Logical block of hardware block b of a grid of `total` blocks. The dispatcher deals
 // blocks to the 8 XCDs in turn (b -> XCD b % 8, its (b / 8)-th block); XCD x is given

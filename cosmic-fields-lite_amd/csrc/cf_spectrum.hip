@@ -46,7 +46,7 @@ struct cf_spectrum_plan {
   int32_t *foff = nullptr;       // the same for the (N/2 + 1) N rows (a'*N + b) of folded powers
   int32_t *frows = nullptr;
   double *red = nullptr;         // reduction scratch (RED_BLOCKS + 1 doubles)
-  double *bins = nullptr;        // one spectrum (nb doubles) for callers inside the library
+  double *bins = nullptr;        // one spectrum (nb doubles) and three results for callers inside the library
 };
 
 namespace cf {
@@ -350,6 +350,28 @@ static cf_status z2d_exec(cf_spectrum_plan *p, double *in, double *out, hipStrea
   return z2d_lib(p, in, out, st);
 }
 
+// Half-spectrum fk *= 2 w[s].
+__global__ void k_weight_modes(double2 *__restrict__ fk, const double *__restrict__ w, int64_t N, int64_t H) {
+  const int64_t total = N * N * H;
+  for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t c = e % H, r = e / H, b = r % N, a = r / N;
+    const int64_t as = a <= N / 2 ? a : N - a, bs = b <= N / 2 ? b : N - b;
+    const double s2 = 2.0 * w[as * as + bs * bs + c * c];
+    double2 v = fk[e];
+    v.x *= s2;
+    v.y *= s2;
+    fk[e] = v;
+  }
+}
+
+// Half spectrum fk (overwritten) times 2 w[s] -> real field.
+cf_status plan_z2d_weighted(cf_spectrum_plan *p, double *fk, const double *w, double *out, hipStream_t st) {
+  if (p->fft.N) return fft_inverse(p->fft, (const double2 *)fk, (double2 *)p->cbuf0, FftScale{w, 2.0, 0.0}, out, st);
+  hipLaunchKernelGGL(k_weight_modes, dim3(4096), dim3(256), 0, st, (double2 *)fk, w, p->N, p->H);
+  CF_LAUNCHED();
+  return z2d_lib(p, fk, out, st);
+}
+
 // Spectrum factories over s, |k| = sqrt(s)*2*pi/L (random_field.cpp:67,212-254).
 static void spectrum_table(int kind, int64_t N, double L, const double *prm, double *P) {
   const double pi = 3.14159265358979323846;
@@ -463,7 +485,7 @@ cf_status cf_spectrum_plan_create(int64_t N, cf_spectrum_plan **out) {
       hipMalloc((void **)&p->foff, ((size_t)p->nr + 1) * sizeof(int32_t)) != hipSuccess ||
       hipMalloc((void **)&p->frows, (size_t)((N / 2 + 1) * N) * sizeof(int32_t)) != hipSuccess ||
       hipMalloc((void **)&p->red, (RED_BLOCKS + 1) * sizeof(double)) != hipSuccess ||
-      hipMalloc((void **)&p->bins, (size_t)p->nb * sizeof(double)) != hipSuccess) {
+      hipMalloc((void **)&p->bins, ((size_t)p->nb + 3) * sizeof(double)) != hipSuccess) {
     set_error("cf_spectrum_plan_create(N=%lld): device allocation failed", (long long)N);
     return fail(CF_E_NOMEM);
   }

@@ -225,3 +225,59 @@ def test_config5_finite_differences(cfl, O):
     print(f"m: adjoint {gm:.12e} fd {fdm:.12e} rel {abs(fdm - gm) / abs(gm):.2e}", flush=True)
     assert max(errs) < 1e-5
     assert abs(fdm - gm) / abs(gm) < 1e-6
+
+
+@pytest.mark.parametrize("N,n_steps,ckpt", [(12, 5, 1), (12, 6, 2), (22, 7, 3), (12, 0, 3), (130, 3, 2)])
+def test_states_kept_in_place(cfl, O, N, n_steps, ckpt):
+    """Segments of every length that the buffers are taken in turn for, a size without own
+    transforms (22) and one past the tiles of the density's adjoint: the gradient equals
+    that of a chain with one segment, also when it is written over x0, and x0 is left
+    alone otherwise."""
+    import ctypes as C
+    from cfl_amd.adjoint import AdjointProblem
+    lam, m = 0.2, 1.1
+    rng = np.random.default_rng(N)
+    x0 = torch.from_numpy(0.4 * rng.standard_normal(2 * N ** 3)).cuda()
+    p = cfl.kg_params(N, float(N), m, lam, cfl.radiation(**FRW))
+
+    def run(ck, x, g):
+        prob = AdjointProblem(N, float(N), lam, cfl.radiation(**FRW), 1.0, 0.05, n_steps, ck)
+        Lo, dm = C.c_double(), C.c_double()
+        cfl.check(cfl.lib.cf_adjoint_spectrum_loss(prob.plan.h, C.byref(p), cfl._ptr(x), 1.0, 0.05, n_steps, ck,
+                                                   cfl._ptr(prob.weights), cfl._ptr(g), C.byref(Lo), C.byref(dm),
+                                                   cfl._ptr(prob.work), cfl._stream()))
+        return Lo.value, dm.value
+    one, seg, same = torch.empty_like(x0), torch.full_like(x0, float("nan")), x0.clone()
+    keep = x0.clone()
+    ref = run(max(n_steps, 1), x0, one)
+    assert run(ckpt, x0, seg) == ref and torch.equal(seg, one) and torch.equal(x0, keep)
+    assert run(ckpt, same, same) == ref and torch.equal(same, one)
+    if n_steps == 0:  # the loss alone, against torch
+        from cfl_amd.adjoint import spectral_weights
+        cosmo_o = O.Cosmo.radiation(**FRW)
+        xt = torch.tensor(host(x0), requires_grad=True)
+        W = torch.from_numpy(spectral_weights(N, float(N))[shift_sq(N)])
+        Lt = t_loss(xt, N, m, lam, O.inv_ah_sqr(N, float(N), O.cosmo_a(cosmo_o, 1.0)), W)
+        assert abs(ref[0] - Lt.item()) <= 1e-12 * abs(Lt.item())
+        assert rel(host(one), torch.autograd.grad(Lt, xt)[0].numpy()) < 1e-12
+
+
+@pytest.mark.parametrize("N", [4, 22, 126, 130])
+def test_loss_adjoint_tile_edges_vs_torch(cfl, O, N):
+    """The density's adjoint where its tiles (128 columns, 4 rows, 8 planes) end early or
+    one past, and a size without own transforms."""
+    from cfl_amd.adjoint import AdjointProblem, spectral_weights
+    lam, m, t = 0.2, 1.1, 2.0
+    cosmo_o = O.Cosmo.radiation(**FRW)
+    rng = np.random.default_rng(N)
+    x = np.concatenate([0.5 * rng.standard_normal(N ** 3), 0.3 * rng.standard_normal(N ** 3)])
+    prob = AdjointProblem(N, float(N), lam, cfl.radiation(**FRW), 1.0, 0.05, 20, 4)
+    Lg, gx, dm = prob.loss_at(torch.from_numpy(x).cuda(), m)
+    W = torch.from_numpy(spectral_weights(N, float(N))[shift_sq(N)])
+    xt = torch.tensor(x, requires_grad=True)
+    mt = torch.tensor(m, dtype=torch.float64, requires_grad=True)
+    Lt = t_loss(xt, N, mt, lam, O.inv_ah_sqr(N, float(N), O.cosmo_a(cosmo_o, t)), W)
+    gxt, gmt = torch.autograd.grad(Lt, (xt, mt))
+    assert abs(Lg - Lt.item()) <= 1e-12 * abs(Lt.item())
+    assert rel(host(gx), gxt.numpy()) < 1e-12
+    assert abs(dm - gmt.item()) <= 1e-11 * abs(gmt.item())
