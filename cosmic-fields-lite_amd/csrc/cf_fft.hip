@@ -257,9 +257,12 @@ __global__ __launch_bounds__(512) void k_fft_c2r(FftLen p, const double2 *__rest
 // First pass (along a) of the inverse of two fields: in * tab.x and in * tab.y into the two
 // fields of `out`, interleaved by column ([a][b][c][field]). A block's eight lines are four
 // columns of both fields, so the spectrum and the factors are read once and the stores
-// still fill whole lines; blocks x and x + 8 (one XCD) share the lines they read. (Separate
-// field arrays at N=384: half-line stores 0.53 ms, a block per field 0.68, two buffers and
-// one block per CU 0.66.)
+// still fill whole lines; blocks x and x + 8 (one XCD) share the lines of factors they read.
+// (Separate field arrays at N=384: half-line stores 0.53 ms, a block per field 0.68, two
+// buffers and one block per CU 0.66; here 0.50.) What bounds it: two blocks a CU, each with
+// 24 KB of reads, its stages and 49 KB of stores in sequence. The stores alone take 0.24
+// ms, without the factors it is no faster, and a third block (roots read from memory
+// instead of LDS, 96 VGPRs) spills: 0.9.
 __global__ __launch_bounds__(512) void k_fft_pair(FftLen p, const double2 *__restrict__ in,
                                                   const double2 *__restrict__ tab, double2 *__restrict__ out,
                                                   int pitch) {
@@ -274,13 +277,13 @@ __global__ __launch_bounds__(512) void k_fft_pair(FftLen p, const double2 *__res
   const int c = ct * (FFT_CW / 2) + (l >> 1);
   const bool rd = c <= p.n / 2;
   const int64_t e_stride = (int64_t)p.n * pitch;
-  const double2 *src = in + (int64_t)row * pitch + c;
+  const double2 *src = in + fft_line_index(p.n, pitch, 0, row, c);
   double2 *dst = out + 2 * ((int64_t)row * pitch + c) + f;
   const int rf = fft_fold(row, p.n);
   auto gl = [&](int e) -> double2 {
     if (!rd) return make_double2(0.0, 0.0);
     const int ef = fft_fold(e, p.n), hi = ef > rf ? ef : rf, lo = ef > rf ? rf : ef;
-    const double2 x = src[e * e_stride], t = tab[(int64_t)(hi * (hi + 1) / 2 + lo) * pitch + c];
+    const double2 x = src[e * FFT_LW], t = tab[(int64_t)(hi * (hi + 1) / 2 + lo) * pitch + c];
     const double m = f == 0 ? t.x : t.y;
     return make_double2(x.x * m, x.y * m);
   };

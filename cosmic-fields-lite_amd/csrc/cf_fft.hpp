@@ -218,13 +218,21 @@ cf_status fft_forward_fold(const FftPlan &p, const double *in, double2 *spec, do
 // Inverse: half spectrum `in` (unchanged unless it is spec) -> real N^3.
 cf_status fft_inverse(const FftPlan &p, const double2 *in, double2 *spec, const FftScale &scale, double *out,
                       hipStream_t st);
-// Inverse of two fields from one spectrum R (rows of `pitch`, a multiple of eight; only
-// read): R times tab's x and y -> out, out + N^3. tab: a row of `pitch` factors (by c) for
+// Inverse of two fields from one spectrum R (in fft_line_index's order, `pitch` a multiple of
+// eight; only read): R times tab's x and y -> out, out + N^3. tab: a row of `pitch` factors (by c) for
 // every pair a' >= b' of folded indices, row a' (a' + 1) / 2 + b' (a table over s = a'^2 +
 // b'^2 + c^2 would be an eighth of the size, but every look-up a line of its own: 0.77 ms
 // for the first pass at N=384). `spec` is scratch of 2 * N^2 * pitch entries.
 cf_status fft_inverse_pair(const FftPlan &p, const double2 *R, const double2 *tab, double2 *spec, int64_t pitch,
                            double *out, hipStream_t st);
+
+// Where fft_inverse_pair's R holds entry (a, b, c): four columns' lines along a lie together,
+// so a block of its first pass (four columns, both fields) reads one run of 64 N bytes. In
+// rows it read half a 128-byte line per element, each in another plane (N=384 522 against 495 us for the pass).
+constexpr int FFT_LW = FFT_CW / 2;
+__host__ __device__ __forceinline__ int64_t fft_line_index(int64_t N, int64_t pitch, int64_t a, int64_t b, int64_t c) {
+  return ((b * (pitch / FFT_LW) + c / FFT_LW) * N + a) * FFT_LW + c % FFT_LW;
+}
 
 // Rows of fft_inverse_pair's table.
 inline int64_t fft_pair_rows(int64_t N) { return (N / 2 + 1) * (N / 2 + 2) / 2; }

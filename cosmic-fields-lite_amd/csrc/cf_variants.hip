@@ -257,23 +257,27 @@ __global__ void k_comoving_table(int64_t pitch, double g3, double2 *__restrict__
 
 // Half spectrum of N^3 -> half spectrum of M^3 (compute_cutoff_fouriers,
 // fdm3d.cpp:105-130): low |k| modes kept, divided by (N/M)^3.
+// LINES: into fft_line_index's order of rows of pitch_out (cf_fft.hpp).
+template <bool LINES>
 __global__ void k_cutoff(int64_t N, int64_t M, const double *__restrict__ in, int64_t pitch_in,
                          double *__restrict__ out, int64_t pitch_out, double scale3) {
   const int64_t HM = M / 2 + 1, n = M * M * HM;
   for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < n; e += (int64_t)gridDim.x * blockDim.x) {
     const int64_t c = e % HM, b = (e / HM) % M, a = e / (HM * M);
     const int64_t aN = (a < M / 2) ? a : N - (M - a), bN = (b < M / 2) ? b : N - (M - b);
-    const int64_t f = (aN * N + bN) * pitch_in + c, o = (a * M + b) * pitch_out + c;
+    const int64_t f = (aN * N + bN) * pitch_in + c;
+    const int64_t o = LINES ? fft_line_index(M, pitch_out, a, b, c) : (a * M + b) * pitch_out + c;
     out[2 * o] = in[2 * f] / scale3;
     out[2 * o + 1] = in[2 * f + 1] / scale3;
   }
 }
 
 static unsigned grid_for(int64_t n);
+template <bool LINES>
 static cf_status launch_cutoff(int64_t N, int64_t M, const double *in, int64_t pitch_in, double *out,
                                int64_t pitch_out, hipStream_t st) {
   const double sd = static_cast<double>(N) / static_cast<double>(M);
-  hipLaunchKernelGGL(k_cutoff, dim3(grid_for(M * M * (M / 2 + 1))), dim3(256), 0, st, N, M, in, pitch_in, out,
+  hipLaunchKernelGGL(k_cutoff<LINES>, dim3(grid_for(M * M * (M / 2 + 1))), dim3(256), 0, st, N, M, in, pitch_in, out,
                      pitch_out, pow(sd, 3));
   CF_LAUNCHED();
   return CF_OK;
@@ -292,9 +296,9 @@ static unsigned grid_for(int64_t n) {
 struct PsiGrid {
   int64_t G = 0;
   FftPlan fft;             // fft.N != 0: own passes
-  int64_t pitch = 0;       // entries per row of R and spec
+  int64_t pitch = 0;       // entries per row of R (own passes: in fft_line_index's order) and spec
   double2 *tab = nullptr;  // transfer factors (own passes)
-  double *R = nullptr;     // comoving curvature, half spectrum (rows of `pitch`)
+  double *R = nullptr;     // comoving curvature, half spectrum
   double *spec = nullptr;  // 2 half spectra: Psi^, dPsi^
   // Psi | dPsi (2*G^3 each) at up to three times, least recently used replaced: a
   // temporally blocked step needs t, t + dt/2 and t + dt at once, and the next step
@@ -334,9 +338,8 @@ struct PsiGrid {
   }
   // R from a half spectrum without padding.
   cf_status set_R(const double *field, hipStream_t st) {
-    const size_t row = (size_t)(G / 2 + 1) * sizeof(double2);
-    CF_HIP(hipMemcpy2DAsync(R, (size_t)pitch * sizeof(double2), field, row, row, (size_t)(G * G),
-                            hipMemcpyDeviceToDevice, st));
+    if (fft.N) return launch_cutoff<true>(G, G, field, G / 2 + 1, R, pitch, st);  // every mode, over one
+    CF_HIP(hipMemcpyAsync(R, field, half() * sizeof(double), hipMemcpyDeviceToDevice, st));
     return CF_OK;
   }
   void release() {
@@ -482,7 +485,7 @@ cf_status cf_cutoff_fouriers(int64_t N, int64_t M, const double *in, double *out
   CF_REQUIRE(valid_N(N) && valid_N(M) && M <= N, "cf_cutoff_fouriers: need even 4 <= M <= N <= 2048 (N=%lld M=%lld)",
              (long long)N, (long long)M);
   CF_REQUIRE(in && out && (const void *)in != (const void *)out, "cf_cutoff_fouriers: null or aliased buffers");
-  return launch_cutoff(N, M, in, N / 2 + 1, out, M / 2 + 1, S(stream));
+  return launch_cutoff<false>(N, M, in, N / 2 + 1, out, M / 2 + 1, S(stream));
 }
 
 cf_status cf_comoving_psi_fft(int64_t G, const double *R_fft, double *psi_fft, double *dpsi_fft, double factor,
@@ -531,7 +534,9 @@ cf_status cf_variant_create(const cf_kg_params *p, int kind, double f_a, int64_t
     rc = v->grid.init(M);
     if (rc == CF_OK) rc = v->full.init(N);
     if (rc == CF_OK) rc = v->full.set_R(field, st);
-    if (rc == CF_OK) rc = launch_cutoff(N, M, v->full.R, v->full.pitch, v->grid.R, v->grid.pitch, st);
+    if (rc == CF_OK)
+      rc = v->grid.fft.N ? launch_cutoff<true>(N, M, field, N / 2 + 1, v->grid.R, v->grid.pitch, st)
+                         : launch_cutoff<false>(N, M, field, N / 2 + 1, v->grid.R, v->grid.pitch, st);
     v->full_ready = (rc == CF_OK);
   }
   if (rc == CF_OK && hipStreamSynchronize(st) != hipSuccess) {

@@ -219,3 +219,18 @@ def test_rk4_tb_comoving_equals_stage_kernels(cfl, O, name, kind, N, M, steps):
     close(host(xb), ov.rk4_run(x0.copy(), t0, dt, steps, k0=1), f"{name} tb vs oracle")
     v.close()
     v2.close()
+
+
+@pytest.mark.parametrize("name,kind,N,M", [("comoving", 3, 22, 0), ("comoving", 3, 18, 0), ("approx", 4, 44, 4),
+                                           ("approx", 4, 44, 22), ("approx", 4, 20, 10)])
+def test_stored_spectrum_orders(cfl, O, name, kind, N, M):
+    """The comoving spectrum is kept in the order its transform reads: with and without own
+    transforms on the full and the coarse grid (22 and 44 have a factor of eleven)."""
+    print(f"case spectrum order {name} N={N} M={M}", flush=True)
+    v, ov = setup(cfl, O, kind, N, M=M)
+    x0 = rand_state(N, 14, 0.3)
+    x = dev(x0)
+    v.rk4_run_tb(x, 1.0, 0, 2, 0.05)
+    close(host(x), ov.rk4_run(x0.copy(), 1.0, 0.05, 2), f"{name} tb vs oracle")
+    close(host(v.energy_density(x, 1.1)), ov.energy_density(host(x), 1.1), f"{name} rho")
+    v.close()
