@@ -82,9 +82,9 @@ __global__ __launch_bounds__(SH::NT) __attribute__((amdgpu_waves_per_eu(WAVES, W
 // less time per plane.
 //
 // t1 and tau are the time of a plane iteration in us with one block on a CU and, per
-// block, with `resident` blocks, the CU full; bw the rate in bytes per us at which
-// launches that stream through HBM pass their loads (halo and warm-up included) and
-// stores. Measured over N = 32 .. 512 on 256 CUs; see tb_cost.
+// block, with `resident` blocks, the CU full (states in cache); bw the rate in bytes per us
+// at which launches that stream through HBM pass their loads (halo and warm-up included)
+// and stores. Measured over N = 32 .. 512 on 256 CUs; see tb_cost.
 struct TbShapeInfo {
   int rb, rc, resident;
   double t1, tau, bw;
@@ -107,11 +107,11 @@ static const double tb_load_bytes[7] = {16.0, 16.0, 16.0, 24.0, 16.0, 64.0, 22.0
 
 static const std::vector<TbShapeInfo> &tb_shapes(int family) {
   static const std::vector<TbShapeInfo> t[7] = {
-      {{12, 20, 8, 0.68, 0.26, 4.9e6}, {14, 36, 4, 0.70, 0.47, 5.0e6}, {28, 36, 2, 1.00, 0.92, 5.1e6},
-       {30, 68, 1, 2.00, 2.00, 5.55e6}},
-      {{14, 36, 2, 0.75, 0.58, 4.6e6}, {28, 36, 1, 1.22, 1.22, 4.4e6}, {22, 68, 1, 1.73, 1.73, 5.0e6}},
-      {{12, 20, 8, 0.60, 0.18, 3.9e6}, {14, 36, 4, 0.65, 0.39, 4.6e6}, {28, 36, 2, 0.84, 0.78, 4.65e6},
-       {30, 68, 1, 1.65, 1.65, 5.2e6}, {15, 132, 1, 1.55, 1.55, 5.8e6}},
+      {{12, 20, 8, 0.68, 0.26, 4.9e6}, {14, 36, 4, 0.70, 0.47, 5.0e6}, {28, 36, 2, 1.00, 0.92, 5.3e6},
+       {30, 68, 1, 2.00, 2.00, 5.57e6}},
+      {{14, 36, 2, 0.75, 0.58, 4.6e6}, {28, 36, 1, 1.22, 1.22, 4.35e6}, {22, 68, 1, 1.73, 1.73, 5.1e6}},
+      {{12, 20, 8, 0.60, 0.18, 3.9e6}, {14, 36, 4, 0.65, 0.39, 4.7e6}, {28, 36, 2, 0.84, 0.78, 4.7e6},
+       {30, 68, 1, 1.65, 1.65, 5.15e6}, {15, 132, 1, 1.50, 1.50, 5.85e6}},
       {{14, 36, 2, 0.82, 0.68, 5.3e6}, {28, 36, 1, 1.44, 1.44, 5.1e6}, {22, 68, 1, 1.99, 1.99, 5.5e6}},
       {{14, 36, 2, 1.22, 1.13, 5.0e6}, {28, 36, 1, 2.29, 2.29, 5.0e6}, {22, 68, 1, 3.40, 3.40, 5.2e6}},
       {{14, 36, 2, 1.25, 1.09, 6.1e6}, {28, 36, 1, 2.28, 2.28, 5.9e6}},
@@ -155,27 +155,36 @@ static TbGeom tb_geom(int family, int shape, int64_t N, int A, int64_t a_lo, int
   return g;
 }
 
-// Modelled time of a launch in us: the larger of
-//   the launch itself and the busiest CU's plane iterations: its n = ceil(blocks / CUs)
-//   blocks run `resident` at a time, A + 4 iterations each at tau per block (t1 when one
-//   runs alone), of which the two that only load and the two without k3 and k4 cost two;
-//   the bytes it passes: the loads of every region and iteration and the stores, at bw
-//   (60% more while all of it fits the 256 MB cache). Beyond it blocks of long chunks
-//   drift apart and find less of their neighbours' planes in L2: 5% per 100 planes.
-// Few chunks leave CUs idle, many repeat warm-up planes; small regions repeat halos.
-// Within 4% of the best of 6 to 12 measured (shape, chunk) pairs at each of N = 32, 64,
-// 96, 128, 160, 200, 250, 300, 384, 512 and storage form, in half of them the best (the
-// variants, to N=384: mostly the best, within 11%).
+// Modelled time of a launch in us. Few chunks leave CUs idle, many repeat warm-up planes;
+// small regions repeat halos. A block takes A + 4 iterations, of which the two that only
+// load and the two without k3 and k4 cost two.
+//   While all of it fits the 256 MB cache: the larger of the busiest CU's iterations (its n
+//   = ceil(blocks / CUs) blocks, `resident` at a time) and the bytes passed at 1.6 bw.
+//   Beyond: rounds of CUs * resident blocks, each the larger of its iterations, at 0.7 of
+//   the above (what is left of them when the blocks of a round run against each other and
+//   HBM), and its bytes at bw; a last round that fills a part of the chip lies by that part
+//   between the two. (With the launch's bytes over bw instead, launches a little over a
+//   whole number of rounds were picked: N=300, FP64, 420 blocks 212 us, 240 blocks 188.)
+// Of the (shape, chunk) pairs measured at 17 sizes, N = 32 .. 512, and every storage form
+// and variant, 6 to 30 each, it picks one within 0.4% of the fastest on average, 8% at worst.
 static double tb_cost(int family, const TbShapeInfo &s, const TbGeom &g, int cus) {
-  const int64_t n = cdiv(g.total, cus), full = n / s.resident, rest = n % s.resident;
-  const double one = std::max(s.t1, (double)rest * s.tau);
-  const double cu = 1.8 + (double)(g.A + 2) * ((double)full * s.resident * s.tau + (rest ? one : 0.0));
+  const double lb = tb_load_bytes[family], launch = 1.8, it = (double)(g.A + 2);
   const double sites = (double)g.N * (double)g.N * (double)(g.a_hi - g.a_lo);
-  const double lb = tb_load_bytes[family];
-  const bool cached = (lb + 16.0) * sites <= 256e6;
-  const double drift = cached ? 1.0 : 1.0 + 5e-4 * (double)g.A;
-  const double loads = lb * (double)g.ntb * g.ntc * g.n_ac * s.rb * s.rc * (double)(g.A + 2 * TBH) * drift;
-  return std::max(cu, (loads + 16.0 * sites) / (cached ? 1.6 * s.bw : s.bw));
+  const double loads = lb * (double)g.ntb * g.ntc * g.n_ac * s.rb * s.rc * (double)(g.A + 2 * TBH);
+  const double bytes = loads + 16.0 * sites;
+  if ((lb + 16.0) * sites <= 256e6) {
+    const int64_t n = cdiv(g.total, cus), full = n / s.resident, rest = n % s.resident;
+    const double last = rest ? std::max(s.t1, (double)rest * s.tau) : 0.0;
+    return std::max(launch + it * ((double)full * s.resident * s.tau + last), bytes / (1.6 * s.bw));
+  }
+  const int64_t slots = (int64_t)cus * s.resident, full = g.total / slots, rest = g.total % slots;
+  const double round = std::max(0.7 * s.resident * s.tau * it, bytes / g.total * (double)slots / s.bw);
+  double t = launch + (double)full * round;
+  if (rest) {
+    const double least = 0.7 * std::max(s.t1, (double)cdiv(rest, cus) * s.tau) * it;
+    t += least + std::max(round - least, 0.0) * (double)rest / (double)slots;
+  }
+  return t;
 }
 
 // The cheapest (shape, chunk) of a launch, or the cheapest shape for a given chunk. With
