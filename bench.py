@@ -231,7 +231,8 @@ def ensemble_workload(args):
     ens.init_grf(seeds, cfl.CF_SPEC_GAUSS, (0.5,), 0.5)
     tuned_grid = ens.tune(dt, reps=3)
     plan = {n: ens.get_plan(n)[0] for n in (64, 96, 128)}
-    shapes = {cfl.CF_ENS_REGION_24X40: "24x40", cfl.CF_ENS_REGION_32X32: "32x32", cfl.CF_ENS_REGION_28X36: "28x36"}
+    shapes = {cfl.CF_ENS_REGION_24X40: "24x40", cfl.CF_ENS_REGION_32X32: "32x32", cfl.CF_ENS_REGION_28X36: "28x36",
+              cfl.CF_ENS_REGION_15X68: "15x68"}
     regions = {n: shapes[ens.get_region(n)] for n in (64, 96, 128)}
     # capture + first launch outside the timed region (the graph is reused)
     ens.run(t0, 0, steps, dt, use_graph=True)
@@ -426,8 +427,8 @@ def adjoint_workload(args):
 def pacing_workload(args):
     """The single-precision-stencil step (f32s) of the N=512 FRW workload at each pace of
     --paces and at the tuner's pick, --steps timed steps per pace after 4 untimed ones,
-    two passes over the list. Paced and unpaced launches are different kernels
-    (k_rk4_tb_sa<LAM, true, ...> / <LAM, false, ...>), so a profiler separates them."""
+    two passes over the list. Paced and unpaced launches are different kernels (the last
+    template argument of k_rk4_tb<2, LAM, ...>), so a profiler separates them."""
     import torch
     import cfl_amd as cfl
     N, L, dt, t0 = args.n, float(args.n), 0.05, 1.0

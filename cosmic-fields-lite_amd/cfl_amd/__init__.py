@@ -12,7 +12,7 @@ import numpy as np
 import torch
 
 from . import _lib
-from ._lib import (CF_ENS_GRID_FLAT, CF_ENS_REGION_24X40, CF_ENS_REGION_28X36, CF_ENS_REGION_32X32, CF_PREC_F32C, CF_PREC_F32S, CF_PREC_F64, CF_SPEC_DERIV_POWER_CUTOFF, CF_SPEC_GAUSS,  # noqa: F401
+from ._lib import (CF_ENS_GRID_FLAT, CF_ENS_REGION_15X68, CF_ENS_REGION_24X40, CF_ENS_REGION_28X36, CF_ENS_REGION_32X32, CF_PREC_F32C, CF_PREC_F32S, CF_PREC_F64, CF_SPEC_DERIV_POWER_CUTOFF, CF_SPEC_GAUSS,  # noqa: F401
                    CF_SPEC_KM3_GAUSS, CF_SPEC_POWER_CUTOFF, CF_SPEC_SCALE_INV,
                    CF_VAR_APPROX_COMOVING_CURVATURE, CF_VAR_COMOVING_CURVATURE, CF_VAR_FIXED_CURVATURE,
                    CF_VAR_SQRT_POTENTIAL, CfError, Cosmology, KGParams, check)
@@ -248,7 +248,7 @@ def join_f64(hi, lo, stream=None):
 
 # ---------------------------------------------------------------- spectra
 class SpectrumPlan:
-    """hipFFT plans + bin table for an N^3 lattice (cufftWrapperNoBatching analogue)."""
+    """Transform plan and bin tables of an N^3 lattice (cufftWrapperNoBatching analogue)."""
 
     def __init__(self, N):
         self.N = int(N)

@@ -28,6 +28,7 @@ CF_ENS_GRID_FLAT = -1  # ensemble plan: one block per work unit
 CF_ENS_REGION_32X32 = 0  # ensemble block region (b rows x c columns): 28 x 28 tiles
 CF_ENS_REGION_24X40 = 1  # 20 x 36 tiles
 CF_ENS_REGION_28X36 = 2  # 24 x 32 tiles
+CF_ENS_REGION_15X68 = 3  # 11 x 64 tiles
 
 CF_VAR_FIXED_CURVATURE = 1
 CF_VAR_SQRT_POTENTIAL = 2

@@ -7,7 +7,7 @@
 // the host balanced by longest-processing-time-first over their iteration counts
 // (so the mix of N = 64 / 96 / 128 lattices finishes together), or one block per
 // unit, longest first. No atomics and no inter-block communication. The block's
-// region shape (32 x 32, 24 x 40 or 28 x 36 sites, so 28 x 28, 20 x 36 or 24 x 32 tiles)
+// region shape (32 x 32, 24 x 40, 28 x 36 or 15 x 68 sites, so 28 x 28, 20 x 36, 24 x 32 or 11 x 64 tiles)
 // and the chunk are chosen per lattice size; the autotuner times the candidates.
 //
 // The step scalars a(t), H(t) of every stage live in a device table, so the
@@ -46,9 +46,11 @@ struct EnsUnit {
 // Region shapes of a unit's block, by CF_ENS_REGION_*. With float forces blocks are 512
 // threads with two columns each, two blocks per CU; with FP64 arithmetic 1024 threads with
 // one column each (two columns of FP64 and the unit's descriptors exceed 128 VGPRs: 30
-// spilled).
-constexpr int ENS_REGIONS = 3;
-constexpr int ENS_RB[ENS_REGIONS] = {32, 24, 28}, ENS_RC[ENS_REGIONS] = {32, 40, 36};
+// spilled). The 11 x 64 tiles load as many sites per output site as the 24 x 32 ones but
+// pass 8 bytes of 128-byte lines per output float instead of 12 (float forces, us a step:
+// four each of N = 64, 96 and 128 114 -> 107, eight of N=128 143 -> 127).
+constexpr int ENS_REGIONS = 4;
+constexpr int ENS_RB[ENS_REGIONS] = {32, 24, 28, 15}, ENS_RC[ENS_REGIONS] = {32, 40, 36, 68};
 template <int MODE, int REGION>
 using EnsShape = std::conditional_t<MODE != TB_F32S, TbShape<ENS_RB[REGION], ENS_RC[REGION], 1, 1024>,
                                     TbShape<ENS_RB[REGION], ENS_RC[REGION], 2, 512>>;
@@ -58,7 +60,7 @@ constexpr int ens_threads() {
 }
 template <int MODE>
 constexpr int ens_lds() {
-  return std::max({EnsShape<MODE, 0>::LDS, EnsShape<MODE, 1>::LDS, EnsShape<MODE, 2>::LDS});
+  return std::max({EnsShape<MODE, 0>::LDS, EnsShape<MODE, 1>::LDS, EnsShape<MODE, 2>::LDS, EnsShape<MODE, 3>::LDS});
 }
 inline int ens_tile_b(int region, int64_t N) {
   const int t = ENS_RB[region] - 2 * TBH;
@@ -156,6 +158,8 @@ __device__ __forceinline__ void ens_unit_any(void *smem, const EnsReal *__restri
   const EnsUnit e = wave_uniform(unit);
   if (e.region == CF_ENS_REGION_28X36)
     ens_unit<MODE, LAM, EnsShape<MODE, CF_ENS_REGION_28X36>, PACE>(smem, reals, e, sc, parity, c_m, lam, dt, pace);
+  else if (e.region == CF_ENS_REGION_15X68)
+    ens_unit<MODE, LAM, EnsShape<MODE, CF_ENS_REGION_15X68>, PACE>(smem, reals, e, sc, parity, c_m, lam, dt, pace);
   else if (e.region == CF_ENS_REGION_24X40)
     ens_unit<MODE, LAM, EnsShape<MODE, CF_ENS_REGION_24X40>, PACE>(smem, reals, e, sc, parity, c_m, lam, dt, pace);
   else
@@ -670,7 +674,7 @@ cf_status cf_ensemble_tune(cf_ensemble *e, double dt, int reps, int *grid_out) {
       std::vector<int> chunks;
       for (int A : {(int)N, (int)(N + 1) / 2, 256, 128, 64, 32, 16, 8})
         if (A <= N && std::find(chunks.begin(), chunks.end(), A) == chunks.end()) chunks.push_back(A);
-      for (int reg : {CF_ENS_REGION_28X36, CF_ENS_REGION_32X32})
+      for (int reg : {CF_ENS_REGION_28X36, CF_ENS_REGION_15X68, CF_ENS_REGION_32X32})
         for (int A : chunks) {
           if (A == was_a && reg == was_r) continue;
           e->chunk[N] = A;

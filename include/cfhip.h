@@ -274,12 +274,13 @@ cf_status cf_ensemble_set_plan(cf_ensemble *e, int64_t N, int chunk, int grid);
 cf_status cf_ensemble_get_plan(const cf_ensemble *e, int64_t N, int *chunk, int *grid);
 /* Region shape of the blocks that advance lattices of size N (rows along b x columns
  * along c, halo of two sites included): CF_ENS_REGION_32X32 (28 x 28 output tiles, the
- * default), CF_ENS_REGION_24X40 (20 x 36) or CF_ENS_REGION_28X36 (24 x 32 tiles, which
- * divide N = 96 and whose rows fall on 128-byte lines for N = 64, 96 and 128). Same bits
- * in all of them. */
+ * default), CF_ENS_REGION_24X40 (20 x 36), CF_ENS_REGION_28X36 (24 x 32 tiles, which
+ * divide N = 96 and whose rows fall on 128-byte lines for N = 64, 96 and 128) or
+ * CF_ENS_REGION_15X68 (11 x 64 tiles). Same bits in all of them. */
 #define CF_ENS_REGION_32X32 0
 #define CF_ENS_REGION_24X40 1
 #define CF_ENS_REGION_28X36 2
+#define CF_ENS_REGION_15X68 3
 cf_status cf_ensemble_set_region(cf_ensemble *e, int64_t N, int region);
 cf_status cf_ensemble_get_region(const cf_ensemble *e, int64_t N, int *region);
 /* Autotuner: times candidate grids (persistent and flat), then per N candidate
@@ -410,9 +411,10 @@ cf_status cf_wkb_tables_host(int64_t N, double L, double m, double a1, double H1
                              double *cos_host, double *sin_host, double *sqrt_omega_host, double *phase_host);
 
 /* ---------------------------------------------------------------- FFT and spectra
- * A spectrum plan owns the hipFFT D2Z/Z2D plans of an N^3 lattice with one shared
- * work area (cufftWrapperNoBatching, src/cuda_wrapper.cu:202-255), scratch buffers,
- * and the bin table used by the deterministic binning kernels. */
+ * A spectrum plan (cufftWrapperNoBatching, src/cuda_wrapper.cu:202-255) owns the tables of
+ * the library's own transform passes, or hipFFT D2Z/Z2D plans with one shared work area
+ * where N has a prime factor above 7; scratch buffers; and the bin tables used by the
+ * deterministic binning kernels. */
 cf_status cf_spectrum_plan_create(int64_t N, cf_spectrum_plan **plan);
 cf_status cf_spectrum_plan_destroy(cf_spectrum_plan *plan);
 int64_t cf_spectrum_bins(int64_t N); /* 3*(N/2)^2 + 1 */

@@ -114,3 +114,30 @@ def test_variant_step_equals_stage_kernels(cfl, O, kind, N, chunk):
     v.rk4_step_tb(y, z, 1.05, 0.05, chunk=chunk)
     assert torch.equal(z, ref)
     v.close()
+
+
+@pytest.mark.parametrize("prec,grid", [(0, -1), (1, -1), (2, 5), (2, -1)])
+def test_ensemble_15x68_keeps_bits(cfl, prec, grid):
+    """11 x 64 tiles: a lattice inside one tile, one of 64 columns, one just past a tile."""
+    print(f"case ensemble 15x68 prec={prec} grid={grid}", flush=True)
+    Ns = [10, 64, 66]
+    ens = cfl.Ensemble(Ns, [float(n) for n in Ns], 1.0, 0.1, cfl.radiation(**FRW), prec)
+    ens.init_grf([1, 2, 3], cfl.CF_SPEC_GAUSS, (0.25,), 1.0)
+    start = [ens.state(r) for r in range(len(Ns))]
+    for n in Ns:
+        ens.set_region(n, cfl.CF_ENS_REGION_15X68)
+        assert ens.get_region(n) == cfl.CF_ENS_REGION_15X68
+    ens.set_plan(66, 13, grid)
+    ens.run(1.0, 0, 3, 0.05)
+    for r, n in enumerate(Ns):
+        p = cfl.kg_params(n, float(n), 1.0, 0.1, cfl.radiation(**FRW))
+        if prec == 0:
+            x = start[r].clone()
+            cfl.rk4_run_tb_f64(p, x, 1.0, 0, 3, 0.05, cfl.alloc_tb_work(n))
+        else:
+            hi, lo = cfl.split_f64(start[r])
+            run = cfl.rk4_run_tb_f32c if prec == 1 else cfl.rk4_run_tb_f32s
+            run(p, hi, lo, 1.0, 0, 3, 0.05, cfl.alloc_tb_work(n, prec))
+            x = cfl.join_f64(hi, lo)
+        torch.cuda.synchronize()
+        assert torch.equal(ens.state(r), x), f"realisation {r}"
