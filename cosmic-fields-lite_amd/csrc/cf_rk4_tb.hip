@@ -114,8 +114,8 @@ static const std::vector<TbShapeInfo> &tb_shapes(int family) {
        {30, 68, 1, 1.65, 1.65, 5.15e6}, {15, 132, 1, 1.50, 1.50, 5.85e6}},
       {{14, 36, 2, 0.82, 0.68, 5.3e6}, {28, 36, 1, 1.44, 1.44, 5.1e6}, {22, 68, 1, 1.99, 1.99, 5.5e6}},
       {{14, 36, 2, 1.22, 1.13, 5.0e6}, {28, 36, 1, 2.29, 2.29, 5.0e6}, {22, 68, 1, 3.40, 3.40, 5.2e6}},
-      {{14, 36, 2, 1.25, 1.09, 6.1e6}, {28, 36, 1, 2.28, 2.28, 5.9e6}},
-      {{14, 36, 2, 1.05, 0.85, 4.0e6}, {28, 36, 1, 1.77, 1.77, 3.8e6}},
+      {{14, 36, 2, 1.25, 1.09, 6.1e6}, {28, 36, 1, 2.20, 2.20, 6.0e6}},
+      {{14, 36, 2, 1.05, 0.85, 4.0e6}, {28, 36, 1, 1.70, 1.70, 3.85e6}},
   };
   return t[family];
 }
@@ -380,16 +380,21 @@ static cf_status tb_check(const cf_kg_params *p) {
 
 // The variants' kernels. 22 x 68 regions of two columns per thread for those whose site
 // factors fit the registers so (168 of them; fixed curvature, N=300: 296 -> 230 us a step,
-// N=256: 173 -> 154); the comoving ones would spill a hundred.
+// N=256: 173 -> 154); the comoving ones would spill a hundred and take two columns over 28 x
+// 36 regions, 512 threads of up to 256 registers (one column of 1024 threads: N=64 11.8
+// against 10.9 us, coarse grid 10.8 against 9.3, N=128 40.4 against 38.1, N=384 1051 against
+// 1039; for the others at N=128 one column is the faster, 23.1 against 24.0).
 template <int VAR>
 static void tb_launch_var(const TbGeom &g, const TbStep &k, const double *xin, double *xout, const double *psi,
                           const TbPsi &cp, hipStream_t st) {
   const dim3 grid((unsigned)g.total);
   if (g.shape == 0) {
     hipLaunchKernelGGL((k_rk4_tb_var<VAR, TbC14x36, 4>), grid, dim3(TbC14x36::NT), 0, st, g, k, xin, xout, psi, cp);
+  } else if constexpr (VAR == TB_COMOVING || VAR == TB_APPROX_COMOVING) {
+    hipLaunchKernelGGL((k_rk4_tb_var<VAR, TbS28x36, 2>), grid, dim3(TbS28x36::NT), 0, st, g, k, xin, xout, psi, cp);
   } else if (g.shape == 1) {
     hipLaunchKernelGGL((k_rk4_tb_var<VAR, TbC28x36, 4>), grid, dim3(TbC28x36::NT), 0, st, g, k, xin, xout, psi, cp);
-  } else if constexpr (VAR == TB_FIXED_CURVATURE || VAR == TB_SQRT_POTENTIAL) {
+  } else {
     hipLaunchKernelGGL((k_rk4_tb_var<VAR, TbC22x68, 3>), grid, dim3(TbC22x68::NT), 0, st, g, k, xin, xout, psi, cp);
   }
 }
