@@ -57,12 +57,11 @@ KERNEL_NAMES = {"f64": "cf::k_march<double, 1, S, false> (4 stage kernels)",
                 "tb_f32c": "cf::k_rk4_tb<1, false, ...>",
                 "tb_f32s": "cf::k_rk4_tb<2, false, ...>"}
 TRAFFIC_PROFILE = os.path.join(ROOT, "profiles", "rk4_tb_N512_pmc_traffic.md")
-# What bounds each path's kernel at N=512, from the committed PMC summaries: the FP32-comp
-# blocked kernel issues VALU 76% of its cycles (float <-> double conversions on top of the
-# FP64 arithmetic); the FP64 blocked kernel runs as fast with its arithmetic cut to a
-# skeleton, so its time is the memory traffic including the halo re-reads.
-LIMITER = {"tb_f32c": "vector-ALU issue", "tb_f64": "memory: HBM + L2 misses on halo re-reads",
-           "tb_f32s": "memory: halo-inclusive plane loads at the paced lock-step (L2 + HBM)",
+# What bounds each path's kernel at N=512, from the committed PMC summaries: the blocked
+# kernels move the state and part of their halos at what a plain copy reaches; the
+# FP32-comp one's float <-> double conversions keep the vector unit busy beside that.
+LIMITER = {"tb_f32c": "memory: HBM, beside vector-ALU issue", "tb_f64": "memory: HBM with halo re-reads",
+           "tb_f32s": "memory: HBM with halo re-reads",
            "f32c": "hbm", "f64": "hbm"}
 
 
