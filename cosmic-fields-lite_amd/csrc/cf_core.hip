@@ -56,13 +56,15 @@ __global__ void k_scale_sum(double *v0, SumArgs args, int64_t n) {  // v0 may al
 typedef double SumPair __attribute__((ext_vector_type(2), aligned(8)));
 template <int K>
 __global__ __launch_bounds__(256) void k_scale_sum_pairs(double *v0, SumArgs args, int64_t n) {
-  const int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 2;
-  if (i + 1 < n) {
+  const int64_t stride = (int64_t)gridDim.x * 512;
+  int64_t i = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 2;
+  for (; i + 1 < n; i += stride) {
     SumPair acc = args.a[0] * *reinterpret_cast<const SumPair *>(args.v[0] + i);
 #pragma unroll
     for (int k = 1; k < K; ++k) acc = acc + args.a[k] * *reinterpret_cast<const SumPair *>(args.v[k] + i);
     *reinterpret_cast<SumPair *>(v0 + i) = acc;
-  } else if (i < n) {
+  }
+  if (i < n) {  // the last element of an odd count
     double acc = args.a[0] * args.v[0][i];
 #pragma unroll
     for (int k = 1; k < K; ++k) acc = acc + args.a[k] * args.v[k][i];
@@ -234,7 +236,7 @@ cf_status cf_scale_sum(int K, double *v0, const double *const *v, const double *
     args.a[k] = alpha[k];
   }
   dim3 g(grid_for(n, 256, 1 << 20)), b(256);
-  const dim3 pairs((unsigned)((n + 511) / 512));
+  const dim3 pairs(grid_for(n, 512, 1 << 22));  // a launch holds fewer than 2^32 threads
   switch (K) {
     case 1: hipLaunchKernelGGL(k_scale_sum_pairs<1>, pairs, b, 0, S(stream), v0, args, n); break;
     case 2: hipLaunchKernelGGL(k_scale_sum_pairs<2>, pairs, b, 0, S(stream), v0, args, n); break;

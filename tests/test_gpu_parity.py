@@ -264,3 +264,19 @@ def test_scale_sum_pairs_edges(cfl, K, n):
         assert torch.isnan(bufs[K][off + n:]).all() and torch.isnan(bufs[K][:off]).all()
         cfl.scale_sum(ins[0], ins[:K], list(a))
         assert np.array_equal(host(ins[0].clone()), ref)
+
+
+def test_scale_sum_above_one_launch(cfl):
+    """A vector that needs more pairs than a launch can hold threads (2^32)."""
+    n = 2 ** 33 + 1025
+    if torch.cuda.mem_get_info()[0] < 8 * n + 2 ** 32:
+        pytest.skip("needs 70 GB of free device memory")
+    print(f"case scale_sum n={n}", flush=True)
+    v = torch.ones(n, dtype=torch.float64, device="cuda")
+    v[-1] = 3.0
+    cfl.scale_sum(v, [v], [2.0])
+    ends = [v[i:i + 1024].clone() for i in (0, 2 ** 31 - 512, 2 ** 32 - 512, 2 ** 33 - 512)]
+    last = v[-1].item()
+    del v
+    torch.cuda.empty_cache()
+    assert all((e == 2.0).all() for e in ends) and last == 6.0
