@@ -24,6 +24,9 @@
 // What bounds it: memory. One pass over the half spectrum reads and writes it once; the
 // library's passes along a and b took 0.70 and 0.78 ms at N=384 for two fields (1.8 GB
 // of traffic each, 2.3-2.6 TB/s).
+//
+// Error against extended precision, N = 32 .. 256: 2.3e-16 to 3.5e-16 relative (2-norm) in
+// either direction; the library's 2.8e-16 to 6.3e-16, the larger at every size measured.
 #pragma once
 
 #include "cf_common.hpp"
