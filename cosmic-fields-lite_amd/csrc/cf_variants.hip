@@ -257,7 +257,9 @@ __global__ void k_comoving_table(int64_t pitch, double g3, double2 *__restrict__
 
 // Half spectrum of N^3 -> half spectrum of M^3 (compute_cutoff_fouriers,
 // fdm3d.cpp:105-130): low |k| modes kept, divided by (N/M)^3.
-// LINES: into fft_line_index's order of rows of pitch_out (cf_fft.hpp).
+// LINES: into fft_line_index's order of rows of pitch_out (cf_fft.hpp), with the mode s = 0
+// cleared: it carries no Psi, whatever it holds, and the transfer's factor of zero would
+// not clear an infinity or a NaN.
 template <bool LINES>
 __global__ void k_cutoff(int64_t N, int64_t M, const double *__restrict__ in, int64_t pitch_in,
                          double *__restrict__ out, int64_t pitch_out, double scale3) {
@@ -267,8 +269,9 @@ __global__ void k_cutoff(int64_t N, int64_t M, const double *__restrict__ in, in
     const int64_t aN = (a < M / 2) ? a : N - (M - a), bN = (b < M / 2) ? b : N - (M - b);
     const int64_t f = (aN * N + bN) * pitch_in + c;
     const int64_t o = LINES ? fft_line_index(M, pitch_out, a, b, c) : (a * M + b) * pitch_out + c;
-    out[2 * o] = in[2 * f] / scale3;
-    out[2 * o + 1] = in[2 * f + 1] / scale3;
+    const bool clear = LINES && e == 0;
+    out[2 * o] = clear ? 0.0 : in[2 * f] / scale3;
+    out[2 * o + 1] = clear ? 0.0 : in[2 * f + 1] / scale3;
   }
 }
 

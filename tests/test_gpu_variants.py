@@ -234,3 +234,24 @@ def test_stored_spectrum_orders(cfl, O, name, kind, N, M):
     close(host(x), ov.rk4_run(x0.copy(), 1.0, 0.05, 2), f"{name} tb vs oracle")
     close(host(v.energy_density(x, 1.1)), ov.energy_density(host(x), 1.1), f"{name} rho")
     v.close()
+
+
+@pytest.mark.parametrize("kind,N,M", [(3, 16, 0), (3, 22, 0), (4, 32, 16), (4, 44, 22)])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_zero_mode_of_the_curvature_is_not_read(cfl, kind, N, M, bad):
+    """Psi has no k = 0 mode, whatever the curvature's spectrum holds there (a spectrum that
+    diverges at k = 0 leaves an infinity or a NaN), with own transforms and with hipFFT."""
+    print(f"case zero mode kind={kind} N={N} M={M} bad={bad}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(9)
+    R = 1e-2 * torch.randn(2 * N * N * (N // 2 + 1), dtype=torch.float64, device="cuda", generator=g)
+    R[:2] = 0.0
+    p = cfl.kg_params(N, float(N), 1.0, 0.0, cfl.radiation(a1=1.0, H1=0.5, t1=1.0))
+    want = cfl.Variant(p, kind, R, M=M)
+    R[:2] = bad
+    got = cfl.Variant(p, kind, R, M=M)
+    for w, h in zip(want.psi(1.1), got.psi(1.1)):
+        assert torch.isfinite(w).all() and torch.equal(w, h)
+    x = dev(rand_state(N, 15, 0.3))
+    assert torch.equal(want.energy_density(x, 1.1), got.energy_density(x, 1.1))
+    want.close()
+    got.close()
