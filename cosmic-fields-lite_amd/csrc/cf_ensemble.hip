@@ -3,12 +3,12 @@
 // All realisations of an ensemble take their RK4 steps in one kernel per step
 // over a table of work units (one output tile of one lattice over a chunk of
 // a-planes, the unit of the temporally blocked step, cf_tb_body.hpp). Two launch
-// forms: a fixed grid of blocks, each running a list of units that
-// the host balanced by longest-processing-time-first over their iteration counts
-// (so the mix of N = 64 / 96 / 128 lattices finishes together), or one block per
-// unit, longest first. No atomics and no inter-block communication. The block's
-// region shape (32 x 32, 24 x 40, 28 x 36 or 15 x 68 sites, so 28 x 28, 20 x 36, 24 x 32 or 11 x 64 tiles)
-// and the chunk are chosen per lattice size; the autotuner times the candidates.
+// forms: a fixed grid of blocks, each running a list of units that the host balanced by
+// longest-processing-time-first over their iteration counts (so the mix of N = 64 / 96 /
+// 128 lattices finishes together), or one block per unit, longest first. No atomics and no inter-block communication. The block's
+// region shape (32 x 32, 24 x 40, 28 x 36 or 15 x 68 sites, so 28 x 28, 20 x 36, 24 x 32
+// or 11 x 64 tiles; ens_shape) and the chunk are chosen per lattice size; the autotuner
+// times the candidates.
 //
 // The step scalars a(t), H(t) of every stage live in a device table, so the
 // kernels of a whole run can be captured once into a hipGraph and replayed
@@ -39,7 +39,7 @@ struct EnsReal {
 struct EnsUnit {
   int32_t real;
   int32_t T, Tc;   // output tile edges along b and c
-  int32_t region;  // CF_ENS_REGION_*: the block's region shape
+  int32_t region;  // the block's region shape (index into ENS_RB)
   int64_t b0, c0, a0, a1;
 };
 
@@ -61,6 +61,35 @@ constexpr int ens_threads() {
 template <int MODE>
 constexpr int ens_lds() {
   return std::max({EnsShape<MODE, 0>::LDS, EnsShape<MODE, 1>::LDS, EnsShape<MODE, 2>::LDS, EnsShape<MODE, 3>::LDS});
+}
+
+// Shape of a region setting for lattices of size N in an ensemble of `sites` sites: its own,
+// but where both states of every lattice do not fit the 256 MB cache (three quarters of it:
+// just below it single runs over 28 x 28 tiles took 189 to 310 us) the 28 x 28 and 20 x 36
+// tiles, whose rows end off the 128-byte lines, cost what they write of other tiles' lines.
+// There a setting of either takes the cheapest of its own, 24 x 32 and 11 x 64 tiles, by
+// the sites they cover (ragged edges included) times a weight for the lines their rows
+// pass. us for two steps over 28 x 28 / 20 x 36 / 24 x 32 / 11 x 64 tiles, flat launches:
+//   float forces: 1 of N=512 4700 / 3330 / 2525 / 2065, 4 of 256 1842 / 1856 / 1234 / 1007, 12 of 128
+//     820 / 765 / 601 / 532, 16 of 96 394 / 378 / 305 / 355, 60 of 56 263 / 294 / 310 / 229
+//   FP64: 2882 / 2660 / 2147 / 2103, 1458 / 1422 / 1080 / 1057, 743 / 682 / 651 / 614, 322 / 302 / 295 / 417,
+//     226 / 294 / 299 / 265
+inline int ens_shape(int region, int prec, int64_t N, int64_t sites) {
+  if ((region != CF_ENS_REGION_32X32 && region != CF_ENS_REGION_24X40) || 32.0 * (double)sites <= 192e6) return region;
+  const double own = prec != CF_PREC_F32S ? 1.2 : (region == CF_ENS_REGION_32X32 ? 1.45 : 1.3);
+  const int shape[3] = {region, CF_ENS_REGION_28X36, CF_ENS_REGION_15X68};
+  const double weight[3] = {own, 1.15, 1.0};
+  int best = region;
+  double least = 0.0;
+  for (int i = 0; i < 3; ++i) {
+    const int64_t tb = ENS_RB[shape[i]] - 2 * TBH, tc = ENS_RC[shape[i]] - 2 * TBH;
+    const double cost = weight[i] * (double)(cdiv(N, tb) * tb) * (double)(cdiv(N, tc) * tc);
+    if (i == 0 || cost < least) {
+      least = cost;
+      best = shape[i];
+    }
+  }
+  return best;
 }
 inline int ens_tile_b(int region, int64_t N) {
   const int t = ENS_RB[region] - 2 * TBH;
@@ -267,9 +296,10 @@ static cf_status ens_build(cf_ensemble *e) {
   CF_HIP(hipStreamSynchronize(e->st));
   std::vector<EnsUnit> units;
   std::vector<int> cost;
+  const int64_t sites_all = cf_ensemble_sites(e);
   for (int r = 0; r < e->n; ++r) {
     const int64_t N = e->reals[r].N;
-    const int reg = e->region[N];
+    const int reg = ens_shape(e->region[N], e->prec, N, sites_all);
     const int Tb = ens_tile_b(reg, N), Tc = ens_tile_c(reg, N);
     const int64_t ntb = cdiv(N, Tb), ntc = cdiv(N, Tc);
     const int A = e->chunk[N];

@@ -276,7 +276,9 @@ cf_status cf_ensemble_get_plan(const cf_ensemble *e, int64_t N, int *chunk, int 
  * along c, halo of two sites included): CF_ENS_REGION_32X32 (28 x 28 output tiles, the
  * default), CF_ENS_REGION_24X40 (20 x 36), CF_ENS_REGION_28X36 (24 x 32 tiles, which
  * divide N = 96 and whose rows fall on 128-byte lines for N = 64, 96 and 128) or
- * CF_ENS_REGION_15X68 (11 x 64 tiles). Same bits in all of them. */
+ * CF_ENS_REGION_15X68 (11 x 64 tiles). The first two describe ensembles that fit the
+ * GPU's cache; in a larger one either may run one of the other tiles (a rule on N and the
+ * precision), whose rows do not share memory lines. Same bits in all of them. */
 #define CF_ENS_REGION_32X32 0
 #define CF_ENS_REGION_24X40 1
 #define CF_ENS_REGION_28X36 2

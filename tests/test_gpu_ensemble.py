@@ -267,3 +267,47 @@ def test_paced_f32s_ensemble_keeps_bits(cfl, grid):
         other.set_pace(100)
     other.set_pace(0)
     other.close()
+
+
+def run_ms(ens, steps):
+    """Shortest time of a run of `steps` steps, of five."""
+    ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+    best = float("inf")
+    for _ in range(6):
+        ev[0].record()
+        ens.run(1.0, 0, steps, 1e-6)
+        ev[1].record()
+        torch.cuda.synchronize()
+        best = min(best, ev[0].elapsed_time(ev[1]))
+    return best
+
+
+def test_streaming_tiles_end_on_lines(cfl):
+    """An ensemble too large for the cache and left untuned, or set to 24 x 40, is about as
+    fast as over 11 x 64 tiles (its own 28 x 28 or 20 x 36 ones take 1.6 to 2.3 times that)."""
+    print("case ensemble streaming tiles", flush=True)
+    ens = cfl.Ensemble([512], [512.0], 1.0, 0.0, cfl.radiation(**FRW), cfl.CF_PREC_F32S)
+    ens.init_grf([1], cfl.CF_SPEC_GAUSS, (0.25,), 1.0)
+    ms = {"untuned": run_ms(ens, 2)}
+    for name, region in (("24x40", cfl.CF_ENS_REGION_24X40), ("15x68", cfl.CF_ENS_REGION_15X68)):
+        ens.set_region(512, region)
+        ms[name] = run_ms(ens, 2)
+    ens.close()
+    assert ms["untuned"] < 1.3 * ms["15x68"] and ms["24x40"] < 1.3 * ms["15x68"], ms
+
+
+@pytest.mark.parametrize("prec", [0, 1, 2])
+@pytest.mark.parametrize("N,count", [(56, 36), (96, 8), (184, 1)])
+def test_streaming_tiles_keep_bits(cfl, prec, N, count):
+    """Sizes whose default tiles beyond the cache are 28 x 28 or 11 x 64, 24 x 32, and 11 x
+    64 ones: the bits of single-lattice runs, in both settings that choose."""
+    print(f"case ensemble streaming bits prec={prec} N={N}", flush=True)
+    ens = cfl.Ensemble([N] * count, [float(N)] * count, 1.0, 0.1, cfl.radiation(**FRW), prec)
+    ens.init_grf(list(range(1, count + 1)), cfl.CF_SPEC_GAUSS, (0.25,), 1.0)
+    for k, region in enumerate((cfl.CF_ENS_REGION_32X32, cfl.CF_ENS_REGION_24X40)):
+        ens.set_region(N, region)
+        assert ens.get_region(N) == region
+        init = [raw_state(cfl, ens, r) for r in range(count)]
+        ens.run(1.0, k, 1, 0.05)
+        check_single_lattice_runs(cfl, ens, prec, init, 1.0, k, 1, 0.05)
+    ens.close()
