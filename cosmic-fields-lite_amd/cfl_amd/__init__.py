@@ -190,8 +190,17 @@ def rk4_tb_get_chunk(N):
     return lib.cf_rk4_tb_get_chunk(N)
 
 
+def rk4_tb_geometry(N, precision=CF_PREC_F64, chunk=0):
+    """What the blocked step of an N^3 lattice runs over: (region rows, region columns, tile
+    rows, tile columns, planes per block, blocks)."""
+    geom = (C.c_int * 6)()
+    check(lib.cf_rk4_tb_geometry(N, precision, chunk, geom))
+    return tuple(geom)
+
+
 def rk4_tb_f32s_region(N):
-    """(rows, columns) of the regions the f32s step covers an N^3 lattice with."""
+    """(rows, columns) of the f32s step's regions while they had halos of four sites (kept
+    for callers that hold the answers; rk4_tb_geometry tells what runs)."""
     rows, cols = C.c_int(0), C.c_int(0)
     check(lib.cf_rk4_tb_f32s_region(N, C.byref(rows), C.byref(cols)))
     return rows.value, cols.value

@@ -106,6 +106,7 @@ _SIGS = [
     ("cf_rk4_tb_tune_pace", st, [C.POINTER(KGParams), vp, vp, dbl, dbl, C.c_int, vp, vp, C.POINTER(C.c_int)]),
     ("cf_rk4_tb_set_pace", st, [i64, C.c_int, C.c_int]),
     ("cf_rk4_tb_get_pace", C.c_int, [i64, C.c_int]),
+    ("cf_rk4_tb_geometry", st, [i64, C.c_int, C.c_int, C.POINTER(C.c_int)]),
     ("cf_rk4_tb_f32s_region", st, [i64, C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     ("cf_rk4_tb_set_chunk", st, [i64, C.c_int]),
     ("cf_rk4_tb_get_chunk", C.c_int, [i64]),

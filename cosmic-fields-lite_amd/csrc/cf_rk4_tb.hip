@@ -282,9 +282,10 @@ static TbGeom tb_comp_geom(bool sa, int64_t N, int chunk) {
   return tb_plan(TB_FAM_F32S, N, chunk, 0, N, N);
 }
 
-// The region class of a lattice size that cf_rk4_tb_f32s_region reports: 24 x 40 unless
-// rounds x (chunk + 8) of a launch over 32 x 32 regions with halos of four is more than
-// 20% lower. Callers file tuned settings by it; the kernel's own shapes are tb_shapes'.
+// The regions that cf_rk4_tb_f32s_region reports: those of the step while its regions had
+// halos of four, 24 x 40 unless rounds x (chunk + 8) of a launch over 32 x 32 ones was more
+// than 20% lower. Kept for callers that hold its answers; what a launch runs over is tb_plan's
+// choice (cf_rk4_tb_geometry).
 static void tb_f32s_class(int64_t N, int *rows, int *cols) {
   const int cus = tb_cus();
   auto least = [&](int64_t tb, int64_t tc) {
@@ -823,6 +824,17 @@ cf_status cf_rk4_tb_f32s_region(int64_t N, int *rows, int *cols) {
   CF_REQUIRE(valid_N(N), "cf_rk4_tb_f32s_region: unsupported lattice size N=%lld", (long long)N);
   CF_REQUIRE(rows && cols, "cf_rk4_tb_f32s_region: null output");
   tb_f32s_class(N, rows, cols);
+  return CF_OK;
+}
+
+cf_status cf_rk4_tb_geometry(int64_t N, int precision, int chunk, int geom[6]) {
+  CF_REQUIRE(valid_N(N), "cf_rk4_tb_geometry: unsupported lattice size N=%lld", (long long)N);
+  CF_REQUIRE(precision == CF_PREC_F64 || precision == CF_PREC_F32C || precision == CF_PREC_F32S,
+             "cf_rk4_tb_geometry: unknown precision %d", precision);
+  CF_REQUIRE(geom, "cf_rk4_tb_geometry: null output");
+  const TbGeom g = precision == CF_PREC_F64 ? tb_f64_geom(N, chunk) : tb_comp_geom(precision == CF_PREC_F32S, N, chunk);
+  const int v[6] = {g.rb, g.rc, g.Tb, g.Tc, g.A, g.total};
+  for (int i = 0; i < 6; ++i) geom[i] = v[i];
   return CF_OK;
 }
 

@@ -189,10 +189,14 @@ int cf_rk4_tb_get_pace(int64_t N, int chunk);
  * set or the cost model's), -1 for an unsupported N. */
 cf_status cf_rk4_tb_set_chunk(int64_t N, int chunk);
 int cf_rk4_tb_get_chunk(int64_t N);
-/* Region class of the f32s step for N on the current device, 24 x 40 or 32 x 32 (rows
- * along b x columns along c): the shape whose launch over regions with four-site halos
- * the chunk cost is lower for (no reference counterpart). A name to file tuned settings
- * under; the step's own tiles are chosen per launch and may be larger. */
+/* What the blocked step of an N^3 lattice in precision CF_PREC_F64, _F32C or _F32S runs over
+ * with this chunk (<= 0: the default) on the current device (no reference counterpart):
+ * geom = {rows along b and columns along c of a block's region, halo included; rows and
+ * columns of the output tile; planes per block along a; blocks}. */
+cf_status cf_rk4_tb_geometry(int64_t N, int precision, int chunk, int geom[6]);
+/* The f32s step's regions for N (rows along b x columns along c) while they had halos of
+ * four sites: 24 x 40 or 32 x 32. Kept, with its answers, for callers that hold them; no
+ * launch has these shapes any more, cf_rk4_tb_geometry tells what runs. */
 cf_status cf_rk4_tb_f32s_region(int64_t N, int *rows, int *cols);
 /* cf_rk4_run_tb_f64 without a work buffer and without any allocation. No counterpart
  * in the reference: it is for callers that cannot allocate device memory (code
