@@ -187,6 +187,27 @@ static double tb_cost(int family, const TbShapeInfo &s, const TbGeom &g, int cus
   return t;
 }
 
+// A chunk that the caller gives can leave CUs idle. Beyond the cache their share of the rate
+// is lost, so such a launch takes shorter tiles, as many as there are CUs (in doubles four
+// fifths of them: beyond that the blocks run against each other). us a step, tiles as large as
+// the region / here:
+//   float forces, N=256, chunk 128 (24 rows / 16) 179 / 136, 224 of 112 137 / 114, 300 of 300
+//     376 / 280, 320 of 320 390 / 310, 512 of 512 1070 / 939
+//   FP64: 224 of 112 127 / 113, 250 of 125 138 / 130 (256 blocks: 142), 320 of 320 350 / 310
+// FP32-comp and the variants are bound by arithmetic in their largest regions, where shorter
+// tiles lose (FP32-comp, N=320, chunk 160 288 / 308): they keep theirs.
+static void tb_fill(int family, TbGeom &g) {
+  if (family != TB_FAM_F64 && family != TB_FAM_F32S) return;
+  const double sites = (double)g.N * (double)g.N * (double)(g.a_hi - g.a_lo);
+  if ((tb_load_bytes[family] + 16.0) * sites <= 256e6) return;
+  const int cus = tb_cus(), most = family == TB_FAM_F32S ? cus : cus * 4 / 5;
+  const int rows = most / (g.ntc * g.n_ac);  // tiles along b that keep to `most` blocks
+  if (rows <= g.ntb) return;
+  g.Tb = (int)cdiv(g.N, rows);
+  g.ntb = (int)cdiv(g.N, g.Tb);
+  g.total = g.ntb * g.ntc * g.n_ac;
+}
+
 // The cheapest (shape, chunk) of a launch, or the cheapest shape for a given chunk. With
 // `near`, also every chunk length whose best shape costs at most near_pct percent more,
 // cheapest first. Chunk lengths are the ceil(planes / k); there are about 2 sqrt(planes).
@@ -216,6 +237,7 @@ static TbGeom tb_plan_search(int family, int64_t N, int chunk, int64_t a_lo, int
   };
   if (chunk > 0) {
     try_chunk(chunk);
+    tb_fill(family, best);
     return best;
   }
   for (int64_t k = 1; k <= planes;) {  // every distinct ceil(planes / k)

@@ -54,3 +54,14 @@ def test_paced_widest_region(cfl, O, lam):
         check_step(cfl, O, N, 0, "f32s", lam)
     finally:
         cfl.rk4_tb_set_pace(N, 0)
+
+
+@pytest.mark.parametrize("mode", ["f64", "f32s"])
+@pytest.mark.parametrize("lam", [0.0, 0.1])
+def test_shorter_tiles(cfl, O, mode, lam):
+    """Tiles of fewer rows than the region holds (a given chunk that would leave units idle)."""
+    N, chunk = 202, 101
+    print(f"case tb dispatch shorter tiles {mode} lam={lam}", flush=True)
+    rb, _, tb, *_ = cfl.rk4_tb_geometry(N, cfl.CF_PREC_F64 if mode == "f64" else cfl.CF_PREC_F32S, chunk)
+    assert torch.cuda.get_device_properties(0).multi_processor_count != 256 or tb < rb - 4
+    check_step(cfl, O, N, chunk, mode, lam)

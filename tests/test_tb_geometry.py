@@ -53,3 +53,12 @@ def test_bitwise_sizes_reach_every_shape(prec):
         lam[N % 4 != 0].add(cfl.rk4_tb_geometry(N, prec, chunk)[:2])
     assert lam[False] | lam[True] == SHAPES[prec]
     assert lam[True] == SHAPES[prec]  # with the quartic term as well
+
+
+@pytest.mark.parametrize("prec,least", [(cfl.CF_PREC_F64, 0.7), (cfl.CF_PREC_F32S, 0.9)])
+@pytest.mark.parametrize("N,chunk", [(202, 101), (224, 112), (256, 128), (300, 300), (320, 320)])
+def test_given_chunk_leaves_few_units_idle(prec, least, N, chunk):
+    """A long chunk in a lattice beyond the cache: shorter tiles, not a fraction of the chip."""
+    if not plans_for_256():
+        pytest.skip("the sizes are chosen for 256 compute units")
+    assert least * 256 <= cfl.rk4_tb_geometry(N, prec, chunk)[5] <= 256
