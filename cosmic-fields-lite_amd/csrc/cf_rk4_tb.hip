@@ -561,7 +561,16 @@ static cf_status tb_step_comp_slab(const char *name, bool sa, const cf_kg_params
                  disjoint(hi_in, lo_out, b) && disjoint(lo_in, hi_out, b) && disjoint(lo_in, lo_out, b),
              "%s: overlapping buffers", name);
   TbGeom g = tb_plan(sa ? TB_FAM_F32S : TB_FAM_F32C, p->N, chunk, TB_GHOST, TB_GHOST + n_planes, NA);
-  if (sa) CF_TRY(tb_pace_lookup(g));  // the pace tuned for this lattice size and chunk, if any
+  if (sa) {
+    // The pace tuned for this lattice size and chunk, if any. Its ticks are those of a plane
+    // of the whole lattice's regions, so a paced slab runs over the same.
+    TbGeom whole = tb_plan_search(TB_FAM_F32S, p->N, g.A, 0, p->N, p->N);  // (leaves the slab's plan kept)
+    CF_TRY(tb_pace_lookup(whole));
+    if (whole.pace > 0) {
+      g = tb_geom(TB_FAM_F32S, whole.shape, p->N, g.A, TB_GHOST, TB_GHOST + n_planes, NA);
+      g.pace = whole.pace;
+    }
+  }
   return tb_launch_comp(sa, g, tb_step_host(p, t, dt), hi_in, lo_in, hi_out, lo_out, st);
 }
 

@@ -123,3 +123,34 @@ def test_slab_rejects_bad_sizes(cfl):
         cfl.rk4_step_tb_f64_slab(p, 17, buf, out, 1.0, 0.05)
     with pytest.raises(cfl.CfError):
         cfl.rk4_step_tb_f64_slab(p, 1, buf, buf, 1.0, 0.05)
+
+
+def test_slab_is_paced_with_its_chunk(cfl):
+    """The pace kept for (N, chunk) holds for a slab with that chunk, also where the slab alone
+    would run over other regions than the whole lattice: at 20 us a plane a chunk of 16 takes
+    at least 16 planes' time. The bits stay."""
+    N, n, chunk = 256, 32, 16
+    print(f"case slab paced N={N} n={n} chunk={chunk}", flush=True)
+    p = cfl.kg_params(N, float(N), 1.0, 0.0, cfl.radiation(**FRW))
+    hi, lo = cfl.split_f64(slab_of(state(cfl, N, 3), N, 40, n))
+
+    def step():
+        out = torch.zeros_like(hi), torch.zeros_like(lo)
+        ev = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        best = float("inf")
+        for _ in range(4):
+            ev[0].record()
+            cfl.rk4_step_tb_f32s_slab(p, n, hi, lo, *out, 1.3, 0.05, chunk)
+            ev[1].record()
+            torch.cuda.synchronize()
+            best = min(best, ev[0].elapsed_time(ev[1]))
+        return best, out
+
+    free, ref = step()
+    cfl.rk4_tb_set_pace(N, 2000, chunk)
+    try:
+        paced, out = step()
+    finally:
+        cfl.rk4_tb_set_pace(N, 0, chunk)
+    assert torch.equal(out[0], ref[0]) and torch.equal(out[1], ref[1])
+    assert free < 0.2 and paced > 16 * 0.02, (free, paced)
