@@ -172,3 +172,23 @@ def test_wkb_tables_equal_oracle(lib, O, t_f):
     lib.check(L.cf_wkb_tables_host(N, Lb, m, a1, H1, t_i, t_f, *[x.ctypes.data_as(C.c_void_p) for x in g]))
     for a, b in zip(g, O.wkb_tables(N, Lb, m, a1, H1, t_i, t_f)):
         assert np.array_equal(a, b)
+
+
+def test_stream_handles(monkeypatch):
+    """The handle a call runs on: the given stream's, else the current one's, with and without
+    torch's raw accessor (no public name: a build may lack it)."""
+    import torch
+
+    import cfl_amd as cfl
+
+    class Stream:
+        def __init__(self, handle):
+            self.cuda_stream = handle
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream(0x20))
+    monkeypatch.setattr(cfl, "_raw_stream", lambda device: 0x10 + device)
+    assert cfl._stream(Stream(0x30)).value == 0x30
+    assert cfl._stream().value == 0x13
+    monkeypatch.setattr(cfl, "_raw_stream", None)
+    assert cfl._stream().value == 0x20
