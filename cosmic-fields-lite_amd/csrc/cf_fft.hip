@@ -254,6 +254,82 @@ __global__ __launch_bounds__(512) void k_fft_c2r(FftLen p, const double2 *__rest
   fft_stage<1, true>(p, last, tb.tw, w.qm, w.dq, ld_m, gs, tb.idx);
 }
 
+// Passes along b and c of the inverse transform of small lattices at once: a block takes a
+// plane of N rows through both in LDS (rows of an odd number of entries, so that lanes across
+// the rows use different banks). What bounds it is what it saves a launch of: memory latency,
+// 3.7-5 us a pass at N=64 whatever it moves. us for an inverse transform, hipFFT (which takes
+// two kernels to N=84) / three passes / here: N=32 10.0 / 11.3 / 9.1, 64 11.5 / 13.9 / 11.7, 80 15.8 / 19.4 /
+// 16.7, 96 27.5 / 23.5 / 21.1, 128 37.1 / 31.7 / 31.6; Psi and dPsi/dt 64 23.5 / 26.6 / 24.2, 128 73.8 / 67.0 / 59.4.
+// PAIR: `in` holds two fields interleaved by entry; a block for each field's planes.
+template <bool PAIR>
+__global__ __launch_bounds__(512) void k_fft_plane_c2r(FftLen pb, FftLen pc, const double2 *__restrict__ in,
+                                                       int64_t pitch, double2 *__restrict__ out) {
+  extern __shared__ __attribute__((aligned(16))) char smem_raw[];
+  const int N = pb.n, n = pc.n, P = (n + 1) | 1, t = (int)threadIdx.x, nt = (int)blockDim.x;
+  double2 *data = reinterpret_cast<double2 *>(smem_raw), *tw = data + (size_t)N * P;
+  uint16_t *posb = reinterpret_cast<uint16_t *>(tw + N), *posc = posb + N;
+  const int a = PAIR ? (int)blockIdx.x >> 1 : (int)blockIdx.x, f = PAIR ? (int)blockIdx.x & 1 : 0;
+  constexpr int KS = PAIR ? 2 : 1;  // entry stride
+  for (int i = t; i < N; i += nt) {
+    tw[i] = pb.tw[i];
+    posb[i] = pb.pos[i];
+    if (i < n) posc[i] = pc.pos[i];
+  }
+  const int l = t & (FFT_CW - 1), g = t / FFT_CW, groups = nt / FFT_CW;
+  {  // along b: lanes over columns; row slots end in digit-reversed order (posb)
+    const int tiles = (n + FFT_CW) / FFT_CW, dq = groups / tiles, q = g / tiles, c = g % tiles * FFT_CW + l;
+    const bool on = q < dq && c <= n;
+    const double2 *src = in + ((int64_t)a * N * pitch + c) * KS + f;
+    double2 *d = data + c;
+    auto gl = [&](int e) { return src[e * pitch * KS]; };
+    auto ld = [&](int e) { return d[e * P]; };
+    auto st = [&](int e, int, int, double2 v) { d[e * P] = v; };
+    const int last = pb.stages - 1;
+    if (last == 0) {
+      if (on) fft_stage<1, true>(pb, 0, pb.tw, q, dq, gl, st);
+    } else {
+      if (on) fft_stage<1, false>(pb, 0, pb.tw, q, dq, gl, st);
+      for (int s = 1; s < last; ++s) {
+        __syncthreads();
+        if (on) fft_stage<1, false>(pb, s, tw, q, dq, ld, st);
+      }
+      __syncthreads();
+      if (on) fft_stage<1, true>(pb, last, tw, q, dq, ld, st);
+    }
+  }
+  __syncthreads();
+  for (int i = t; i < N * (n / 2 + 1); i += nt) {  // Z[k] and Z[n-k] from X[k] and X[n-k] (k_fft_c2r)
+    const int k = i / N;
+    double2 *d = data + (i - k * N) * P;
+    double2 x = d[k], y = d[n - k];
+    if (k == 0) x.y = y.y = 0.0;
+    const double2 e = make_double2(x.x + y.x, x.y - y.y), m = make_double2(x.x - y.x, x.y + y.y);
+    const double2 v = fft_tw<1>(m, tw[k]);
+    d[k] = make_double2(e.x - v.y, e.y + v.x);
+    if (k > 0 && 2 * k != n) d[n - k] = make_double2(e.x + v.y, v.x - e.y);
+  }
+  {  // along c: lanes over rows
+    const int tiles = (N + FFT_CW - 1) / FFT_CW, dq = groups / tiles, q = g / tiles, r = g % tiles * FFT_CW + l;
+    const bool on = q < dq && r < N;
+    double2 *d = data + r * P;
+    auto ld = [&](int e) { return d[e]; };
+    auto st = [&](int e, int, int, double2 v) { d[e] = v; };
+    const int last = pc.stages - 1;
+    for (int s = 0; s < last; ++s) {
+      __syncthreads();
+      if (on) fft_stage<1, false>(pc, s, tw, q, dq, ld, st);
+    }
+    __syncthreads();
+    if (on) fft_stage<1, true>(pc, last, tw, q, dq, ld, st);
+  }
+  __syncthreads();
+  double2 *dst = out + ((int64_t)f * N + a) * N * n;
+  for (int i = t; i < N * n; i += nt) {
+    const int j = i / n;
+    dst[i] = data[posb[j] * P + posc[i - j * n]];
+  }
+}
+
 // First pass (along a) of the inverse of two fields: in * tab.x and in * tab.y into the two
 // fields of `out`, interleaved by column ([a][b][c][field]). A block's eight lines are four
 // columns of both fields, so the spectrum and the factors are read once and the stores
@@ -369,6 +445,7 @@ static bool fft_len(int n, int tws, FftLen *p, std::vector<uint16_t> *pos, std::
 static cf_status fft_allow_lds() {
   constexpr int most = 160 << 10;
   const void *kernels[] = {(const void *)k_fft_r2c,  (const void *)k_fft_c2r<false>, (const void *)k_fft_c2r<true>,
+                           (const void *)k_fft_plane_c2r<false>, (const void *)k_fft_plane_c2r<true>,
                            (const void *)k_fft_pair, (const void *)k_fft_cols<-1, false, false>,
                            (const void *)k_fft_cols<-1, false, true>, (const void *)k_fft_cols<1, false, false>,
                            (const void *)k_fft_cols<1, true, false>};
@@ -462,6 +539,20 @@ static cf_status pass_c2r(const FftPlan &p, const double2 *in, int64_t pitch, do
   return CF_OK;
 }
 
+// Largest lattice whose inverse takes the passes along b and c in one kernel. There its plane
+// fills a CU's LDS (135 of 160 KB), and one field's inverse is no faster than by two passes
+// (above); two fields' still is.
+constexpr int FFT_PLANE_N = 128;
+template <bool PAIR>
+static cf_status pass_plane(const FftPlan &p, const double2 *in, int64_t pitch, double *out, hipStream_t st) {
+  const size_t lds = (size_t)p.N * ((p.N / 2 + 1) | 1) * sizeof(double2) + (size_t)p.N * sizeof(double2) +
+                     (size_t)(p.N + p.N / 2) * sizeof(uint16_t);
+  hipLaunchKernelGGL(k_fft_plane_c2r<PAIR>, dim3((unsigned)(PAIR ? 2 * p.N : p.N)), dim3(512), lds, st, p.full, p.half,
+                     in, pitch, (double2 *)out);
+  CF_LAUNCHED();
+  return CF_OK;
+}
+
 // Rows of a pass along b: planes a; along a: rows b.
 static ColGeom cols_geom(const FftPlan &p, bool along_a, int64_t pitch) {
   const int64_t H = p.N / 2 + 1, plane = p.N * pitch;
@@ -506,6 +597,7 @@ cf_status fft_inverse(const FftPlan &p, const double2 *in, double2 *spec, const 
   r.ncol = (int)(p.N / 2 + 1);  // a scale's table ends there
   if (scale.table) CF_TRY((pass_cols<1, true, false>(p, r, a, p.N, in, spec, scale, nullptr, st)));
   else CF_TRY((pass_cols<1, false, false>(p, r, a, p.N, in, spec, scale, nullptr, st)));
+  if (p.N <= FFT_PLANE_N) return pass_plane<false>(p, spec, pitch, out, st);
   CF_TRY((pass_cols<1, false, false>(p, b, b, p.N, spec, spec, FftScale{}, nullptr, st)));
   return pass_c2r<false>(p, spec, pitch, out, p.N * p.N, st);
 }
@@ -516,6 +608,7 @@ cf_status fft_inverse_pair(const FftPlan &p, const double2 *R, const double2 *ta
   hipLaunchKernelGGL(k_fft_pair, dim3((unsigned)(cdiv(tiles, 8) * 16)), dim3(fft_threads(fft_lds(p.full))),
                      fft_lds(p.full), st, p.full, R, tab, spec, (int)pitch);
   CF_LAUNCHED();
+  if (p.N <= FFT_PLANE_N) return pass_plane<true>(p, spec, pitch, out, st);
   ColGeom b = cols_geom(p, false, 2 * pitch);
   b.nct = (int)(2 * pitch / FFT_CW);
   CF_TRY((pass_cols<1, false, false>(p, b, b, p.N, spec, spec, FftScale{}, nullptr, st)));
