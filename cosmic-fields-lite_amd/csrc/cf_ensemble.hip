@@ -23,6 +23,7 @@
 #include <algorithm>
 #include <map>
 #include <queue>
+#include <set>
 #include <vector>
 
 #include "cf_tb_body.hpp"
@@ -250,6 +251,7 @@ struct cf_ensemble {
   EnsReal *d_reals = nullptr;
   std::map<int64_t, int> chunk;   // planes per unit, per lattice size
   std::map<int64_t, int> region;  // CF_ENS_REGION_*, per lattice size
+  std::set<int64_t> tuned;        // sizes whose region the tuner timed: that shape itself (ens_shape)
   int grid = 0;
   int n_units = 0;
   int32_t *d_unit_off = nullptr;
@@ -299,7 +301,7 @@ static cf_status ens_build(cf_ensemble *e) {
   const int64_t sites_all = cf_ensemble_sites(e);
   for (int r = 0; r < e->n; ++r) {
     const int64_t N = e->reals[r].N;
-    const int reg = ens_shape(e->region[N], e->prec, N, sites_all);
+    const int reg = e->tuned.count(N) ? e->region[N] : ens_shape(e->region[N], e->prec, N, sites_all);
     const int Tb = ens_tile_b(reg, N), Tc = ens_tile_c(reg, N);
     const int64_t ntb = cdiv(N, Tb), ntc = cdiv(N, Tc);
     const int A = e->chunk[N];
@@ -634,6 +636,7 @@ cf_status cf_ensemble_set_region(cf_ensemble *e, int64_t N, int region) {
   CF_REQUIRE(e->region.count(N), "cf_ensemble_set_region: no lattice of size %lld", (long long)N);
   CF_REQUIRE(region >= 0 && region < ENS_REGIONS, "cf_ensemble_set_region: unknown region shape %d", region);
   e->region[N] = region;
+  e->tuned.erase(N);
   return ens_build(e);
 }
 
@@ -670,6 +673,7 @@ cf_status cf_ensemble_tune(cf_ensemble *e, double dt, int reps, int *grid_out) {
   // Flat launches first, every size at one common chunk and region shape: a start from
   // which no size's later sweep is misled by another size's poor chunk.
   e->grid = CF_ENS_GRID_FLAT;
+  for (const auto &kv : e->chunk) e->tuned.insert(kv.first);
   int best_a = 0, best_r = CF_ENS_REGION_28X36;
   for (int reg : {CF_ENS_REGION_28X36, CF_ENS_REGION_32X32})
     for (int A : {64, 32, 16, 8}) {

@@ -283,7 +283,8 @@ cf_status cf_ensemble_get_plan(const cf_ensemble *e, int64_t N, int *chunk, int 
  * divide N = 96 and whose rows fall on 128-byte lines for N = 64, 96 and 128) or
  * CF_ENS_REGION_15X68 (11 x 64 tiles). The first two describe ensembles that fit the
  * GPU's cache; in a larger one either may run one of the other tiles (a rule on N and the
- * precision), whose rows do not share memory lines. Same bits in all of them. */
+ * precision), whose rows do not share memory lines, unless the tuner chose it. Same bits in
+ * all of them. */
 #define CF_ENS_REGION_32X32 0
 #define CF_ENS_REGION_24X40 1
 #define CF_ENS_REGION_28X36 2
