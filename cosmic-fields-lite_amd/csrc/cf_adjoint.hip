@@ -502,7 +502,9 @@ size_t cf_adjoint_work_bytes(int64_t N, int64_t n_steps, int64_t ckpt) {
   if (!valid_N(N) || n_steps < 0 || ckpt <= 0) return 0;
   const size_t v = 2 * (size_t)N * N * N * sizeof(double);
   const size_t nck = (size_t)((n_steps + ckpt - 1) / ckpt);
-  // checkpoints + one segment of states + lambda (2) + rk4 work (3)
+  // checkpoints + one segment of states + lambda (2) + forward work (3). Callers size buffers
+  // by this; of it the first and last checkpoint (x0 itself; kept with the last segment) and
+  // the third work vector are not touched.
   return nck * v + (size_t)ckpt * v + 2 * v + 3 * v +
          (size_t)(4 * n_steps + 1) * ADJ_BLOCKS * sizeof(double);
 }
@@ -527,8 +529,8 @@ cf_status cf_loss_spectrum_adjoint(cf_spectrum_plan *plan, const cf_kg_params *p
 }
 
 // One backward step from state x at time t: lo = dL/dx_n from li = dL/dx_{n+1};
-// part: 4*ADJ_BLOCKS partials of dL/dm (stages 4, 3, 2, 1). lo overlaps neither x
-// nor li.
+// part: 4*ADJ_BLOCKS partials of dL/dm, one per block over all four stages, zero beyond the
+// grid. lo overlaps neither x nor li.
 static cf_status adj_step(const cf_kg_params *p, const double *x, double t, double dt, const double *li, double *lo,
                           double *part, hipStream_t st) {
   const int64_t N = p->N;

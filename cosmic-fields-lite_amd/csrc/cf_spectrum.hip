@@ -10,12 +10,12 @@
 // Binning without atomics. The half spectrum has N*N*(N/2+1) entries; entry
 // (a,b,c) belongs to bin s = a'^2 + b'^2 + c^2 with x' = min(x, N-x), and counts
 // twice unless c is 0 or N/2 (the full-cube loop of fdm3d.cpp:11-28 visits the
-// mirrored column too). A row (a, b) of the half spectrum has the row class
-// r = a'^2 + b'^2, so s = r + c^2. At plan creation the host sorts the N^2 rows by
-// r (4 B per row). Step A sums, for each class r, its whole rows (each read
-// contiguously, in sorted order) into Q[c][r]; step B forms P(s) as the sum over
-// ascending c of Q[c][s - c^2]. Every sum has a fixed order and no atomics are
-// used, so two runs give identical bits.
+// mirrored column too). A row (a, b) of the half spectrum has r = a'^2 + b'^2, so s = r +
+// c^2. At plan creation the host sorts the N^2 rows by r (4 B per row) and numbers the r
+// that have rows, the classes. Step A sums each class's whole rows (each read contiguously,
+// in sorted order) into Q[c][class]; step B forms P(s) as the sum over c of Q[c][class of s -
+// c^2], eight contiguous ranges of c each in ascending order, then the eight parts in order.
+// Every sum has a fixed order and no atomics are used, so two runs give identical bits.
 #include <hipfft/hipfft.h>
 
 #include <cmath>

@@ -41,10 +41,12 @@
 // it cannot do without (a plain copy reaches 4.8-5.0 on this part); below N=200 vector
 // and LDS issue and the chain of dependent FP64 operations of a plane.
 //
-// Tiles. Tc is 16, 32, 64 or 128, so that a tile's rows begin and end on 128-byte lines
-// where the lattice's rows do: 28 x 28 tiles (32 x 32 regions), whose row ends share
-// lines with their neighbours, ran at 98 GSite*step/s at N=512 in FP64 against 134 for
-// 24 x 32 tiles and 150 for 26 x 64.
+// Tiles. Tc is 16, 32, 64 or 128 in the single-lattice shapes (N where that is smaller), so
+// that a tile's rows begin and end on 128-byte lines where the lattice's rows do: 28 x 28
+// tiles (32 x 32 regions), whose row ends share lines with their neighbours, ran at 98
+// GSite*step/s at N=512 in FP64 against 134 for 24 x 32 tiles and 150 for 26 x 64. (Ensembles
+// that fit the cache may take 28 x 28 or 20 x 36 ones.) T may be less than the region's rows
+// hold, for more and smaller tiles.
 //
 // Arithmetic. Per site and stage the operations, their order and their rounding are
 // those of the fused stage kernels (cf_stencil.hip): FP64 keeps acc = 1*x + dt/6 k1

@@ -22,10 +22,11 @@
 //   dPsi^(k) = R^(k) * H (3x cos x + (x^2-3) sin x) * 2/x^3/G^3,   x = |k| eta/sqrt(3)
 // (equations.cpp:141-183), followed by one batched complex-to-real transform of
 // both fields. A classic RK4 step needs them at t, t+dt/2 and t+dt only (stages
-// 2 and 3 share a time), and the next step's first stage is usually this step's
-// last, so a three-slot cache keyed by the exact stage time leaves two transforms
-// per step; the reference computes two transforms per right-hand side. The
-// temporally blocked step reads the three times' fields in one kernel.
+// 2 and 3 share a time). A three-slot cache keyed by the exact stage time leaves two
+// transforms per step where this step's t + dt is the very double that the next one starts
+// with, t0 + (k + 1) dt, and three where they differ in the last bit (dt = 0.5: two a step;
+// t0 = 1, dt = 0.05: 4.8 per two steps); the reference computes two transforms per
+// right-hand side. The temporally blocked step reads the three times' fields in one kernel.
 //
 // All arithmetic is FP64 and, as in the rest of the library, no multiply is
 // fused into an add (-ffp-contract=off).
@@ -305,7 +306,7 @@ struct PsiGrid {
   double *spec = nullptr;  // 2 half spectra: Psi^, dPsi^
   // Psi | dPsi (2*G^3 each) at up to three times, least recently used replaced: a
   // temporally blocked step needs t, t + dt/2 and t + dt at once, and the next step
-  // starts at the previous t + dt (two new times per step either way).
+  // starts at the previous t + dt or a neighbouring double (two or three new times per step).
   static constexpr int NS = 3;
   double *slot[NS] = {nullptr, nullptr, nullptr};
   double slot_t[NS] = {0.0, 0.0, 0.0};

@@ -383,8 +383,8 @@ cf_status cf_variant_rk4_run(cf_variant v, double *x_dev, double t0, int64_t k0,
                              void *work_dev, cf_stream stream);
 /* The same steps temporally blocked (one kernel per step, as cf_rk4_run_tb_f64) for
  * every variant; same bits as cf_variant_rk4_run. The comoving variants build Psi,
- * dPsi/dt at t, t+dt/2 and t+dt first (two new transforms per step, as the stage
- * kernels). work_dev: cf_rk4_tb_work_bytes(N, CF_PREC_F64). */
+ * dPsi/dt at t, t+dt/2 and t+dt first (those that the cache does not hold: two or three new
+ * transforms per step, as the stage kernels). work_dev: cf_rk4_tb_work_bytes(N, CF_PREC_F64). */
 cf_status cf_variant_rk4_run_tb(cf_variant v, double *x_dev, double t0, int64_t k0, int64_t n_steps, double dt,
                                 int chunk, void *work_dev, cf_stream stream);
 cf_status cf_variant_rk4_step_tb(cf_variant v, const double *x_in_dev, double *x_out_dev, double t, double dt,
